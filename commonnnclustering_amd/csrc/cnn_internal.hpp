@@ -16,7 +16,7 @@ namespace cnn {
 
 constexpr int kTile = 64;        // points per tile: one wave64 lane per row
 constexpr int kWave = 64;
-constexpr int kSpatialMaxD = 8;  // d <= 8: spatial (Morton) order + tile-box culling
+constexpr int kSpatialMaxD = 8;  // d <= 8: spatial (Hilbert curve) order + tile-box culling
 constexpr int kMfmaMinD = 16;    // d >= 16: FP32 Gram form on MFMA in CNN_F32_BAND
 constexpr int kBatchWorkers = 6;    // datasets of a batch fitted at once (own stream each)
 constexpr int64_t kPivotMinN = 2048;  // d > 8: smallest n ordered by nearest-pivot cells
@@ -295,7 +295,7 @@ struct PackedHost {
     std::vector<int32_t> tile_ds;     // dataset of each tile
 };
 // Many datasets (rows offsets[b] .. offsets[b+1] of X, own r2[b]) in one graph:
-// each dataset is Morton-ordered and padded to whole tiles (padding rows have
+// each dataset is curve-ordered and padded to whole tiles (padding rows have
 // perm -1 and NaN coordinates); candidate tile pairs never cross datasets.
 cnn_graph *graph_build_packed(cnn_ctx *ctx, const void *X, const int64_t *offsets, int32_t n_sets, int32_t d,
                               int32_t dtype, const double *r2, int32_t precision, PackedHost &ph);
