@@ -11,7 +11,7 @@ Tuned here (``cnn_tune_params``):
                   (FP32-banded form, d >= 16)
   wide_col_chunk  column tiles per workgroup of the dense plain-FP64 kernel
   emit_waves      waves per workgroup of the neighbour-list emission
-  root_passes     root-hooking passes before the labelling's full round
+  root_passes     root-hooking passes before the full round of a labelling on lists
   words_min_fill  lists with at least this many entries per 64-bit word are
                   tested as per-row word lists (bitset), else merged
 

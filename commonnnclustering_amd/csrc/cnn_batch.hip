@@ -255,7 +255,7 @@ cnn_scan *scan_create(cnn_ctx *ctx, const cnn_graph *g, const double *r2, int32_
         }
     int32_t *own_deg = scan_alloc<int32_t>(sc.get(), n);
     MultiLabelSizes sz;
-    multi_labels_bytes(n, T, n_c, sz);
+    multi_labels_bytes(n, T, P, n_c, sz);
     MultiLabelBufs b;
     b.n_c = n_c;
     b.n = n;
@@ -265,8 +265,10 @@ cnn_scan *scan_create(cnn_ctx *ctx, const cnn_graph *g, const double *r2, int32_
     b.parent = scan_alloc<int>(sc.get(), m);
     b.rank = scan_alloc<uint64_t>(sc.get(), m);
     b.cnt = scan_alloc<int32_t>(sc.get(), m);
-    b.hq = scan_alloc<int32_t>(sc.get(), m);
-    b.hq_len = scan_alloc<unsigned int>(sc.get(), n_c);
+    b.hq = scan_alloc<uint32_t>(sc.get(), m);
+    b.lens = scan_alloc<unsigned int>(sc.get(), 2 * (int64_t)n_c);
+    b.rq = scan_alloc<int2>(sc.get(), sz.round_queue);
+    b.rq_len = scan_alloc<unsigned long long>(sc.get(), n_c);
     b.tmax = scan_alloc<uint64_t>(sc.get(), mt);
     b.cand_max = scan_alloc<uint64_t>(sc.get(), mt);
     b.tile_common = scan_alloc<uint64_t>(sc.get(), mt);
@@ -275,7 +277,6 @@ cnn_scan *scan_create(cnn_ctx *ctx, const cnn_graph *g, const double *r2, int32_
     b.newlab = scan_alloc<int32_t>(sc.get(), m);
     b.ckey = scan_alloc<uint64_t>(sc.get(), m);
     b.cidx = scan_alloc<int32_t>(sc.get(), m);
-    b.ccount = scan_alloc<unsigned int>(sc.get(), n_c);
     int32_t *d_csim = scan_alloc<int32_t>(sc.get(), n_c);
     int32_t *d_mcore = scan_alloc<int32_t>(sc.get(), n_c);
     CNN_HIP(hipMemcpy(d_csim, c_sim, n_c * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -311,7 +312,7 @@ cnn_scan *scan_create(cnn_ctx *ctx, const cnn_graph *g, const double *r2, int32_
                 next ^= 1;
             }
             MultiLabelSource src{cur_mask, cur_nz, g->tp_ptr, g->tp_col, cur_deg, g->perm, g->n_tile_pairs};
-            labels_enqueue_multi(ctx, b, src, g->tune.root_passes, member_cutoff, max_clusters,
+            labels_enqueue_multi(ctx, b, src, member_cutoff, max_clusters,
                                  labels + (int64_t)ri * n_c * n, sc->counters + (int64_t)ri * n_c * 8,
                                  sc->tstats + (int64_t)ri * n_c * kScanStatSlots);
         }

@@ -371,18 +371,19 @@ struct MultiLabelBufs {
     int *parent = nullptr;
     uint64_t *rank = nullptr;
     int32_t *cnt = nullptr;
-    int32_t *hq = nullptr;
-    unsigned int *hq_len = nullptr;
+    uint32_t *hq = nullptr;        // hook queues
+    unsigned int *lens = nullptr;  // 2 * n_c: hook queue lengths, cluster counts
+    int2 *rq = nullptr;            // round queues
+    unsigned long long *rq_len = nullptr;
     uint64_t *tmax = nullptr, *cand_max = nullptr, *tile_common = nullptr;
     int32_t *cmin = nullptr, *csize = nullptr, *newlab = nullptr;
     // sort_by_size: the clusters of each pair (keys, roots) and their count
     uint64_t *ckey = nullptr;
     int32_t *cidx = nullptr;
-    unsigned int *ccount = nullptr;                    // n_c
     const int32_t *csim = nullptr, *mcore = nullptr;  // device, n_c each
 };
 struct MultiLabelSizes {
-    int64_t per_point = 0, per_tile = 0;
+    int64_t per_point = 0, per_tile = 0, round_queue = 0;
 };
 // The row words the pass reads: a spatial graph's tile-pair words at one radius.
 struct MultiLabelSource {
@@ -394,11 +395,11 @@ struct MultiLabelSource {
     const int32_t *perm;
     int64_t n_tile_pairs;  // tp_ptr[n_tiles], known on the host
 };
-void multi_labels_bytes(int64_t n, int64_t n_tiles, int n_c, MultiLabelSizes &sz);
+void multi_labels_bytes(int64_t n, int64_t n_tiles, int64_t n_tile_pairs, int n_c, MultiLabelSizes &sz);
 // labels: n_c blocks of n (block y = pair y), sorted by size; counters: 8 per
 // pair ([2] core points, [3] components, [7] clusters); tstats: 4 * 1024 per pair.
-void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabelSource &src, int root_passes,
-                          int64_t member_cutoff, int64_t max_clusters, int64_t *labels, unsigned long long *counters,
+void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabelSource &src, int64_t member_cutoff,
+                          int64_t max_clusters, int64_t *labels, unsigned long long *counters,
                           unsigned long long *tstats);
 void fill_u64(cnn_ctx *ctx, unsigned long long *p, unsigned long long v, int64_t n);
 

@@ -11,17 +11,20 @@
 // yields the same partition regardless of scheduling.
 //
 // Work plan on the GPU (all on the context stream):
-//   k_init      core flags, parent[i] = i
-//   k_hook      each core row tests its nearest smaller-index core neighbours
-//               and hooks its parent to the first that passes (a forest, no
-//               atomics); links most of every dense region cheaply
-//   k_compress  every parent becomes its root
-//   k_hook_roots roots re-point at a smaller neighbouring root on a pass
-//   k_snapshot  rank[i] = (component size << 32 | root) of core points
-//   k_round_b   every edge between different snapshot components is tested by
+//   k_init      core flags, parent[i] = i, cleared component arrays
+//   k_hook_tile each core row tests its two nearest smaller-index core
+//               neighbours of its own tile and hooks its parent to one that
+//               passes (a forest, no atomics); k_hook_queue tests the rows with
+//               fewer in the tiles below (k_hook: per row, without tile words)
+//   k_compress_roots, k_hook_roots_list  (lists only) flatten; roots re-point
+//               at a smaller neighbouring root on a pass
+//   k_root_count, k_snapshot  rank[i] = (component size << 32 | root) of core
+//               points, and the tiles' largest and common ranks
+//   k_round_tile every edge between different snapshot components is tested by
 //               the endpoint of lower rank, unless the endpoints were joined
 //               meanwhile; rows that own no edge are skipped by a per-tile bound
-//   k_compress, component statistics, label assignment / sort_by_size
+//               (k_round_b: per row, without tile words)
+//   k_comp_stats flatten, component statistics; label assignment / sort_by_size
 #include <algorithm>
 #include <climits>
 #include <memory>
@@ -68,7 +71,7 @@ struct LabelArgs {
     int m_core;
     uint8_t *core;
     int *parent;
-    unsigned long long *stats;  // [slot][0] tests, [slot][1] passed
+    unsigned long long *stats;  // per slot: tests, passed, rows scanned, sampled components
     const uint64_t *rank;       // snapshot rank of core points: (component size << 32) | root; 0 otherwise
     const uint64_t *cand_max;   // per row tile: max rank over its candidate tiles (nullable)
     // per tile: the rank every point of the tile has (0: no core point; all
@@ -96,10 +99,8 @@ struct LabelArgs {
     const int32_t *csim_y;
     const int32_t *mcore_y;
     int64_t tiles;
-    // rows k_round_tile hands to k_round_queue (nullable: it tests them itself):
-    // {row, first pair, end pair (both relative to the row tile's first pair),
-    // component the row has joined or -1}
-    int4 *rq;
+    // tile pairs k_round_tile hands to k_round_queue: {row tile, position in its list}
+    int2 *rq;
     unsigned long long *rq_len;
     int64_t rq_cap;
     // the row tiles in the order the per-tile kernels take them: heavy ones
@@ -116,6 +117,10 @@ __device__ __forceinline__ LabelArgs slice(LabelArgs a) {
     a.parent += y * a.n;
     a.rank += y * a.n;
     a.stats += y * 4 * kStatSlots;
+    if (a.rq) {
+        a.rq += y * a.rq_cap;
+        a.rq_len += y;
+    }
     if (a.cand_max) a.cand_max += y * a.tiles;
     if (a.tile_rank) a.tile_rank += y * a.tiles;
     a.c_sim = a.csim_y[y];
@@ -154,18 +159,29 @@ __device__ __forceinline__ int csim_of(const LabelArgs &a, int64_t w) {
     return a.tile_csim ? a.tile_csim[w >> 6] : a.c_sim;
 }
 
-__device__ __forceinline__ void add_stats(const LabelArgs &a, unsigned tests, unsigned passed, unsigned rows = 0) {
-    if ((threadIdx.x & 63) == 0 && (tests || rows)) {
+__device__ __forceinline__ void add_stats(const LabelArgs &a, unsigned tests, unsigned passed, unsigned rows = 0,
+                                          unsigned roots = 0) {
+    if ((threadIdx.x & 63) == 0 && (tests || rows || roots)) {
         const unsigned slot = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kStatSlots - 1);
         if (tests) {
             atomicAdd(&a.stats[4 * slot], (unsigned long long)tests);
             atomicAdd(&a.stats[4 * slot + 1], (unsigned long long)passed);
         }
         if (rows) atomicAdd(&a.stats[4 * slot + 2], (unsigned long long)rows);
+        if (roots) atomicAdd(&a.stats[4 * slot + 3], (unsigned long long)roots);
     }
 }
 
-__global__ void k_init(LabelArgs a, const uint8_t *__restrict__ consider, const int32_t *__restrict__ perm) {
+// Per-component arrays cleared by k_init (each nullable; one slice per cutoff pair).
+struct ComponentArrays {
+    int32_t *cnt;     // sampled component sizes: 0
+    int32_t *cmin;    // smallest caller index: INT_MAX
+    int32_t *csize;   // final component sizes: 0
+    int32_t *newlab;  // sort_by_size labels: 0
+};
+
+__global__ void k_init(LabelArgs a, const uint8_t *__restrict__ consider, const int32_t *__restrict__ perm,
+                       ComponentArrays ca) {
     a = slice(a);
     int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= a.n) return;
@@ -176,6 +192,11 @@ __global__ void k_init(LabelArgs a, const uint8_t *__restrict__ consider, const 
     if (consider && ok) ok = consider[o] != 0;
     a.core[w] = ok ? 1 : 0;
     a.parent[w] = (int)w;
+    const int64_t at = (int64_t)blockIdx.y * a.n + w;
+    ca.cnt[at] = 0;
+    ca.cmin[at] = INT_MAX;
+    ca.csize[at] = 0;
+    if (ca.newlab) ca.newlab[at] = 0;
 }
 
 // Test edge (w, j) unless the endpoints are already joined; link on a pass.
@@ -220,24 +241,24 @@ __device__ __forceinline__ uint64_t lane_bit_mask(int lane) { return 1ull << lan
 // indices, so the hooks form a forest whose trees are the components of the
 // passing edges tested here -- no atomics, no contention.
 // Hooking of one core row on row words: its smaller-index neighbours in
-// descending order, at most max_tests tests; skip_prev: the test against w - 1
-// was already made (k_hook_tile).
-__device__ __forceinline__ void hook_row_words(const LabelArgs &a, int64_t w, int max_tests, bool skip_prev) {
+// descending order, at most max_tests tests; below_own: those of its own tile
+// were tested already (k_hook_tile), only the tiles below it are searched.
+__device__ __forceinline__ void hook_row_words(const LabelArgs &a, int64_t w, int max_tests, bool below_own) {
     const int lane = threadIdx.x & 63;
     const int64_t dw = deg_of(a, w);
-    const bool tested_prev = skip_prev;
     // the row's words from its own tile down, 64 tiles a step (lane l holds
     // the l-th tile below the window's top), bits from the highest down:
     // smaller indices, nearest first
     const WordRow A = word_row(a, w);
     const int Rw = (int)(w >> 6);
-    int64_t top = 0;  // tiles up to and including the row's own tile
+    int64_t top = 0;  // tiles up to and including the row's own tile (below_own: below it)
     if (a.mask && a.diag && a.diag[Rw] >= 0) {
-        top = a.diag[Rw] + 1;  // recorded when the lists were built
+        top = a.diag[Rw] + (below_own ? 0 : 1);  // recorded when the lists were built
     } else {
+        const int last = below_own ? Rw - 1 : Rw;
         for (int64_t t0 = 0; t0 < A.len; t0 += 64) {
             const int64_t t = t0 + lane;
-            const uint64_t le = __ballot(t < A.len && A.tile[t] <= Rw);
+            const uint64_t le = __ballot(t < A.len && A.tile[t] <= last);
             top += __popcll(le);
             if (__popcll(le) < 64) break;
         }
@@ -268,7 +289,6 @@ __device__ __forceinline__ void hook_row_words(const LabelArgs &a, int64_t w, in
                 const int hb = 63 - __clzll((long long)bits);
                 bits &= ~lane_bit_mask(hb);
                 const int jj = Cs * 64 + hb;
-                if (tested_prev && jj == (int)w - 1) continue;
                 ++attempts;
                 ++tests;
                 const int64_t dj = deg_of(a, jj);
@@ -337,39 +357,40 @@ __global__ __launch_bounds__(256) void k_hook(LabelArgs a, int max_tests) {
     add_stats(a, tests, passed);
 }
 
-// Hooking of adjacent rows on a spatial graph's tile-pair words: one wave per
-// row tile, lane r = row w = 64R + r.  Rows of one tile share the tile's
-// candidate list, and pair k's 64 row words are contiguous (lane r reads row
-// r's word), so one pass over the tile's non-empty pairs counts
-// |N(w) & N(w - 1)| for all 63 adjacent row pairs at once (w - 1's word comes
-// from the lane below).  A core row whose predecessor is a core neighbour with
-// at least c_sim common neighbours hooks to it (to the first row of its run of
-// hooked rows, which is connected to it through them).  The pass stops once
-// every row still in question has reached c_sim.  Writes only parent[w] of
-// hooked rows, to a smaller index: a forest, as the per-row hooking.
-__global__ __launch_bounds__(256) void k_hook_tile(LabelArgs a, int64_t n_tiles, int32_t *__restrict__ queue,
+// Hooking within row tiles on tile-pair words: one wave per row tile, lane r =
+// row w = 64R + r.  A core row tests its two nearest smaller-index core
+// neighbours of its own tile.  Rows of one tile share the tile's candidate
+// list, and pair k's 64 row words are contiguous (lane r reads row r's word),
+// so one pass over the tile's non-empty pairs counts |N(w) & N(j)| of both
+// candidates for all 64 rows at once (row j's word comes from lane j).  The
+// own pair is read first: it names the candidates.  The pass stops once every
+// row has a candidate with c_sim common neighbours.  A row hooks to the first
+// row of its chain of hooked rows within the tile: only own entries are
+// written, to smaller indices (a forest).  Core rows that had fewer than two
+// candidates and no pass go to a queue (2 w + tests made) for k_hook_queue;
+// one counter update per workgroup (a single address: per-wave updates took
+// about 100 us for 21,000 tiles).
+__global__ __launch_bounds__(256) void k_hook_tile(LabelArgs a, int64_t n_tiles, uint32_t *__restrict__ queue,
                                                    unsigned int *__restrict__ queue_len) {
     a = slice(a);
     queue += (int64_t)blockIdx.y * a.n;
     queue_len += blockIdx.y;
-    const int lane = threadIdx.x & 63;
-    const int64_t gR = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (gR >= n_tiles) return;
-    const int64_t R = a.tile_order ? (int64_t)a.tile_order[gR] : gR;
+    __shared__ unsigned s_len[4], s_base;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t gR = (int64_t)blockIdx.x * 4 + wave;
+    const bool valid = gR < n_tiles;
+    const int64_t R = !valid ? 0 : a.tile_order ? (int64_t)a.tile_order[gR] : gR;
     const int64_t w = R * 64 + lane;
-    const bool core_w = w < a.n && a.core[w] != 0;
-    const bool core_p = __shfl_up((int)core_w, 1, 64) != 0;
-    const int c = csim_of(a, R * 64);
-    // rows whose test is still open: core, predecessor core within the tile
-    const bool open = lane > 0 && core_w && core_p;
+    const bool core_w = valid && w < a.n && a.core[w] != 0;
+    const uint64_t cores = __ballot(core_w);
     bool hooked = false;
+    int n_cand = 0;
     unsigned tests = 0, passed = 0;
-    if (__ballot(open) != 0ull) {
+    if (cores & (cores - 1)) {  // at least two core rows
+        const int c = csim_of(a, R * 64);
         const int64_t kb = a.tp_ptr[R], ke = a.tp_ptr[R + 1];
-        // the row tile's own pair first (recorded when the lists were built,
-        // or found by a ballot per 64 of its ascending column tiles): it tells
-        // every row whether w - 1 is a neighbour, so the walk below can stop
-        // as soon as the open rows with that neighbour have c common neighbours
+        // the tile's own pair: recorded when the lists were built, or found by
+        // a ballot per 64 of its ascending column tiles
         int64_t kd = -1;
         if (a.diag && a.diag[R] >= 0) kd = kb + a.diag[R];
         for (int64_t k0 = kb; k0 < ke && kd < 0; k0 += 64) {
@@ -377,15 +398,15 @@ __global__ __launch_bounds__(256) void k_hook_tile(LabelArgs a, int64_t n_tiles,
             const uint64_t hit = __ballot(kk < ke && a.tp_col[kk] == (int)R);
             if (hit) kd = k0 + __ffsll((unsigned long long)hit) - 1;
         }
-        int cnt = 0;
-        bool nbr = false;  // w - 1 in N(w): bit lane-1 of the row's word in its own tile
-        if (kd >= 0 && a.pair_nz[kd] != 0) {
-            const uint64_t v = a.mask[kd * 64 + lane];
-            const uint64_t pv = __shfl_up(v, 1, 64);
-            cnt = __popcll(v & pv);
-            nbr = lane > 0 && ((v >> (lane - 1)) & 1ull) != 0ull;
-        }
-        bool done = __ballot(open && nbr && cnt < c) == 0ull;
+        uint64_t own = 0ull;
+        if (kd >= 0 && a.pair_nz[kd] != 0) own = a.mask[kd * 64 + lane];
+        const uint64_t cand = core_w ? own & cores & ((1ull << lane) - 1ull) : 0ull;
+        const int j1 = cand ? 63 - __clzll((long long)cand) : lane;
+        const uint64_t rest = cand & ~(1ull << j1);
+        const int j2 = rest ? 63 - __clzll((long long)rest) : j1;
+        n_cand = cand ? (rest ? 2 : 1) : 0;
+        int cnt1 = __popcll(own & __shfl(own, j1, 64)), cnt2 = __popcll(own & __shfl(own, j2, 64));
+        bool done = __ballot(n_cand && cnt1 < c && cnt2 < c) == 0ull;
         for (int64_t k0 = kb; k0 < ke && !done; k0 += 64) {
             // the window's other non-empty pairs, then their words 8 at a time (loads in flight together)
             const int64_t kk = k0 + lane;
@@ -403,35 +424,41 @@ __global__ __launch_bounds__(256) void k_hook_tile(LabelArgs a, int64_t n_tiles,
                 for (int u = 0; u < 8; ++u) v[u] = idx[u] >= 0 ? a.mask[(k0 + idx[u]) * 64 + lane] : 0ull;
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
-                    const uint64_t pv = __shfl_up(v[u], 1, 64);
-                    cnt += __popcll(v[u] & pv);
+                    cnt1 += __popcll(v[u] & __shfl(v[u], j1, 64));
+                    cnt2 += __popcll(v[u] & __shfl(v[u], j2, 64));
                 }
-                if (__ballot(open && nbr && cnt < c) == 0ull) done = true;
+                if (__ballot(n_cand && cnt1 < c && cnt2 < c) == 0ull) done = true;
             }
         }
-        hooked = open && nbr && cnt >= c;
-        // a run of hooked rows hangs from the unhooked row before it (lane 0
-        // is never hooked): depth one instead of a chain through w - 1
-        const uint64_t below = ~__ballot(hooked) & (lane == 63 ? ~0ull : ((2ull << lane) - 1ull));
-        if (hooked) a.parent[w] = (int)(R * 64 + (63 - __clzll((long long)below)));
-        tests = (unsigned)__popcll(__ballot(open && nbr));
+        hooked = n_cand && (cnt1 >= c || cnt2 >= c);
+        int p = hooked ? (cnt1 >= c ? j1 : j2) : lane;
+#pragma unroll
+        for (int step = 0; step < 6; ++step) p = __shfl(p, p, 64);  // to the head of the chain
+        if (hooked) a.parent[w] = (int)(R * 64 + p);
+        tests = (unsigned)(__popcll(__ballot(n_cand > 0)) + __popcll(__ballot(n_cand > 1)));
         passed = (unsigned)__popcll(__ballot(hooked));
     }
     // core rows left to the per-row hooking
-    const bool left = core_w && !hooked;
+    const bool left = core_w && !hooked && n_cand < 2;
     const uint64_t lm = __ballot(left);
-    if (lm) {
-        unsigned base = 0;
-        if (lane == 0) base = atomicAdd(queue_len, (unsigned)__popcll(lm));
-        base = __shfl(base, 0, 64);
-        if (left) queue[base + __popcll(lm & ((1ull << lane) - 1ull))] = (int32_t)w;
+    if (lane == 0) s_len[wave] = (unsigned)__popcll(lm);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned total = s_len[0] + s_len[1] + s_len[2] + s_len[3];
+        s_base = total ? atomicAdd(queue_len, total) : 0u;
+    }
+    __syncthreads();
+    if (left) {
+        unsigned base = s_base;
+        for (int q = 0; q < wave; ++q) base += s_len[q];
+        queue[base + __popcll(lm & ((1ull << lane) - 1ull))] = (uint32_t)w * 2u + (uint32_t)n_cand;
     }
     add_stats(a, tests, passed);
 }
 
 // Per-row hooking of the rows k_hook_tile left (a queue; grid-stride, one wave
-// per row).
-__global__ __launch_bounds__(256) void k_hook_queue(LabelArgs a, const int32_t *__restrict__ queue,
+// per row): up to max_tests tests in all, in the tiles below the row's own.
+__global__ __launch_bounds__(256) void k_hook_queue(LabelArgs a, const uint32_t *__restrict__ queue,
                                                     const unsigned int *__restrict__ queue_len, int max_tests) {
     a = slice(a);
     queue += (int64_t)blockIdx.y * a.n;
@@ -439,8 +466,8 @@ __global__ __launch_bounds__(256) void k_hook_queue(LabelArgs a, const int32_t *
     const unsigned nq = *queue_len;
     const int64_t waves = (int64_t)gridDim.x * 4;
     for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); q < (int64_t)nq; q += waves) {
-        const int64_t w = queue[q];
-        hook_row_words(a, w, max_tests, (w & 63) != 0);
+        const uint32_t e = queue[q];
+        hook_row_words(a, (int64_t)(e >> 1), max_tests - (int)(e & 1u), true);
     }
 }
 
@@ -529,16 +556,8 @@ __device__ void hook_root(const LabelArgs &a, int64_t w, int max_tests) {
     add_stats(a, tests, passed);
 }
 
-template <bool WORDS>
-__global__ __launch_bounds__(256) void k_hook_roots(LabelArgs a, int max_tests) {
-    a = slice(a);
-    const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (w >= a.n || !a.core[w] || a.parent[w] != (int)w) return;
-    hook_root<WORDS>(a, w, max_tests);
-}
-
-// The same for the roots k_compress_roots listed, one wave each (grid-stride):
-// no wave is started for the points that are not roots.
+// The roots k_compress_roots listed, one wave each (grid-stride): no wave is
+// started for the points that are not roots.
 template <bool WORDS>
 __global__ __launch_bounds__(256) void k_hook_roots_list(LabelArgs a, const int32_t *__restrict__ roots,
                                                          const unsigned int *__restrict__ n_roots, int max_tests) {
@@ -550,23 +569,21 @@ __global__ __launch_bounds__(256) void k_hook_roots_list(LabelArgs a, const int3
     }
 }
 
-// Row w's part of a full round on row words, over its candidate tiles
-// [t_from, t_to) (clamped to the row's tiles): 64 tiles a step (ascending
-// column tile, so entries come in list order), tiles whose points share a
-// rank that is not above w's, or that w has joined, are skipped without
-// reading their bits; tests are bitset intersections of the two rows' words.
-// resolved: the snapshot component w is known to have joined (-1: none).
-__device__ void round_row_words(const LabelArgs &a, int w, uint64_t rw, int c, int64_t t_from, int64_t t_to,
-                                int resolved, unsigned &tests, unsigned &passed) {
+// Row w's part of a full round on row words, over its candidate tiles, 64 a
+// step (ascending column tile, so entries come in list order); tiles whose
+// points share a rank that is not above w's, or that w has joined, are skipped
+// without reading their bits; tests are bitset intersections of the two rows'
+// words.
+__device__ void round_row_words(const LabelArgs &a, int w, uint64_t rw, int c, unsigned &tests, unsigned &passed) {
     const int lane = threadIdx.x & 63;
     const WordRow A = word_row(a, w);
     const int64_t dw = deg_of(a, w);
-    t_to = min(t_to, A.len);
-    for (int64_t t0 = t_from; t0 < t_to; t0 += 64) {
+    int resolved = -1;  // the snapshot component w is known to have joined
+    for (int64_t t0 = 0; t0 < A.len; t0 += 64) {
         const int64_t t = t0 + lane;
         uint64_t v = 0ull, tr = 0ull;
         int C = 0;
-        if (t < t_to) {
+        if (t < A.len) {
             // the tile id with the pair's flag, the tile's rank with the word
             C = A.tile[t];
             v = word_at(A, t);
@@ -620,12 +637,12 @@ __global__ __launch_bounds__(256) void k_round_b(LabelArgs a) {
     if (a.cand_max && rw >= a.cand_max[w >> 6]) return;
     const int c = csim_of(a, w);
     unsigned tests = 0, passed = 0;
-    int resolved = -1;  // last snapshot component found joined to w
     if constexpr (WORDS) {
-        round_row_words(a, (int)w, rw, c, 0, INT64_MAX, resolved, tests, passed);
+        round_row_words(a, (int)w, rw, c, tests, passed);
         add_stats(a, tests, passed, 1);
         return;
     }
+    int resolved = -1;  // last snapshot component found joined to w
     // four 64-entry windows per step: their loads and rank lookups are issued
     // together, so a row's scan waits on one memory round trip per 256 entries
     const int64_t b = a.row_ptr[w], e = a.row_ptr[w + 1];
@@ -688,54 +705,259 @@ __device__ __forceinline__ uint64_t columns_above(uint64_t rk, uint64_t rw, int 
     return bits;
 }
 
-// Full round on a spatial graph's tile-pair words, `split` waves per row tile
-// (lane r owns row w = 64R + r; wave q of the tile takes the q-th of `split`
-// equal parts of its candidate pairs), with k_round_b's ownership and skip
-// rules: an edge is examined by the endpoint of lower snapshot rank, rows at
-// or above the tile's candidate maximum own none, and a row drops every column
-// of a component it has joined (per wave: the skip is only a saving, every
-// test re-checks with two finds).  The pairs are walked once for all 64 rows
-// -- pair k's 64 row words are one contiguous 512-byte load, 8 pairs in
+// Column tiles that hold words of both of two row tiles, as pairs of positions
+// in the two tiles' candidate lists, written to buf (at most kMatchCap a
+// chunk) by the whole wave; a chunk continues where the last one ended.
+// 64-wide windows of both ascending lists advance like a two-pointer merge,
+// each lane looking its B tile up in the A window by a shuffle binary search.
+constexpr int kMatchCap = 256;
+
+struct TileMatch {
+    const int32_t *ta, *tb;   // column tiles of the two lists
+    const uint8_t *za, *zb;   // flags of the non-empty pairs
+    int64_t la, lb;
+    int64_t ia = 0, ib = 0;   // first positions not yet matched
+    __device__ __forceinline__ bool end() const { return ia >= la || ib >= lb; }
+    __device__ __forceinline__ void rewind() { ia = ib = 0; }
+    __device__ int next(int2 *buf) {
+        const int lane = threadIdx.x & 63;
+        const uint64_t below = (1ull << lane) - 1ull;
+        int m = 0;
+        while (!end() && m + 64 <= kMatchCap) {
+            bool hit;
+            int64_t pa, pb = ib + lane;
+            int64_t na, nb;
+            if (ta == tb) {  // the rows of one tile
+                hit = pb < lb && zb[pb] != 0;
+                pa = pb;
+                na = nb = ib + 64;
+            } else {
+                const int va = (int)min<int64_t>(64, la - ia), vb = (int)min<int64_t>(64, lb - ib);
+                const int a = lane < va ? ta[ia + lane] : INT_MAX;
+                const int b = lane < vb ? tb[ib + lane] : INT_MAX;
+                const int fa = lane < va ? (int)za[ia + lane] : 0;
+                const int fb = lane < vb ? (int)zb[ib + lane] : 0;
+                const int top = min(__shfl(a, va - 1, 64), __shfl(b, vb - 1, 64));
+                int lo = 0, hi = va;
+#pragma unroll
+                for (int step = 0; step < 7; ++step) {
+                    const int mid = (lo + hi) >> 1;
+                    const int am = __shfl(a, min(mid, 63), 64);
+                    if (lo < hi) {
+                        if (am < b) lo = mid + 1;
+                        else hi = mid;
+                    }
+                }
+                const int found = __shfl(a, min(lo, 63), 64), ffound = __shfl(fa, min(lo, 63), 64);
+                hit = lane < vb && b <= top && lo < va && found == b && ffound != 0 && fb != 0;
+                pa = ia + lo;
+                na = ia + __popcll(__ballot(lane < va && a <= top));
+                nb = ib + __popcll(__ballot(lane < vb && b <= top));
+            }
+            const uint64_t hm = __ballot(hit);
+            if (hit) buf[m + __popcll(hm & below)] = make_int2((int)pa, (int)pb);
+            m += __popcll(hm);
+            ia = na;
+            ib = nb;
+        }
+        return m;
+    }
+};
+
+// The wave's LDS writes before, its reads after (one wave's LDS accesses run
+// in order; this keeps the compiler from reordering them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One row tile of the full round, as its wave holds it (lane r = row 64R + r).
+struct RoundRows {
+    int64_t R;
+    int64_t kb, ke;      // the tile's candidate pairs
+    uint64_t rw;         // the row's snapshot rank (0: not core)
+    int c;
+    int resolved = -1;   // last snapshot component this row was found joined to
+    unsigned tests = 0, passed = 0;
+};
+
+// The edges of tile pair (R, C), C the column tile at position k of R's list:
+// v holds the row words (0 for rows that own nothing), tr the tile's common
+// rank (all ones: mixed, rk then holds lane b's rank of column b).  Edges to
+// higher ranks whose endpoints are still apart are tested together: up to 64,
+// 64 / E lanes each (one edge a row; up to eight columns of a row when few
+// rows are open).  Both rows' words over the tiles common to R's and C's lists
+// (found once per tile pair) are and-ed and their bits counted, so 64 tests
+// share one walk of the lists, and their words the same cache lines.  Stops
+// after `budget` such batches (it is counted down); true when no edge is left.
+__device__ bool round_pair(const LabelArgs &a, RoundRows &rr, int C, uint64_t v, uint64_t tr, uint64_t rk, int &budget,
+                           int2 *match, uint16_t *edge) {
+    const int lane = threadIdx.x & 63;
+    const int w = (int)(rr.R * 64 + lane);
+    const bool common = tr != ~0ull;
+    uint64_t bits;
+    if (common) bits = (tr > rr.rw && (int)(uint32_t)tr != rr.resolved) ? v : 0ull;
+    else bits = columns_above(rk, rr.rw, rr.resolved) & v;
+    TileMatch tm;
+    int n_match = -1;  // tiles common to R and C (-1: not matched yet)
+    while (__ballot(bits != 0ull)) {
+        const int col = bits ? __ffsll((unsigned long long)bits) - 1 : 0;
+        const uint64_t rb = common ? tr : __shfl(rk, col, 64);
+        bool changed = false, open = false;
+        if (bits) {
+            changed = uf_find(a.parent, w) == uf_find(a.parent, C * 64 + col);
+            open = !changed;
+        }
+        if (changed) rr.resolved = (int)(uint32_t)rb;
+        const uint64_t need = __ballot(open);
+        if (need) {
+            if (budget-- <= 0) return false;
+            const int rows = __popcll(need);
+            const int quota = rows >= 32 ? 1 : min(8, 32 / rows);
+            const int mine = open ? min(__popcll(bits), quota) : 0;
+            const int incl = wave_incl_scan(mine), off = incl - mine;
+            const int E = __builtin_amdgcn_readlane(incl, 63);
+            uint64_t left = bits;
+            for (int x = 0; x < mine; ++x) {
+                edge[off + x] = (uint16_t)((lane << 6) | (__ffsll((unsigned long long)left) - 1));
+                left &= left - 1;
+            }
+            if (n_match < 0) {
+                const int64_t kc = a.tp_ptr[C];
+                tm.ta = a.tp_col + rr.kb;
+                tm.za = a.pair_nz + rr.kb;
+                tm.la = rr.ke - rr.kb;
+                tm.tb = a.tp_col + kc;
+                tm.zb = a.pair_nz + kc;
+                tm.lb = a.tp_ptr[C + 1] - kc;
+                n_match = tm.next(match);
+            }
+            wave_lds_fence();
+            int shift = 6;  // 2^shift lanes per edge
+            while ((E << shift) > 64) --shift;
+            const int grp = lane >> shift, sub = lane & ((1 << shift) - 1);
+            const bool on = grp < E;
+            const int ed = on ? edge[grp] : 0;
+            const int er = ed >> 6, ec = ed & 63;
+            const uint64_t *__restrict__ wa = a.mask + rr.kb * 64 + er;
+            const uint64_t *__restrict__ wb = a.mask + (tm.tb - a.tp_col) * 64 + ec;
+            int cnt = 0, sum = 0;
+            bool dec = !on || rr.c <= 0;
+            bool again = false;  // the lists took more than one chunk
+            for (;;) {
+                constexpr int kU = 8;
+                for (int t0 = 0; t0 < n_match && __ballot(!dec); t0 += kU << shift) {
+                    uint64_t x[kU], y[kU];
+#pragma unroll
+                    for (int z = 0; z < kU; ++z) {
+                        const int t = t0 + (z << shift) + sub;
+                        x[z] = y[z] = 0ull;
+                        if (!dec && t < n_match) {
+                            const int2 m = match[t];
+                            x[z] = wa[(int64_t)m.x * 64];
+                            y[z] = wb[(int64_t)m.y * 64];
+                        }
+                    }
+#pragma unroll
+                    for (int z = 0; z < kU; ++z) cnt += __popcll(x[z] & y[z]);
+                    sum = cnt;
+                    for (int o = 0; o < shift; ++o) sum += __shfl_xor(sum, 1 << o, 64);
+                    dec = dec || sum >= rr.c;
+                }
+                if (tm.end() || __ballot(!dec) == 0ull) break;
+                wave_lds_fence();
+                n_match = tm.next(match);
+                again = true;
+                wave_lds_fence();
+            }
+            if (again) {  // the next test of this tile pair starts over
+                tm.rewind();
+                n_match = -1;
+            }
+            const bool pass = on && (rr.c <= 0 || sum >= rr.c);
+            if (pass && sub == 0) uf_union(a.parent, (int)(rr.R * 64 + er), C * 64 + ec);
+            const uint64_t pm = __ballot(pass && sub == 0);
+            rr.tests += (unsigned)E;
+            rr.passed += (unsigned)__popcll(pm);
+            // each row takes up the results of its edges
+            uint64_t todo = bits;
+            for (int x = 0; x < quota; ++x) {
+                const int cx = todo ? __ffsll((unsigned long long)todo) - 1 : 0;
+                const uint64_t rx = common ? tr : __shfl(rk, cx, 64);
+                if (x < mine) {
+                    if ((pm >> ((off + x) << shift)) & 1ull) {
+                        changed = true;
+                        rr.resolved = (int)(uint32_t)rx;
+                    }
+                    todo &= todo - 1;
+                }
+            }
+            if (open) bits = left;
+            wave_lds_fence();
+        }
+        // a joined component: its remaining columns are joined as well
+        if (__ballot(changed)) {
+            if (common) {
+                if (changed) bits = 0ull;
+            } else {
+                if (changed && !open) bits &= bits - 1;
+                bits &= columns_above(rk, rr.rw, rr.resolved);
+            }
+        }
+    }
+    return true;
+}
+
+// Full round on a graph's tile-pair words, `split` waves per row tile (lane r
+// owns row w = 64R + r; wave q of the tile takes the q-th of `split` equal
+// parts of its candidate pairs), with k_round_b's ownership and skip rules: an
+// edge is examined by the endpoint of lower snapshot rank, rows at or above
+// the tile's candidate maximum own none, and a row drops every column of a
+// component it has joined (per wave: the skip is only a saving, every row
+// checks with two finds before a test).  The pairs are walked once for all 64
+// rows -- pair k's 64 row words are one contiguous 512-byte load, 8 pairs in
 // flight -- and the rank filter and the already-joined check run for all rows
-// in parallel.  An edge whose endpoints are still apart needs a wave-wide bitset
-// test (test_and_link_words): the wave runs kInlineTests of them itself, then
-// hands each row that still has one, with the rest of the wave's pairs, to
-// k_round_queue (one wave per row there, as k_round_b), so no wave runs the
-// tests of many rows one after another; when the queue is full (or absent)
-// the wave tests every edge itself.
+// in parallel (round_pair).  A wave runs kInlineTests batches of tests itself:
+// a pass usually joins the components of the other open edges too.  After
+// them, a pair with open edges goes to a queue ({R, pair}; one counter update
+// per 64 pairs) that k_round_queue serves, one wave per pair, so that no wave
+// runs the tests of many pairs one after another; a full queue falls back to
+// tests here.
+// Bound by the latency of dependent loads.  Tested one edge per wave from a
+// queue of rows, the round took 622 us at n = 1e6, d = 3, 708 us at n = 2e5,
+// d = 64 and 182 us at n = 3e4, d = 3; batched by tile pair
+// 284, 198 and 72 us.
 __global__ __launch_bounds__(256) void k_round_tile(LabelArgs a, int64_t n_tiles, int split) {
     a = slice(a);
-    const int lane = threadIdx.x & 63;
-    const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    __shared__ int2 s_match[4][kMatchCap];
+    __shared__ uint16_t s_edge[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t g = (int64_t)blockIdx.x * 4 + wave;
     if (g >= n_tiles * split) return;
     const int64_t gR = g / split;
     const int q = (int)(g - gR * split);
-    const int64_t R = a.tile_order ? (int64_t)a.tile_order[gR] : gR;
-    const int64_t w = R * 64 + lane;
-    const uint64_t rw = w < a.n ? a.rank[w] : 0ull;
-    const uint64_t cmax = a.cand_max ? a.cand_max[R] : ~0ull;
-    const bool active = rw != 0ull && rw < cmax;
+    RoundRows rr;
+    rr.R = a.tile_order ? (int64_t)a.tile_order[gR] : gR;
+    const int64_t w = rr.R * 64 + lane;
+    rr.rw = w < a.n ? a.rank[w] : 0ull;
+    const uint64_t cmax = a.cand_max ? a.cand_max[rr.R] : ~0ull;
+    const bool active = rr.rw != 0ull && rr.rw < cmax;
     const uint64_t act = __ballot(active);
     if (act == 0ull) return;
     // a column tile whose points share a rank not above every active row's has no candidate
-    uint64_t rmin = active ? rw : ~0ull;
+    uint64_t rmin = active ? rr.rw : ~0ull;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         const uint64_t o = __shfl_xor(rmin, off, 64);
         rmin = o < rmin ? o : rmin;
     }
-    const int c = csim_of(a, R * 64);
-    unsigned tests = 0, passed = 0;
-    int resolved = -1;  // last snapshot component this row was found joined to
-    bool live = active;  // false once the row is queued
-    bool rq_full = false;
-    // wave-wide tests a wave runs itself before it queues open rows: a passing
-    // test usually joins the components the other rows' open edges connect
-    constexpr unsigned kInlineTests = 2;
-    const int64_t kb0 = a.tp_ptr[R], ke0 = a.tp_ptr[R + 1];
-    const int64_t per = (ke0 - kb0 + split - 1) / split;
-    const int64_t kb = kb0 + q * per, ke = min(ke0, kb + per);
-    constexpr int kInFlight = 8;
+    rr.c = csim_of(a, rr.R * 64);
+    rr.kb = a.tp_ptr[rr.R];
+    rr.ke = a.tp_ptr[rr.R + 1];
+    const int64_t per = (rr.ke - rr.kb + split - 1) / split;
+    const int64_t kb = rr.kb + q * per, ke = min(rr.ke, kb + per);
+    constexpr int kInFlight = 8, kInlineTests = 2;
+    int budget = kInlineTests;
     for (int64_t k0 = kb; k0 < ke; k0 += 64) {
         const int64_t kk = k0 + lane;
         int C = 0;
@@ -746,7 +968,7 @@ __global__ __launch_bounds__(256) void k_round_tile(LabelArgs a, int64_t n_tiles
             tr = a.tile_rank ? a.tile_rank[C] : ~0ull;
             want = tr == ~0ull || tr > rmin;
         }
-        uint64_t wm = __ballot(want);
+        uint64_t wm = __ballot(want), open = 0ull;
         while (wm) {
             int idx[kInFlight];
 #pragma unroll
@@ -761,121 +983,92 @@ __global__ __launch_bounds__(256) void k_round_tile(LabelArgs a, int64_t n_tiles
                 rk[u] = 0ull;
                 if (idx[u] >= 0) {
                     const int64_t Cu = __builtin_amdgcn_readlane(C, idx[u]);
-                    if (live) v[u] = a.mask[(k0 + idx[u]) * 64 + lane];
+                    if (active) v[u] = a.mask[(k0 + idx[u]) * 64 + lane];
                     if (readlane_u64(tr, idx[u]) == ~0ull && Cu * 64 + lane < a.n) rk[u] = a.rank[Cu * 64 + lane];
                 }
             }
-#pragma unroll
+#pragma unroll 1
             for (int u = 0; u < kInFlight; ++u) {
-                if (!live) v[u] = 0ull;  // queued by an earlier pair of this batch
-                if (idx[u] < 0 || __ballot(v[u] != 0ull) == 0ull) continue;
-                const int Cu = __builtin_amdgcn_readlane(C, idx[u]);
-                const uint64_t tru = readlane_u64(tr, idx[u]);
-                const bool common = tru != ~0ull;
-                uint64_t bits;
-                if (common) bits = (tru > rw && (int)(uint32_t)tru != resolved) ? v[u] : 0ull;
-                else bits = columns_above(rk[u], rw, resolved) & v[u];
-                while (__ballot(bits != 0ull)) {
-                    const int col = bits ? __ffsll((unsigned long long)bits) - 1 : 0;
-                    const uint64_t rb = common ? tru : __shfl(rk[u], col, 64);
-                    int j = -1;
-                    bool joined = false;
-                    if (bits) {
-                        bits &= bits - 1;
-                        j = Cu * 64 + col;
-                        joined = uf_find(a.parent, (int)w) == uf_find(a.parent, j);
+                uint64_t vu = 0ull, rku = 0ull;
+                int iu = -1;
+                // (a private array indexed at run time would live in memory)
+#pragma unroll
+                for (int x = 0; x < kInFlight; ++x)
+                    if (x == u) {
+                        vu = v[x];
+                        rku = rk[x];
+                        iu = idx[x];
                     }
-                    bool changed = joined;
-                    uint64_t need = __ballot(j >= 0 && !joined);
-                    while (need) {
-                        if (tests >= kInlineTests && a.rq && !rq_full) {
-                            // queue the rows still open, from this pair on
-                            unsigned long long base = 0;
-                            if (lane == 0) base = atomicAdd(a.rq_len, (unsigned long long)__popcll(need));
-                            base = __shfl(base, 0, 64);
-                            const bool mine = ((need >> lane) & 1ull) != 0ull;
-                            const unsigned long long slot = base + __popcll(need & ((1ull << lane) - 1ull));
-                            const bool queued = mine && slot < (unsigned long long)a.rq_cap;
-                            if (queued) {
-                                a.rq[slot] = make_int4((int)w, (int)(k0 + idx[u] - kb0), (int)(ke - kb0), resolved);
-                                live = false;
-                                bits = 0ull;
-                            }
-                            rq_full = __ballot(mine && !queued) != 0ull;
-                            need &= ~__ballot(queued);
-                            if (!need) break;
-                        }
-                        const int src = __ffsll((unsigned long long)need) - 1;
-                        need &= need - 1;
-                        const int ws = (int)(R * 64 + src);
-                        const int js = __builtin_amdgcn_readlane(j, src);
-                        if (test_and_link_words(a, ws, js, word_row(a, ws), deg_of(a, ws), c, tests, passed) &&
-                            lane == src)
-                            changed = true;
-                    }
-                    // a joined component: its remaining columns are joined as well
-                    if (changed) resolved = (int)(uint32_t)rb;
-                    if (__ballot(changed)) {
-                        if (common) {
-                            if (changed) bits = 0ull;
-                        } else {
-                            bits &= columns_above(rk[u], rw, resolved);
-                        }
-                    }
-                }
+                if (iu < 0 || __ballot(vu != 0ull) == 0ull) continue;
+                if (!round_pair(a, rr, __builtin_amdgcn_readlane(C, iu), vu, readlane_u64(tr, iu), rku, budget,
+                                s_match[wave], s_edge[wave]))
+                    open |= 1ull << iu;
+            }
+        }
+        if (open) {
+            unsigned long long base = 0;
+            if (lane == 0) base = atomicAdd(a.rq_len, (unsigned long long)__popcll(open));
+            base = __shfl(base, 0, 64);
+            const bool mine = ((open >> lane) & 1ull) != 0ull;
+            const unsigned long long slot = base + __popcll(open & ((1ull << lane) - 1ull));
+            const bool queued = mine && slot < (unsigned long long)a.rq_cap;
+            if (queued) a.rq[slot] = make_int2((int)rr.R, (int)(kk - rr.kb));
+            open &= ~__ballot(queued);
+            while (open) {
+                const int iu = __ffsll((unsigned long long)open) - 1;
+                open &= open - 1;
+                const int Cu = __builtin_amdgcn_readlane(C, iu);
+                const uint64_t vu = active ? a.mask[(k0 + iu) * 64 + lane] : 0ull;
+                const uint64_t rku = (int64_t)Cu * 64 + lane < a.n ? a.rank[(int64_t)Cu * 64 + lane] : 0ull;
+                int all = INT_MAX;
+                (void)round_pair(a, rr, Cu, vu, readlane_u64(tr, iu), rku, all, s_match[wave], s_edge[wave]);
             }
         }
     }
-    add_stats(a, tests, passed, q == 0 ? (unsigned)__popcll(act) : 0u);
+    add_stats(a, rr.tests, rr.passed, q == 0 ? (unsigned)__popcll(act) : 0u);
 }
 
-// The rows k_round_tile queued, one wave each (grid-stride): the row's
-// candidate pairs from the queued one to the end of its wave's part, with the
-// per-row walk of k_round_b.
+// The tile pairs k_round_tile queued, one wave each (grid-stride).
 __global__ __launch_bounds__(256) void k_round_queue(LabelArgs a) {
     a = slice(a);
+    __shared__ int2 s_match[4][kMatchCap];
+    __shared__ uint16_t s_edge[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t nq = (int64_t)min<unsigned long long>(*a.rq_len, (unsigned long long)a.rq_cap);
     const int64_t waves = (int64_t)gridDim.x * 4;
-    for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); q < nq; q += waves) {
-        const int4 e = a.rq[q];
-        unsigned tests = 0, passed = 0;
-        round_row_words(a, e.x, a.rank[e.x], csim_of(a, e.x), e.y, e.z, e.w, tests, passed);
-        add_stats(a, tests, passed);
+    for (int64_t q = (int64_t)blockIdx.x * 4 + wave; q < nq; q += waves) {
+        const int2 e = a.rq[q];
+        RoundRows rr;
+        rr.R = uniform(e.x);
+        rr.kb = a.tp_ptr[rr.R];
+        rr.ke = a.tp_ptr[rr.R + 1];
+        const int64_t k = rr.kb + uniform(e.y);
+        const int C = uniform(a.tp_col[k]);
+        const int64_t w = rr.R * 64 + lane, j = (int64_t)C * 64 + lane;
+        rr.rw = w < a.n ? a.rank[w] : 0ull;
+        const uint64_t v = rr.rw != 0ull ? a.mask[k * 64 + lane] : 0ull;
+        const uint64_t rk = j < a.n ? a.rank[j] : 0ull;
+        const uint64_t tr = a.tile_rank ? a.tile_rank[C] : ~0ull;
+        rr.c = csim_of(a, rr.R * 64);
+        int all = INT_MAX;
+        (void)round_pair(a, rr, C, v, tr, rk, all, s_match[wave], s_edge[wave]);
+        add_stats(a, rr.tests, rr.passed);
     }
 }
 
-// Waves per row tile for k_round_tile: about 64 candidate pairs each.
+// Queue entries of one full round over that many tile pairs.
+static int64_t round_queue_cap(int64_t n_tile_pairs, int n_c) {
+    return std::min<int64_t>(std::max<int64_t>(n_tile_pairs, 1), ((int64_t)1 << 21) / n_c);
+}
+
+// Waves per row tile for k_round_tile: one per 128 candidate pairs, and with few
+// tiles enough for about 4096 waves of at least 8 pairs.  (Twice and half as
+// many waves were within 2 % of this from n = 1e3 to 1e6.)
 static int round_split(int64_t n_tile_pairs, int64_t n_tiles) {
     if (n_tiles <= 0) return 1;
-    const int64_t per_tile = (n_tile_pairs + n_tiles - 1) / n_tiles;
-    return (int)std::min<int64_t>(32, std::max<int64_t>(1, (per_tile + 63) / 64));
-}
-
-// Largest snapshot rank among the core points of each tile (0: none), and the
-// tile's common rank: the rank of all its points when they share one (a
-// non-core point has rank 0), all ones when they differ.
-__global__ void k_tile_rank_max(const uint64_t *__restrict__ rank, int64_t n, int64_t n_tiles,
-                                uint64_t *__restrict__ tmax, uint64_t *__restrict__ tcommon) {
-    rank += (int64_t)blockIdx.y * n;  // cutoff pair blockIdx.y (one pair: 0)
-    tmax += (int64_t)blockIdx.y * n_tiles;
-    tcommon += (int64_t)blockIdx.y * n_tiles;
-    const int lane = threadIdx.x & 63;
-    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= n_tiles) return;
-    const int64_t w = t * 64 + lane;
-    const bool real = w < n;
-    const uint64_t mine = real ? rank[w] : 0ull;
-    uint64_t v = mine;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const uint64_t o = __shfl_xor(v, off, 64);
-        v = o > v ? o : v;
-    }
-    const bool same = __ballot(real && mine != v) == 0ull;  // every real point has the largest rank
-    if (lane == 0) {
-        tmax[t] = v;
-        tcommon[t] = same ? v : ~0ull;
-    }
+    const int64_t per_tile = ceil_div(n_tile_pairs, n_tiles);
+    const int64_t want = std::max(ceil_div(per_tile, 128), std::min(ceil_div(4096, n_tiles), ceil_div(per_tile, 8)));
+    return (int)std::min<int64_t>(64, std::max<int64_t>(1, want));
 }
 
 // Largest rank over the candidate column tiles of each row tile, one
@@ -911,26 +1104,40 @@ __global__ __launch_bounds__(256) void k_cand_max(const uint64_t *__restrict__ t
     }
 }
 
-__global__ void k_snapshot(const uint8_t *core, const int *parent, const int32_t *cnt, int64_t n, uint64_t *rank) {
+// rank[w] = (component size << 32 | root) of core points, 0 otherwise; with a
+// tile structure also, per tile of 64 points, the largest rank (0: no core
+// point) and the tile's common rank: the rank of all its points when they
+// share one, all ones when they differ.
+__global__ __launch_bounds__(256) void k_snapshot(const uint8_t *core, const int *parent, const int32_t *cnt, int64_t n,
+                                                  uint64_t *rank, int64_t n_tiles, uint64_t *tmax, uint64_t *tcommon) {
     const int64_t off = (int64_t)blockIdx.y * n;
-    core += off;
-    parent += off;
-    cnt += off;
-    rank += off;
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= n) return;
-    const int r = parent[w];
-    rank[w] = core[w] ? (((uint64_t)(uint32_t)cnt[r] << 32) | (uint32_t)r) : 0ull;
+    const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    uint64_t mine = 0ull;
+    if (w < n) {
+        const int r = parent[off + w];
+        mine = core[off + w] ? (((uint64_t)(uint32_t)cnt[off + r] << 32) | (uint32_t)r) : 0ull;
+        rank[off + w] = mine;
+    }
+    const int64_t t = w >> 6;  // one wave per tile
+    if (t >= n_tiles) return;
+    uint64_t v = mine;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        const uint64_t x = __shfl_xor(v, o, 64);
+        v = x > v ? x : v;
+    }
+    const bool same = __ballot(w < n && mine != v) == 0ull;  // every real point has the largest rank
+    if ((threadIdx.x & 63) == 0) {
+        tmax[(int64_t)blockIdx.y * n_tiles + t] = v;
+        tcommon[(int64_t)blockIdx.y * n_tiles + t] = same ? v : ~0ull;
+    }
 }
 
 // Flatten: every entry points at its root afterwards.  The walk only reads
 // (entries of other threads may change meanwhile, but only towards their
 // roots) and each thread writes only its own entry, so no write can leave an
 // entry below its root.
-__global__ void k_compress(int *parent, int64_t n) {
-    parent += (int64_t)blockIdx.y * n;
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= n) return;
+__device__ __forceinline__ int flatten(int *parent, int64_t w) {
     int x = (int)w;
     int p = atomic_load_relaxed(&parent[x]);
     while (p != x) {
@@ -938,32 +1145,33 @@ __global__ void k_compress(int *parent, int64_t n) {
         p = atomic_load_relaxed(&parent[x]);
     }
     __hip_atomic_store(&parent[w], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return x;
 }
 
-// k_compress that also lists the core points that are roots afterwards
-// (one atomic per wave), for k_hook_roots_list.
-__global__ void k_compress_roots(int *parent, const uint8_t *__restrict__ core, int64_t n, int32_t *__restrict__ roots,
-                                 unsigned int *__restrict__ n_roots) {
-    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool root = false;
-    if (w < n) {
-        int x = (int)w;
-        int p = atomic_load_relaxed(&parent[x]);
-        while (p != x) {
-            x = p;
-            p = atomic_load_relaxed(&parent[x]);
-        }
-        __hip_atomic_store(&parent[w], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        root = x == (int)w && core[w] != 0;
-    }
+// Flattening that also lists the core points that are roots afterwards, for
+// k_hook_roots_list; one counter update per workgroup of 1024 points (the
+// counter is a single address).
+__global__ __launch_bounds__(1024) void k_compress_roots(int *parent, const uint8_t *__restrict__ core, int64_t n,
+                                                         int32_t *__restrict__ roots,
+                                                         unsigned int *__restrict__ n_roots) {
+    __shared__ unsigned s_cnt[16], s_base;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t w = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+    const bool root = w < n && flatten(parent, w) == (int)w && core[w] != 0;
     const uint64_t m = __ballot(root);
-    if (m) {
-        const int lane = threadIdx.x & 63;
-        unsigned base = 0;
-        if (lane == 0) base = atomicAdd(n_roots, (unsigned)__popcll(m));
-        base = __shfl(base, 0, 64);
-        if (root) roots[base + __popcll(m & ((1ull << lane) - 1ull))] = (int32_t)w;
+    if (lane == 0) s_cnt[wave] = (unsigned)__popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned total = 0;
+        for (int q = 0; q < 16; ++q) {
+            const unsigned x = s_cnt[q];
+            s_cnt[q] = total;
+            total += x;
+        }
+        s_base = total ? atomicAdd(n_roots, total) : 0u;
     }
+    __syncthreads();
+    if (root) roots[s_base + s_cnt[wave] + __popcll(m & ((1ull << lane) - 1ull))] = (int32_t)w;
 }
 
 // Lanes sharing a key are combined before one atomic per distinct key (points
@@ -986,11 +1194,12 @@ __device__ __forceinline__ void wave_add_by_key(int32_t *cnt, int32_t *mins, boo
     }
 }
 
-// Per-key sums over consecutive points: a wave walks kRunSteps steps of 64
+// Per-key sums over consecutive points: a wave walks `steps` steps of 64
 // points and keeps one run (key, count, minimum) while every active lane of a
 // step has the run's key, so a large component costs one atomic per run, not
-// one per wave (same-address atomics serialize).
-constexpr int kRunSteps = 16;
+// one per wave (same-address atomics serialize).  Few points take few steps:
+// 16 steps of dependent loads on 8 workgroups took 22 and 35 us at n = 3e4.
+static int run_steps(int64_t n) { return (int)std::min<int64_t>(16, std::max<int64_t>(1, ceil_div(n, 64 * 2048))); }
 
 struct KeyRun {
     int key = -1;
@@ -1029,64 +1238,75 @@ __device__ __forceinline__ void run_add(KeyRun &run, int32_t *cnt, int32_t *mins
     }
 }
 
-__device__ __forceinline__ int64_t run_base() {
-    return ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * (64 * kRunSteps);
+__device__ __forceinline__ int64_t run_base(int steps) {
+    return ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * (64 * steps);
 }
 
-__global__ __launch_bounds__(256) void k_root_count(const uint8_t *core, const int *parent, int64_t n,
-                                                    int32_t *cnt) {
-    const int64_t off = (int64_t)blockIdx.y * n;
-    core += off;
-    parent += off;
-    cnt += off;
-    const int64_t base = run_base();
+// Flattens the forest and counts the core points of every component; the
+// components go into the striped statistics.
+__global__ __launch_bounds__(256) void k_root_count(LabelArgs a, int32_t *cnt, int steps) {
+    a = slice(a);
+    cnt += (int64_t)blockIdx.y * a.n;
+    const int64_t base = run_base(steps);
     KeyRun run;
-    for (int it = 0; it < kRunSteps; ++it) {
+    unsigned roots = 0;
+    for (int it = 0; it < steps; ++it) {
         const int64_t w = base + it * 64 + __lane_id();
-        const bool active = w < n && core[w];
-        run_add(run, cnt, nullptr, active, active ? parent[w] : 0, 0);
+        int r = 0;
+        bool active = false;
+        if (w < a.n) {
+            r = flatten(a.parent, w);
+            active = a.core[w] != 0;
+        }
+        run_add(run, cnt, nullptr, active, r, 0);
+        roots += (unsigned)__popcll(__ballot(active && r == (int)w));
     }
     run_flush(run, cnt, nullptr);
-}
-
-__global__ void k_count_roots(const int32_t *cnt, int64_t n, unsigned long long *roots) {
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t b = __ballot(w < n && cnt[w] > 0);
-    if ((threadIdx.x & 63) == 0 && b) atomicAdd(roots, (unsigned long long)__popcll(b));
+    add_stats(a, 0, 0, 0, roots);
 }
 
 // ------------------------------------------------------------------ labels
 
-__global__ __launch_bounds__(256) void k_comp_stats(const uint8_t *core, const int *parent, const int32_t *perm,
-                                                    int64_t n, int32_t *cmin, int32_t *csize,
-                                                    unsigned long long *counters) {
+// Flattens the forest; size and smallest caller index of every component, core
+// points and components counted into counters[0] and [1].
+__global__ __launch_bounds__(256) void k_comp_stats(const uint8_t *core, int *parent, const int32_t *perm, int64_t n,
+                                                    int32_t *cmin, int32_t *csize, unsigned long long *counters,
+                                                    int steps) {
     const int64_t off = (int64_t)blockIdx.y * n;
     core += off;
     parent += off;
     cmin += off;
     csize += off;
     counters += 8 * blockIdx.y;
-    const int64_t base = run_base();
+    const int64_t base = run_base(steps);
     KeyRun run;
-    unsigned long long nc = 0, nr = 0;
-    for (int it = 0; it < kRunSteps; ++it) {
+    unsigned nc = 0, nr = 0;
+    for (int it = 0; it < steps; ++it) {
         const int64_t w = base + it * 64 + __lane_id();
-        bool is_core = false, is_root = false;
+        bool is_core = false;
         int r = 0, orig = 0;
-        if (w < n && core[w]) {
-            is_core = true;
-            r = parent[w];
-            is_root = r == (int)w;
-            orig = perm ? perm[w] : (int32_t)w;
+        if (w < n) {
+            r = flatten(parent, w);
+            is_core = core[w] != 0;
+            if (is_core) orig = perm ? perm[w] : (int32_t)w;
         }
         run_add(run, csize, cmin, is_core, r, orig);
-        nc += __popcll(__ballot(is_core));
-        nr += __popcll(__ballot(is_root));
+        nc += (unsigned)__popcll(__ballot(is_core));
+        nr += (unsigned)__popcll(__ballot(is_core && r == (int)w));
     }
     run_flush(run, csize, cmin);
+    // one update per workgroup: the counters are single addresses
+    __shared__ unsigned s_nc[4], s_nr[4];
     if (__lane_id() == 0) {
-        if (nc) atomicAdd(&counters[0], nc);
-        if (nr) atomicAdd(&counters[1], nr);
+        s_nc[threadIdx.x >> 6] = nc;
+        s_nr[threadIdx.x >> 6] = nr;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        nc = s_nc[0] + s_nc[1] + s_nc[2] + s_nc[3];
+        nr = s_nr[0] + s_nr[1] + s_nr[2] + s_nr[3];
+        if (nc) atomicAdd(&counters[0], (unsigned long long)nc);
+        if (nr) atomicAdd(&counters[1], (unsigned long long)nr);
     }
 }
 
@@ -1350,9 +1570,9 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
     Scratch<uint64_t> rank(ctx, n);
     Scratch<int> parent(ctx, n);
     // the pass's small counters in one buffer, zeroed by one fill kernel:
-    // counters (8), striped test statistics (4 per slot), then one 8-byte slot
-    // each for the hook queue length, the round queue length and the root count
-    constexpr int64_t kSmallSlots = 8 + 4 * kStatSlots + 3;
+    // counters (8), striped test statistics (4 per slot), the hook and the round
+    // queue length, then one root count per root hooking pass
+    const int64_t kSmallSlots = 8 + 4 * kStatSlots + 2 + std::max(req.root_passes, 0);
     Scratch<unsigned long long> small(ctx, kSmallSlots);
     fill_u64(ctx, small.p, 0ull, kSmallSlots);
     unsigned long long *const counters_p = small.p, *const tstats_p = small.p + 8;
@@ -1418,12 +1638,17 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
     }
     if (!words && !req.col) throw InvalidArg{"the sorted-list merge needs the neighbour lists"};
 
-    k_init<<<blocks_for(n), 256, 0, s>>>(a, req.consider, req.perm);
+    Scratch<int32_t> cmin(ctx, n), csize(ctx, n);
+    std::unique_ptr<Scratch<int32_t>> snewlab;
+    if (req.sort) snewlab.reset(new Scratch<int32_t>(ctx, n));
+    std::unique_ptr<Scratch<int32_t>> cnt(new Scratch<int32_t>(ctx, n));  // until the snapshot
+    k_init<<<blocks_for(n), 256, 0, s>>>(a, req.consider, req.perm,
+                                         ComponentArrays{cnt->p, cmin.p, csize.p, req.sort ? snewlab->p : nullptr});
     CNN_HIP(hipGetLastError());
     CNN_HIP(hipEventRecord(ctx->ev[8], s));
     if (words && a.mask) {
-        // adjacent rows per row tile, then the rows left, one wave each
-        Scratch<int32_t> hq(ctx, n);
+        // within row tiles, then the rows left, one wave each
+        Scratch<uint32_t> hq(ctx, n);
         unsigned int *const hq_len = (unsigned int *)(slot_p + 0);  // zeroed with the counters
         k_hook_tile<<<blocks_for(req.n_tiles, 4), 256, 0, s>>>(a, req.n_tiles, hq.p, hq_len);
         CNN_HIP(hipGetLastError());
@@ -1436,86 +1661,71 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
     }
     CNN_HIP(hipGetLastError());
     CNN_HIP(hipEventRecord(ctx->ev[9], s));
-    // flatten (every parent becomes its root), then let roots re-point to smaller
-    // neighbouring roots root_passes times, flattening after each pass; each
-    // flattening before a pass lists the core roots, and only they get a wave
-    if (req.root_passes <= 0) {
-        k_compress<<<blocks_for(n), 256, 0, s>>>(parent.p, n);
-    } else {
+    // lists: root_passes times flatten (every parent becomes its root) listing
+    // the core roots, and let those re-point to smaller neighbouring roots.  On
+    // tile-pair words the full round joins components for less (no pass against
+    // two: 446 against 518 us a fit at n = 3e4, d = 3; 2.11 against 2.17 ms at
+    // n = 1e6); on lists its tests run one row a wave and two passes save 8 to
+    // 15 % of the label pass.
+    if (req.root_passes > 0 && !(words && a.mask)) {
         Scratch<int32_t> roots(ctx, n);
-        unsigned int *const n_roots = (unsigned int *)(slot_p + 2);  // zeroed with the counters
         const unsigned rblocks = (unsigned)std::min<int64_t>(blocks_for(n, 4), 4096);
         for (int pass = 0; pass < req.root_passes; ++pass) {
-            if (pass > 0) fill_u64(ctx, slot_p + 2, 0ull, 1);
-            k_compress_roots<<<blocks_for(n), 256, 0, s>>>(parent.p, core.p, n, roots.p, n_roots);
+            unsigned int *const n_roots = (unsigned int *)(slot_p + 2 + pass);  // zeroed with the counters
+            k_compress_roots<<<blocks_for(n, 1024), 1024, 0, s>>>(parent.p, core.p, n, roots.p, n_roots);
             if (words) k_hook_roots_list<true><<<rblocks, 256, 0, s>>>(a, roots.p, n_roots, 4);
             else k_hook_roots_list<false><<<rblocks, 256, 0, s>>>(a, roots.p, n_roots, 4);
         }
-        k_compress<<<blocks_for(n), 256, 0, s>>>(parent.p, n);
     }
     CNN_HIP(hipGetLastError());
-    {
-        Scratch<int32_t> cnt(ctx, n);
-        fill_i32(ctx, cnt.p, 0, n);
-        k_root_count<<<blocks_for(n, 256 * kRunSteps), 256, 0, s>>>(core.p, parent.p, n, cnt.p);
-        k_count_roots<<<blocks_for(n), 256, 0, s>>>(cnt.p, n, counters_p + 6);
-        k_snapshot<<<blocks_for(n), 256, 0, s>>>(core.p, parent.p, cnt.p, n, rank.p);
-        CNN_HIP(hipGetLastError());
-    }
+    const int steps = run_steps(n);
     std::unique_ptr<Scratch<uint64_t>> cand_max, tile_common;
+    k_root_count<<<blocks_for(n, 256 * steps), 256, 0, s>>>(a, cnt->p, steps);
     if (req.n_tiles > 0) {
         Scratch<uint64_t> tmax(ctx, req.n_tiles);
         cand_max.reset(new Scratch<uint64_t>(ctx, req.n_tiles));
         tile_common.reset(new Scratch<uint64_t>(ctx, req.n_tiles));
-        k_tile_rank_max<<<blocks_for(req.n_tiles, 4), 256, 0, s>>>(rank.p, n, req.n_tiles, tmax.p,
-                                                                   tile_common->p);
+        k_snapshot<<<blocks_for(n), 256, 0, s>>>(core.p, parent.p, cnt->p, n, rank.p, req.n_tiles, tmax.p,
+                                                 tile_common->p);
         k_cand_max<<<blocks_for(req.n_tiles, 1), 256, 0, s>>>(tmax.p, req.tp_ptr, req.tp_col, req.n_tiles,
                                                               cand_max->p);
         CNN_HIP(hipGetLastError());
         a.cand_max = cand_max->p;
         a.tile_rank = tile_common->p;
+    } else {
+        k_snapshot<<<blocks_for(n), 256, 0, s>>>(core.p, parent.p, cnt->p, n, rank.p, 0, nullptr, nullptr);
+        CNN_HIP(hipGetLastError());
+        cnt.reset();
     }
     CNN_HIP(hipEventRecord(ctx->ev[10], s));
     if (words && a.mask && req.n_tiles > 0) {
-        // rows with tests to run go to a queue of at most kRoundQueueMax
-        // entries (beyond it the tile kernel tests them itself)
-        constexpr int64_t kRoundQueueMax = int64_t(1) << 22;
         const int split = round_split(req.n_tile_pairs, req.n_tiles);
-        const int64_t cap = std::min<int64_t>(std::max<int64_t>(n, 64), kRoundQueueMax);
-        Scratch<int4> rq(ctx, cap);
+        Scratch<int2> rq(ctx, round_queue_cap(req.n_tile_pairs, 1));
         a.rq = rq.p;
         a.rq_len = slot_p + 1;  // zeroed with the counters
-        a.rq_cap = cap;
+        a.rq_cap = round_queue_cap(req.n_tile_pairs, 1);
         k_round_tile<<<blocks_for(req.n_tiles * split, 4), 256, 0, s>>>(a, req.n_tiles, split);
-        k_round_queue<<<(unsigned)std::min<int64_t>(blocks_for(n, 4), 4096), 256, 0, s>>>(a);
+        k_round_queue<<<(unsigned)std::min<int64_t>(blocks_for(a.rq_cap, 4), 2048), 256, 0, s>>>(a);
         a.rq = nullptr;
-        a.rq_len = nullptr;
-        a.rq_cap = 0;
     } else if (words) k_round_b<true><<<blocks_for(n, 4), 256, 0, s>>>(a);
     else k_round_b<false><<<blocks_for(n, 4), 256, 0, s>>>(a);
     CNN_HIP(hipEventRecord(ctx->ev[11], s));
     CNN_HIP(hipGetLastError());
-    k_compress<<<blocks_for(n), 256, 0, s>>>(parent.p, n);
     CNN_HIP(hipEventRecord(ctx->ev[1], s));
 
-    Scratch<int32_t> cmin(ctx, n), csize(ctx, n);
-    fill_i32(ctx, cmin.p, INT_MAX, n);
-    fill_i32(ctx, csize.p, 0, n);
-    k_comp_stats<<<blocks_for(n, 256 * kRunSteps), 256, 0, s>>>(core.p, parent.p, req.perm, n, cmin.p, csize.p,
-                                                                counters_p + 2);
+    k_comp_stats<<<blocks_for(n, 256 * steps), 256, 0, s>>>(core.p, parent.p, req.perm, n, cmin.p, csize.p,
+                                                            counters_p + 2, steps);
     CNN_HIP(hipGetLastError());
     // the cluster keys outlive the sort block: a fit with more clusters than
     // k_rank_clusters_small takes sorts them again after the final read
     std::unique_ptr<Scratch<uint64_t>> skeys;
-    std::unique_ptr<Scratch<int32_t>> svals, snewlab;
+    std::unique_ptr<Scratch<int32_t>> svals;
     bool big_sort = false;
     if (req.sort) {
         skeys.reset(new Scratch<uint64_t>(ctx, n));
         svals.reset(new Scratch<int32_t>(ctx, n));
-        snewlab.reset(new Scratch<int32_t>(ctx, n));
         Scratch<uint64_t> &keys = *skeys;
         Scratch<int32_t> &vals = *svals, &newlab = *snewlab;
-        fill_i32(ctx, newlab.p, 0, n);
         if (req.packed) {
             // (only the packed keys: their top bits are the dataset, which
             // k_first_of_set and k_rank_clusters_packed use as an index)
@@ -1565,11 +1775,10 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
     unsigned long long ht[4 * kStatSlots];
     {
         PinnedReads rd(ctx);
-        const unsigned long long *hp = rd.get(counters_p, 8);
-        const unsigned long long *htp = rd.get(tstats_p, 4 * kStatSlots);
+        const unsigned long long *hp = rd.get(counters_p, 8 + 4 * kStatSlots);
         rd.wait();
         std::copy(hp, hp + 8, h);
-        std::copy(htp, htp + 4 * kStatSlots, ht);
+        std::copy(hp + 8, hp + 8 + 4 * kStatSlots, ht);
     }
     if (big_sort) {
         const int64_t K = (int64_t)h[5];
@@ -1585,13 +1794,14 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
         local.n_clusters = (req.max_clusters >= 0) ? std::min<int64_t>(K, req.max_clusters) : K;
     }
     h[0] = h[1] = 0;
-    unsigned long long rows = 0;
+    unsigned long long rows = 0, sampled = 0;
     for (int i = 0; i < kStatSlots; ++i) {
         h[0] += ht[4 * i];
         h[1] += ht[4 * i + 1];
         rows += ht[4 * i + 2];
+        sampled += ht[4 * i + 3];
     }
-    local.sampled_components = (int64_t)h[6];
+    local.sampled_components = (int64_t)sampled;
     local.rows_scanned = (int64_t)rows;
     float t1 = 0, t2 = 0;
     CNN_HIP(hipEventElapsedTime(&t1, ctx->ev[0], ctx->ev[1]));
@@ -1686,26 +1896,24 @@ __global__ __launch_bounds__(256) void k_rank_count(const uint64_t *ckey, const 
     if ((threadIdx.x & 63) == 0 && b) atomicAdd(&counters[8 * y + 7], (unsigned long long)__popcll(b));
 }
 
-void multi_labels_bytes(int64_t n, int64_t n_tiles, int n_c, MultiLabelSizes &sz) {
+void multi_labels_bytes(int64_t n, int64_t n_tiles, int64_t n_tile_pairs, int n_c, MultiLabelSizes &sz) {
     sz.per_point = n * n_c;
     sz.per_tile = std::max<int64_t>(n_tiles, 1) * n_c;
+    sz.round_queue = round_queue_cap(n_tile_pairs, n_c) * n_c;
 }
 
-void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabelSource &src, int root_passes,
-                          int64_t member_cutoff, int64_t max_clusters, int64_t *labels, unsigned long long *counters,
+void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabelSource &src, int64_t member_cutoff,
+                          int64_t max_clusters, int64_t *labels, unsigned long long *counters,
                           unsigned long long *tstats) {
     hipStream_t s = ctx->stream;
     const int64_t n = b.n, T = b.n_tiles;
     const unsigned nc = (unsigned)b.n_c;
     if (n == 0 || nc == 0) return;
     fill_u64(ctx, counters, 0, 8 * (int64_t)nc);
+    fill_u64(ctx, b.rq_len, 0, nc);
     fill_u64(ctx, tstats, 0, 4 * (int64_t)kStatSlots * nc);
-    fill_i32(ctx, (int32_t *)b.hq_len, 0, nc);
-    fill_i32(ctx, (int32_t *)b.ccount, 0, nc);
-    fill_i32(ctx, b.cnt, 0, n * nc);
-    fill_i32(ctx, b.cmin, INT_MAX, n * nc);
-    fill_i32(ctx, b.csize, 0, n * nc);
-    fill_i32(ctx, b.newlab, 0, n * nc);
+    fill_i32(ctx, (int32_t *)b.lens, 0, 2 * (int64_t)nc);
+    unsigned int *const hq_len = b.lens, *const ccount = b.lens + nc;
     LabelArgs a{};
     a.n = n;
     a.core = b.core;
@@ -1721,29 +1929,29 @@ void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabe
     a.mcore_y = b.mcore;
     a.tiles = T;
     auto g2 = [&](int64_t items, int per) { return dim3(blocks_for(items, per), nc); };
-    k_init<<<g2(n, 256), 256, 0, s>>>(a, nullptr, src.perm);
-    k_hook_tile<<<g2(T, 4), 256, 0, s>>>(a, T, b.hq, b.hq_len);
-    k_hook_queue<<<dim3((unsigned)std::min<int64_t>(blocks_for(n, 4), 4096), nc), 256, 0, s>>>(a, b.hq, b.hq_len,
-                                                                                                   2);
-    k_compress<<<g2(n, 256), 256, 0, s>>>(b.parent, n);
-    for (int pass = 0; pass < root_passes; ++pass) {
-        k_hook_roots<true><<<g2(n, 4), 256, 0, s>>>(a, 4);
-        k_compress<<<g2(n, 256), 256, 0, s>>>(b.parent, n);
-    }
+    const unsigned waves = (unsigned)std::min<int64_t>(blocks_for(n, 4), 4096);
+    k_init<<<g2(n, 256), 256, 0, s>>>(a, nullptr, src.perm, ComponentArrays{b.cnt, b.cmin, b.csize, b.newlab});
+    k_hook_tile<<<g2(T, 4), 256, 0, s>>>(a, T, b.hq, hq_len);
+    k_hook_queue<<<dim3(waves, nc), 256, 0, s>>>(a, b.hq, hq_len, 2);
     CNN_HIP(hipGetLastError());
-    k_root_count<<<g2(n, 256 * kRunSteps), 256, 0, s>>>(b.core, b.parent, n, b.cnt);
-    k_snapshot<<<g2(n, 256), 256, 0, s>>>(b.core, b.parent, b.cnt, n, b.rank);
-    k_tile_rank_max<<<g2(T, 4), 256, 0, s>>>(b.rank, n, T, b.tmax, b.tile_common);
+    const int steps = run_steps(n * nc);
+    k_root_count<<<g2(n, 256 * steps), 256, 0, s>>>(a, b.cnt, steps);
+    k_snapshot<<<g2(n, 256), 256, 0, s>>>(b.core, b.parent, b.cnt, n, b.rank, T, b.tmax, b.tile_common);
     k_cand_max<<<g2(T, 1), 256, 0, s>>>(b.tmax, src.tp_ptr, src.tp_col, T, b.cand_max);
     CNN_HIP(hipGetLastError());
     a.cand_max = b.cand_max;
     a.tile_rank = b.tile_common;
-    k_round_b<true><<<g2(n, 4), 256, 0, s>>>(a);
-    k_compress<<<g2(n, 256), 256, 0, s>>>(b.parent, n);
-    k_comp_stats<<<g2(n, 256 * kRunSteps), 256, 0, s>>>(b.core, b.parent, src.perm, n, b.cmin, b.csize, counters);
+    const int split = round_split(src.n_tile_pairs, T * nc);
+    a.rq = b.rq;
+    a.rq_len = b.rq_len;
+    a.rq_cap = round_queue_cap(src.n_tile_pairs, b.n_c);
+    k_round_tile<<<g2(T * split, 4), 256, 0, s>>>(a, T, split);
+    k_round_queue<<<dim3((unsigned)std::min<int64_t>(blocks_for(a.rq_cap, 4), 2048), nc), 256, 0, s>>>(a);
+    k_comp_stats<<<g2(n, 256 * steps), 256, 0, s>>>(b.core, b.parent, src.perm, n, b.cmin, b.csize, counters + 2,
+                                                    steps);
     k_collect_multi<<<g2(n, 256), 256, 0, s>>>(b.core, b.parent, b.cmin, b.csize, n, member_cutoff, b.ckey,
-                                               b.cidx, b.ccount);
-    k_rank_count<<<g2(n, 256), 256, 0, s>>>(b.ckey, b.cidx, b.ccount, n, max_clusters, b.newlab, counters);
+                                               b.cidx, ccount);
+    k_rank_count<<<g2(n, 256), 256, 0, s>>>(b.ckey, b.cidx, ccount, n, max_clusters, b.newlab, counters);
     k_write_sorted<<<g2(n, 256), 256, 0, s>>>(b.core, b.parent, b.newlab, src.perm, n, labels);
     CNN_HIP(hipGetLastError());
 }

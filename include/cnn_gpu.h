@@ -348,7 +348,7 @@ typedef struct {
     int32_t mfma_col_chunk;  /* column tiles per workgroup of the dense MFMA distance kernel (8..1024; 64) */
     int32_t wide_col_chunk;  /* column tiles per workgroup of the dense plain-FP64 kernel (1..1024; 32) */
     int32_t emit_waves;      /* waves per workgroup of the neighbour-list emission (4 or 8; 8) */
-    int32_t root_passes;     /* root-hooking passes of the labelling before its full round (0..8; 2) */
+    int32_t root_passes;     /* root-hooking passes before the full round of a labelling on lists (0..8; 2) */
     int32_t words_min_fill;  /* CNN_SIM_AUTO on lists: per-row word lists when the lists hold at least
                                 this many entries per word (estimated on every 16th row), else the
                                 merge; 0 or more than 2^24: always the merge (0..2^30; 8) */

@@ -1,0 +1,59 @@
+"""The label pass on tile-pair words at the places where its kernels can go
+wrong: tests that fail over many columns (batches of several columns a row, the
+queue of tile pairs), tiles with more common candidate tiles than one chunk of
+the match holds, ragged tiles, a cutoff of zero, mixed components per tile.
+Labels are whole numbers: equal to the oracle's."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle as C
+from commonnnclustering_amd import engine
+
+pytestmark = pytest.mark.gpu
+
+
+def _blobs(n, d, sep, seed):
+    rng = np.random.default_rng(seed)
+    x = rng.normal(size=(n, d))
+    x[: n // 2, 0] += sep
+    x[-n // 20:] = rng.uniform(-4.0, 4.0 + sep, size=(len(x[-n // 20:]), d))
+    return x[rng.permutation(n)]
+
+
+# (n, d, separation, radius, cutoffs): the degrees run from a few to thousands,
+# the cutoffs from passing everywhere to failing for most edges
+CASES = [
+    (65, 2, 3.0, 1.0, (0, 3, 20)),
+    (129, 3, 3.0, 0.8, (0, 2, 8)),
+    (5003, 3, 2.0, 0.3, (2, 6, 12, 25)),
+    (20011, 2, 3.0, 1.2, (50, 900, 1800, 2600)),
+    (4111, 16, 6.0, 4.6, (5, 60, 200)),
+]
+
+
+@pytest.mark.parametrize("n,d,sep,r,cuts", CASES)
+def test_round_matches_oracle(cuda, n, d, sep, r, cuts):
+    x = _blobs(n, d, sep, n)
+    X = torch.from_numpy(x).cuda()
+    for c in cuts:
+        want = C.fit(x, r, c, member_cutoff=2)
+        lab, _, _, ls = engine.fit(X, r * r, c + 2, c + 1, precision="f64", member_cutoff=2)
+        assert (lab.cpu().numpy() == want).all(), f"c={c}"
+        if c == 0:  # c_sim = 0: every edge between core points passes
+            lab = engine.fit(X, r * r, 0, 1, precision="f64", member_cutoff=1)[0].cpu().numpy()
+            full = C.fit(x, r, 0, member_cutoff=1)
+            assert ((lab > 0) >= (full > 0)).all()
+
+
+@pytest.mark.parametrize("n,d,sep,r,cuts", [c for c in CASES if c[1] <= 3 and c[0] > 128])
+def test_scan_rounds_match_oracle(cuda, n, d, sep, r, cuts):
+    """Every cutoff of a radius in one launch, twice over the same graph."""
+    x = _blobs(n, d, sep, n)
+    radii = [r, 0.7 * r]
+    lab, _, _ = engine.fit_scan(torch.from_numpy(x).cuda(), radii, list(cuts), precision="f64", member_cutoff=2)
+    lab = lab.cpu().numpy()
+    for ri, rad in enumerate(radii):
+        for ci, c in enumerate(cuts):
+            assert (lab[ri, ci] == C.fit(x, rad, c, member_cutoff=2)).all(), (rad, c)
