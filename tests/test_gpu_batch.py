@@ -123,11 +123,10 @@ def test_batch_many_sets_concurrent(cuda, d):
         assert ls["n_clusters"] == sum(int(w.max(initial=0)) for w in want)
 
 
-@pytest.mark.parametrize("scale,form", [(1.5, "tile words"), (0.05, "lists")])
-def test_packed_batch_similarity_forms(cuda, scale, form):
-    """The label pass of a packed batch runs on the tile-pair words when they are
-    the smaller form (dense neighbourhoods) and on lists otherwise; tile edges,
-    empty and one-point datasets among the sets."""
+@pytest.mark.parametrize("scale", [1.5, 0.3, 0.05])
+def test_packed_batch_tile_words(cuda, scale):
+    """The label pass of a packed batch runs on the tile-pair words, dense or
+    sparse; tile edges, empty and one-point datasets among the sets."""
     rng = np.random.default_rng(11)
     sets = []
     for n in [0, 1, 63, 64, 65, 127, 129, 700, 1500]:
@@ -137,4 +136,4 @@ def test_packed_batch_similarity_forms(cuda, scale, form):
     got, _, ls = _run_batch(sets, "f32_band", member_cutoff=2)
     for b, (g, w) in enumerate(zip(got, want)):
         assert (g == w).all(), f"dataset {b} (n={len(w)})"
-    assert (ls["sim_form"] == 2) == (form == "tile words")
+    assert ls["sim_form"] == 2  # CNN_SIM_FORM_TILE_WORDS
