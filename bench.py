@@ -45,13 +45,13 @@ sys.path.insert(0, ROOT)
 METRIC = "fit points/s (plain FP64 vs FP32-banded) bit-exact labels; served p50/p99 ms"
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3     # vector and dense MFMA FP32
+FP16_PEAK_TFLOPS = 2500.0    # dense MFMA
 FP64_PEAK_TFLOPS = 78.6      # FMA-counted; separately rounded sub/mul/add reach half of it
 
 # HBM traffic per launch, from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs
 # scaled by a copy kernel of known size (profiles/*_traffic.json).
 TRAFFIC_FILES = {
     ("k_dist_f32_cols", "md_basins_3d"): "profiles/k_dist_f32_cols_md_basins_3d_traffic.json",
-    ("k_dist_mfma_lds", "features_64d"): "profiles/k_dist_mfma_lds_features_64d_traffic.json",
     ("round", "md_basins_3d"): "profiles/round_md_basins_3d_traffic.json",
     ("hook", "md_basins_3d"): "profiles/hook_md_basins_3d_traffic.json",
     ("round", "features_64d"): "profiles/round_features_64d_traffic.json",
@@ -137,10 +137,12 @@ def distance_roofline(gs, d, precision, workload_name):
     flops = (2.0 if gram else 3.0) * d * pairs
     if precision == "f32_band":
         if gram:
-            kernel = "k_dist_mfma_lds" if (d + 2 + 7) // 8 <= 10 else "k_dist_mfma"
+            kernel = "k_dist_split" if d <= 128 else "k_dist_mfma"
         else:
             kernel = "k_dist_f32_cols" if d <= 8 else "k_dist_f32_generic"
         bound, peak = ("mfma" if gram else "valu"), FP32_PEAK_TFLOPS
+        if kernel == "k_dist_split":  # three FP16 products per FP32 product
+            peak = FP16_PEAK_TFLOPS / 3
     else:
         kernel = "k_dist_f64_cols" if d <= 8 else "k_dist_f64_wide"
         bound, peak = "valu", FP64_PEAK_TFLOPS

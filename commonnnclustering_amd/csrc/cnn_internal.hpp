@@ -443,6 +443,13 @@ __device__ __forceinline__ long long wave_sum64(long long v) {
     return v;
 }
 
+// The wave's LDS writes before, its reads after (one wave's LDS accesses run
+// in order; this keeps the compiler from reordering them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 template <typename T>
 __device__ __forceinline__ T uniform(T v) {
     return __builtin_amdgcn_readfirstlane(v);

@@ -764,13 +764,6 @@ struct TileMatch {
     }
 };
 
-// The wave's LDS writes before, its reads after (one wave's LDS accesses run
-// in order; this keeps the compiler from reordering them).
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // One row tile of the full round, as its wave holds it (lane r = row 64R + r).
 struct RoundRows {
     int64_t R;

@@ -805,7 +805,14 @@ struct DistArgs {
     const uint64_t *live;
     const int32_t *live_pre;
     int64_t live_words;
-    int deal_rr;  // dense MFMA kernel: work items dealt round-robin over the XCDs
+    // split FP16 Gram form (d <= kSplitMaxD, nullptr otherwise): operands, the
+    // points' scaled terms, the tiles' margins and scales (k_split_tiles); both
+    // Gram forms: the points' unscaled terms r2/4 - |x|^2/2
+    const uint4 *sx;
+    const float *sc;
+    const float *se;
+    const float *ss;
+    const float *caug;
     // spatial layout, one batch: the row tile of workgroup b is row_order[b]
     // (heavy tiles first), nullptr: R0 + b
     const int32_t *row_order;
@@ -1513,50 +1520,31 @@ __device__ __forceinline__ uint64_t pack_halves(uint32_t a_lo, uint32_t a_hi, ui
     return (uint64_t)(a_lo | (a_hi << 4)) | ((uint64_t)(b_lo | (b_hi << 4)) << 32);
 }
 
-// Guard-band elements of the listed tile pairs, settled one per thread.  The
-// records (k, R, 64 per-lane flag words) are flattened into a list of
-// elements (record << 12 | lane << 6 | bit): k_band_count counts each
-// record's elements, an exclusive scan places them, k_band_list writes them,
-// and k_band_settle decides each in FP64 in reference order and ors its bit
-// into the stored words of the pair and of its mirror (and counts it in both
-// degrees).  The FP32 statistics recompute the Gram value from the augmented
-// vectors (sequential FMAs; statistics only).
-__global__ __launch_bounds__(256) void k_band_count(const int64_t *__restrict__ band_list, int64_t n_rec,
-                                                    int32_t *__restrict__ cnt) {
-    const int lane = threadIdx.x & 63;
-    const int64_t rec = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (rec >= n_rec) return;
-    if (band_list[rec * 66] < 0) {  // a reserved slot left empty
-        if (lane == 0) cnt[rec] = 0;
-        return;
-    }
-    const int c = wave_sum(__popcll((uint64_t)band_list[rec * 66 + 2 + lane]));
-    if (lane == 0) cnt[rec] = c;
-}
-
-__global__ __launch_bounds__(256) void k_band_list(const int64_t *__restrict__ band_list, int64_t n_rec,
-                                                   const int64_t *__restrict__ off, int64_t *__restrict__ elem) {
-    const int lane = threadIdx.x & 63;
-    const int64_t rec = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (rec >= n_rec || band_list[rec * 66] < 0) return;
-    uint64_t f = (uint64_t)band_list[rec * 66 + 2 + lane];
-    const int c = __popcll(f);
-    int64_t o = off[rec] + wave_incl_scan(c) - c;
-    while (f) {
-        const int b = __ffsll((unsigned long long)f) - 1;
-        f &= f - 1;
-        elem[o++] = (rec << 12) | ((int64_t)lane << 6) | b;
-    }
-}
+// Guard-band elements of the listed tile pairs, settled one per thread
+// (k_band_settle): a workgroup takes 64 records (k, R, 64 per-lane flag words)
+// at a time -- a wave loads its 16 records' flag words together and keeps them
+// in registers -- flattens their elements into an LDS list (record, lane, bit)
+// and decides each in FP64 in reference order, or-ing its bit into the stored
+// words of the pair and of its mirror and counting it in both degrees.  The
+// number of records is read on the device.  The FP32 statistics add the FP32
+// products along the way (statistics only).
+// Bound by the latency of the record and row reads: with the records read one
+// after another, 68 KB of LDS and whole-row loads it took 508 us for 443,000
+// elements of 64 dimensions, as here 218 us.
+constexpr int kBandGroup = 64;     // records a workgroup flattens at a time
+constexpr int kBandElems = 4096;   // elements of its list; one record has at most as many
 
 // exact_d2 with the row reads grouped: eight dimensions of both rows loaded
 // together as 16-byte pairs (rows start 16-byte aligned when d is even), so a
 // thread's accesses to a row's cache lines come close together; the sum is
-// the same sequence of separately rounded steps in ascending k.
-__device__ __forceinline__ double exact_d2_grouped(const double *__restrict__ xw64, int d, int64_t i, int64_t j) {
+// the same sequence of separately rounded steps in ascending k.  prod: the FP32
+// products' sum.
+__device__ __forceinline__ double exact_d2_grouped(const double *__restrict__ xw64, int d, int64_t i, int64_t j,
+                                                   float &prod) {
     const double *a = xw64 + i * d;
     const double *b = xw64 + j * d;
     double s = 0.0;
+    float p = 0.0f;
     int k = 0;
     if ((d & 1) == 0) {
         for (; k + 8 <= d; k += 8) {
@@ -1569,67 +1557,116 @@ __device__ __forceinline__ double exact_d2_grouped(const double *__restrict__ xw
             for (int q = 0; q < 8; ++q) {
                 const double t = av[q] - bv[q];
                 s = s + t * t;
+                p = __builtin_fmaf((float)av[q], (float)bv[q], p);
             }
         }
     }
     for (; k < d; ++k) {
         const double t = a[k] - b[k];
         s = s + t * t;
+        p = __builtin_fmaf((float)a[k], (float)b[k], p);
     }
+    prod = p;
     return s;
 }
 
-// FP32 Gram value of points gi, gj from the packed augmented vectors (four
-// dimensions per float4; statistics only).
+// FP32 Gram value of points gi, gj from the plain FP32 rows (statistics only).
 __device__ __forceinline__ float gram_value(const DistArgs &a, int64_t gi, int64_t gj) {
-    const int G = a.dp >> 3;
-    const float4 *pa = (const float4 *)a.xra + (gi >> 6) * G * 128 + (gi & 63);
-    const float4 *pb = (const float4 *)a.xca + (gj >> 6) * G * 128 + (gj & 63);
+    const float *x = a.xw32 + gi * a.d, *y = a.xw32 + gj * a.d;
     float prod = 0.0f;
-    for (int g = 0; g < G; ++g) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const float4 x = pa[(g * 2 + h) * 64], y = pb[(g * 2 + h) * 64];
-            prod = __builtin_fmaf(x.x, y.x, prod);
-            prod = __builtin_fmaf(x.y, y.y, prod);
-            prod = __builtin_fmaf(x.z, y.z, prod);
-            prod = __builtin_fmaf(x.w, y.w, prod);
-        }
-    }
-    return prod;
+    for (int k = 0; k < a.d; ++k) prod = __builtin_fmaf(x[k], y[k], prod);
+    return prod + a.caug[gi] + a.caug[gj];
 }
 
-__global__ __launch_bounds__(256) void k_band_settle(DistArgs a, const int64_t *__restrict__ elem, int64_t n_el) {
+__global__ __launch_bounds__(256) void k_band_settle(DistArgs a) {
+    __shared__ uint32_t s_elem[kBandElems];
+    __shared__ int s_cnt[kBandGroup];
+    __shared__ int64_t s_k[kBandGroup];
+    __shared__ int2 s_rc[kBandGroup];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t n_rec = min((int64_t)*a.band_cnt, a.band_cap);
     unsigned hits = 0, flips = 0;
     double maxerr = 0.0;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n_el; t += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t v = elem[t];
-        const int64_t rec = v >> 12;
-        const int le = (int)((v >> 6) & 63), e = (int)(v & 63);
-        const int64_t k = a.band_list[rec * 66], R = a.band_list[rec * 66 + 1];
-        int64_t kb, ke;
-        tile_range(a, R, kb, ke);
-        const int64_t C = tile_col(a, k, kb);
-        int row, col;
-        band_element(le, e, row, col);
-        const int64_t gi = R * 64 + row, gj = C * 64 + col;
-        const double ex = exact_d2_grouped(a.xw64, a.d, gi, gj);
-        const bool in = ex <= a.bp.r2;
-        const double d2 = a.bp.r2 - 2.0 * (double)gram_value(a, gi, gj);
-        ++hits;
-        flips += in != (d2 <= a.bp.r2);
-        const double err = fabs(d2 - ex);
-        if (err == err) maxerr = fmax(maxerr, err);
-        if (in) {
-            atomicOr(&a.mask[(k - a.k_base) * 64 + row], 1ull << col);
-            atomicAdd(&a.deg[gi], 1);
-            if (a.pair_nz) a.pair_nz[k - a.k_base] = 1;
-            if (a.sym && C != R) {
-                const int64_t km = mirror_of(a, k, R, C);
-                atomicOr(&a.mask[(km - a.k_base) * 64 + col], 1ull << row);
-                atomicAdd(&a.deg[gj], 1);
-                if (a.pair_nz) a.pair_nz[km - a.k_base] = 1;
+    for (int64_t base = (int64_t)blockIdx.x * kBandGroup; base < n_rec; base += (int64_t)gridDim.x * kBandGroup) {
+        // a wave's 16 records: all flag words in flight together, kept in registers
+        constexpr int kRec = kBandGroup / 4;
+        uint64_t f[kRec];
+        int64_t k_rec = -1;
+        if (lane < kRec && base + wave * kRec + lane < n_rec) k_rec = a.band_list[(base + wave * kRec + lane) * 66];
+#pragma unroll
+        for (int q = 0; q < kRec; ++q) {
+            const int64_t r = base + wave * kRec + q;
+            f[q] = r < n_rec ? (uint64_t)a.band_list[r * 66 + 2 + lane] : 0ull;
+        }
+        if (lane < kRec) {
+            int64_t R = 0, C = 0;
+            if (k_rec >= 0) {  // (else a reserved slot left empty)
+                R = a.band_list[(base + wave * kRec + lane) * 66 + 1];
+                int64_t kb, ke;
+                tile_range(a, R, kb, ke);
+                C = tile_col(a, k_rec, kb);
             }
+            s_k[wave * kRec + lane] = k_rec;
+            s_rc[wave * kRec + lane] = make_int2((int)R, (int)C);
+        }
+        const uint64_t used = __ballot(k_rec >= 0);
+        int incl[kRec];
+#pragma unroll
+        for (int q = 0; q < kRec; ++q) {
+            if (!((used >> q) & 1ull)) f[q] = 0ull;
+            incl[q] = wave_incl_scan(__popcll(f[q]));
+            if (lane == 63) s_cnt[wave * kRec + q] = incl[q];
+        }
+        __syncthreads();
+        // the records [r0, r1) whose elements fit the list, until all are done
+        for (int r0 = 0; r0 < kBandGroup;) {
+            int r1 = r0, total = 0, before = 0;  // before: elements of earlier waves' records
+            while (r1 < kBandGroup && total + s_cnt[r1] <= kBandElems) {
+                if (r1 < wave * kRec) before += s_cnt[r1];
+                total += s_cnt[r1++];
+            }
+#pragma unroll
+            for (int q = 0; q < kRec; ++q) {
+                const int r = wave * kRec + q;
+                if (r < r0 || r >= r1) continue;
+                uint64_t x = f[q];
+                int o = before + incl[q] - __popcll(x);
+                while (x) {
+                    const int b = __ffsll((unsigned long long)x) - 1;
+                    x &= x - 1;
+                    s_elem[o++] = ((uint32_t)r << 12) | ((uint32_t)lane << 6) | (uint32_t)b;
+                }
+                before += s_cnt[r];
+            }
+            __syncthreads();
+            for (int t = threadIdx.x; t < total; t += 256) {
+                const uint32_t v = s_elem[t];
+                const int64_t k = s_k[v >> 12], R = s_rc[v >> 12].x, C = s_rc[v >> 12].y;
+                int row, col;
+                band_element((int)((v >> 6) & 63), (int)(v & 63), row, col);
+                const int64_t gi = R * 64 + row, gj = C * 64 + col;
+                float prod;
+                const double ex = exact_d2_grouped(a.xw64, a.d, gi, gj, prod);
+                const bool in = ex <= a.bp.r2;
+                const double d2 = a.bp.r2 - 2.0 * (double)(prod + a.caug[gi] + a.caug[gj]);
+                ++hits;
+                flips += in != (d2 <= a.bp.r2);
+                const double err = fabs(d2 - ex);
+                if (err == err) maxerr = fmax(maxerr, err);
+                if (in) {
+                    atomicOr(&a.mask[(k - a.k_base) * 64 + row], 1ull << col);
+                    atomicAdd(&a.deg[gi], 1);
+                    if (a.pair_nz) a.pair_nz[k - a.k_base] = 1;
+                    if (a.sym && C != R) {
+                        const int64_t km = mirror_of(a, k, R, C);
+                        atomicOr(&a.mask[(km - a.k_base) * 64 + col], 1ull << row);
+                        atomicAdd(&a.deg[gj], 1);
+                        if (a.pair_nz) a.pair_nz[km - a.k_base] = 1;
+                    }
+                }
+            }
+            __syncthreads();
+            r0 = r1;
         }
     }
     flush_band(a, hits, flips, maxerr);
@@ -1663,6 +1700,31 @@ __device__ __forceinline__ void band_slots_release(const DistArgs &a, BandSlots 
     if ((threadIdx.x & 63) == 0)
         for (unsigned long long q = bs.next; q < bs.end && (int64_t)q < a.band_cap; ++q) a.band_list[q * 66] = -1;
     bs.next = bs.end;
+}
+
+// Queues the guard-band elements of pair k of row tile R (the lane's flags).
+__device__ __forceinline__ void queue_band(const DistArgs &a, int64_t k, int64_t R, uint64_t flags, BandSlots &bs) {
+    const int lane = threadIdx.x & 63;
+    if (bs.next == bs.end) {
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(a.band_cnt, (unsigned long long)kBandSlotChunk);
+        base = __shfl(base, 0, 64);
+        bs.next = base;
+        bs.end = base + kBandSlotChunk;
+    }
+    const unsigned long long slot = bs.next++;
+    if ((int64_t)slot < a.band_cap) {
+        int64_t *p = a.band_list + (int64_t)slot * 66;
+        if (lane == 0) {
+            p[0] = k;
+            p[1] = R;
+        }
+        p[2 + lane] = (int64_t)flags;
+    } else if (lane == 0) {
+        const unsigned long long rs = atomicAdd(a.redo_cnt, 1ull);
+        a.redo[2 * rs] = k;
+        a.redo[2 * rs + 1] = R;
+    }
 }
 
 __device__ __forceinline__ int mfma_settle_store(const DistArgs &a, const MfmaTile &t, int64_t k, int64_t R,
@@ -1713,26 +1775,7 @@ __device__ __forceinline__ int mfma_settle_store(const DistArgs &a, const MfmaTi
         }
         if (__ballot(flags != 0ull)) {
             queued = true;
-            if (bs.next == bs.end) {
-                unsigned long long base = 0;
-                if (lane == 0) base = atomicAdd(a.band_cnt, (unsigned long long)kBandSlotChunk);
-                base = __shfl(base, 0, 64);
-                bs.next = base;
-                bs.end = base + kBandSlotChunk;
-            }
-            const unsigned long long slot = bs.next++;
-            if ((int64_t)slot < a.band_cap) {
-                int64_t *p = a.band_list + (int64_t)slot * 66;
-                if (lane == 0) {
-                    p[0] = k;
-                    p[1] = R;
-                }
-                p[2 + lane] = (int64_t)flags;
-            } else if (lane == 0) {
-                const unsigned long long rs = atomicAdd(a.redo_cnt, 1ull);
-                a.redo[2 * rs] = k;
-                a.redo[2 * rs + 1] = R;
-            }
+            queue_band(a, k, R, flags, bs);
         }
         colword = merge_col_words(a_lo, a_hi, b_lo, b_hi);
         word = transpose_bits(colword);
@@ -1764,182 +1807,539 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     finish_deg(a, i, mydeg);
 }
 
-// Row blocks of the dense LDS MFMA kernel with work in column chunk cc: all of
-// them, or (symmetric evaluation, C >= R only) those starting before the
-// chunk's end.
-__host__ __device__ inline int64_t mfma_chunk_blocks(int sym, int64_t cc, int64_t chunk, int64_t n_tiles,
-                                                     int64_t R0, int64_t n_rb) {
-    if (!sym) return n_rb;
-    const int64_t c_hi = cc * chunk + chunk < n_tiles ? cc * chunk + chunk : n_tiles;
-    const int64_t b = (c_hi - R0 + 3) / 4;
-    return b < 0 ? 0 : (b < n_rb ? b : n_rb);
+// m u / (1 - m u): the relative bound of m rounded operations of unit u.
+static double gamma_m(int m, double u) { return m * u / (1.0 - m * u); }
+
+// ------------------------------------------------------------------ split FP16 Gram form on MFMA (16 <= d <= 128)
+//
+// T = x_i . x_j + c_i + c_j = (r2 - d2)/2 as in the FP32 Gram form, with each
+// FP32 coordinate split into two FP16 parts, s x = h + l (s a power of two per
+// tile), and x.y ~ h.h' + h.l' + l.h' on v_mfma_f32_32x32x16_f16 with FP32
+// accumulators: three products at 16 times the FP32 MFMA's rate.  The small
+// products are summed first, so only the 16 KS products h.h' and the two terms
+// c meet the large partial sums; c enters through one FP32 MFMA step.  The error
+// against FP64 is 0.3 to 0.7 of the FP32 form's over d = 16 .. 128 (figures at
+// split_margin).
+constexpr int kSplitMaxD = 128;
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+// Operand of step s (16 dimensions), part p (0: h, 1: l) and 32-row block b of a
+// tile: 64 lanes x 16 bytes, lane l holding point 32b + l%32, dimensions
+// 16s + 8(l/32) .. + 7 -- one contiguous KiB per wave-wide load; 4 KiB a step.
+template <int KS>
+__device__ __forceinline__ constexpr int split_at(int s, int p, int b) {
+    return ((s * 2 + p) * 2 + b) * 64;
 }
 
-// Dense MFMA form for d + 2 <= 8G.  A workgroup takes 4 consecutive row tiles
-// (one per wave, its operands held in registers for the whole launch) and a
-// chunk of column tiles; each column tile is staged once in LDS (double
-// buffered: the next tile's loads are in flight during the current tile's
-// MFMAs) and read by all 4 waves.  The work items (column chunk, row block)
-// that hold any pair are numbered chunk-major and dealt to the 8 XCDs in
-// contiguous ranges of equal length (workgroup b runs on XCD b % 8), so every
-// XCD gets the same work and workgroups that share an L2 read the same column
-// tiles.  Degrees are added atomically (several chunks contribute to a row).
-constexpr int kMfmaMaxChunk = 1024;  // largest column chunk of the tuning table
-template <int G>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_dist_mfma_lds(
-    DistArgs a, int64_t n_rt, int64_t n_rb, int64_t n_cc, int64_t per_xcd, int64_t n_items) {
-    constexpr int kTileF4 = G * 128;  // float4 per packed tile
-    constexpr int kPer = (kTileF4 + 255) / 256;
-    __shared__ float4 sB[2][kTileF4];
-    __shared__ float sE[2];  // largest margin of the staged column tile
-    __shared__ int32_t sCol[kMfmaMaxChunk];  // live column tiles of the item (culled layout)
-    __shared__ int sNcol;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = lane & 31, h = lane >> 5;
-    // items in contiguous ranges per XCD, or dealt round-robin (deal_rr)
-    const int64_t item = a.deal_rr ? (int64_t)blockIdx.x : (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (item >= n_items) return;
-    int64_t cc = 0, rb = item;
-    for (; cc < n_cc; ++cc) {
-        const int64_t nb = mfma_chunk_blocks(a.sym, cc, a.col_chunk, a.n_tiles, a.R0, n_rb);
-        if (rb < nb) break;
-        rb -= nb;
-    }
-    if (cc >= n_cc) return;  // not reached: item < n_items
-    const int64_t R_lo = a.R0 + 4 * rb;
-    const int64_t R = R_lo + wave;
-    const bool rvalid = R < a.R0 + n_rt;
-    const int64_t c_lo = cc * a.col_chunk;
-    const int64_t c_hi = min(a.n_tiles, c_lo + a.col_chunk);
-    const int64_t c_begin = a.sym ? max(c_lo, R_lo) : c_lo;
-    if (c_begin >= c_hi) return;  // the whole workgroup
-    const int tail = a.mfma_k - 4 * (G - 1);
-    // the column tiles to visit: all of [c_begin, c_hi), or (culled layout)
-    // those with a live pair for any of the 4 row tiles
-    int n_col = (int)(c_hi - c_begin);
-    if (a.live) {
-        if (wave == 0) {
-            const int64_t r_end = a.R0 + n_rt;
-            int cnt = 0;
-            for (int64_t cw = c_begin; cw < c_hi; cw += 64) {
-                const int64_t C = cw + lane;
-                bool any = false;
-                if (C < c_hi) {
-                    for (int q = 0; q < 4; ++q) {
-                        const int64_t Rq = R_lo + q;
-                        if (Rq < r_end && (!a.sym || C >= Rq) && pair_live(a, Rq, C)) any = true;
-                    }
-                }
-                const uint64_t m = __ballot(any);
-                const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                if (any) sCol[cnt + rank] = (int32_t)C;
-                cnt += __popcll(m);
-            }
-            if (lane == 0) sNcol = cnt;
-        }
-        __syncthreads();
-        n_col = sNcol;
-        if (n_col == 0) return;  // the whole workgroup
-    }
-    auto col_at = [&](int idx) -> int64_t { return a.live ? (int64_t)sCol[idx] : c_begin + idx; };
-    const int64_t C0 = col_at(0);
+// Margin of a point in the split form.  |T_hat - T| <= e_i + e_j with, for
+// w = |x|^2, u = 2^-24 and m the tile's largest |coordinate| or r if larger:
+//   accumulation: at most 16 KS + 6 roundings that see the full sum (16 KS
+//     products h.h', the terms c; the small products' own sums are 2^-10 of it
+//     and are covered by the surplus), each at most 2u of Sabs <= (w_i + w_j) +
+//     r2/2 -- 2u also if the unit truncates;
+//   the split: |x - (h + l)/s| <= 2^-22 |x| and the dropped l.l' <= 2^-22 |x||y|,
+//     in all 12u |x||y| <= 6u (w_i + w_j);
+//   FP16 subnormals, flushed or not: 2^-13/s absolute per coordinate and
+//     1/s <= 2^-13 m, so 2^-26 sqrt(d) m |y| on either side, at most
+//     2^-27 sqrt(d) (w + m^2) a point;
+//   rounding c and its scaled form, r2/4: u w + u r2/2 (w is summed in FP64);
+//   f64 input rounded to f32: u w + u r2/2;
+//   the reference's FP64 rounding near the threshold: gamma_{2d+2}(2^-53) r2/2.
+// Measured |d2_hat - d2| on 5e5 pairs of unit Gaussians around shared centres of
+// spread 2, split against FP32 form: d = 16 rms 7.6e-6 / 1.2e-5, largest
+// 7.6e-5 / 1.1e-4; d = 64 3.3e-5 / 8.4e-5, 2.0e-4 / 4.8e-4; d = 128 8.3e-5 /
+// 2.3e-4, 4.1e-4 / 1.4e-3; the same points 30 from the origin: d = 16 1.0e-3 /
+// 2.2e-3, d = 64 5.6e-3 / 1.6e-2, d = 128 1.4e-2 / 4.6e-2 rms.
+struct SplitMargin {
+    double a;   // times w
+    double f;   // times w + m^2
+    double b;   // constant
+};
+static SplitMargin split_margin(int d, int ks, bool rounded_coords, double r2) {
+    const double u = std::ldexp(1.0, -24), u64 = std::ldexp(1.0, -53);
+    const double g = gamma_m(16 * ks + 6, 2.0 * u);
+    SplitMargin m;
+    const double S = 1.0 + 64.0 * u;  // evaluating the margin itself
+    m.a = S * (g + 6.0 * u + u + (rounded_coords ? u : 0.0));
+    m.f = S * std::ldexp(std::sqrt((double)d), -27);
+    m.b = S * (0.25 * g + u + 0.5 * gamma_m(2 * d + 2, u64) + (rounded_coords ? 0.5 * u : 0.0)) * r2 + 1e-30;
+    return m;
+}
 
-    float4 A0[G], A1[G];
-    float e_row = 0.0f;
-    if (rvalid) {
-        const float4 *__restrict__ pa = (const float4 *)a.xra + R * kTileF4 + h * 64 + r;
+// The split operands, terms and margins of one tile per workgroup, its
+// coordinates staged in LDS (rows padded by one: no bank conflicts).  Points
+// that are non-finite or have |x|^2 > 1e36 get zero operands and an infinite
+// tile margin, which sends every element of the tile's pairs to the FP64
+// settling; padding rows get a term that is out of every radius.
+template <int KS>
+__global__ __launch_bounds__(256) void k_split_tiles(const float *__restrict__ xw32, int64_t n, int d, double r2,
+                                                     SplitMargin sm, uint4 *__restrict__ sx, float *__restrict__ sc,
+                                                     float *__restrict__ se, float *__restrict__ ss,
+                                                     float *__restrict__ caug) {
+    constexpr int kD = 16 * KS;
+    __shared__ float sxr[64 * (kD + 1)];
+    __shared__ float s_max[4], s_e[4];
+    __shared__ int s_bad[64];
+    const int64_t R = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int t = tid; t < 64 * kD; t += 256) sxr[(t / kD) * (kD + 1) + t % kD] = 0.0f;
+    __syncthreads();
+    const int rows = (int)min<int64_t>(64, n - R * 64);
+    for (int t = tid; t < rows * d; t += 256) sxr[(t / d) * (kD + 1) + t % d] = xw32[R * 64 * d + t];
+    __syncthreads();
+    // four threads a row
+    const int row = tid >> 2, part = tid & 3;
+    double w = 0.0;
+    float mx = 0.0f;
+    for (int k = part; k < d; k += 4) {
+        const float x = sxr[row * (kD + 1) + k];
+        w += (double)x * (double)x;
+        mx = fmaxf(mx, fabsf(x));
+    }
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            A0[g] = pa[g * 128];
-            A1[g] = pa[g * 128 + 32];
+    for (int o = 1; o <= 2; o <<= 1) {
+        w += __shfl_xor(w, o, 64);
+        mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    }
+    const bool bad = !(w <= 1e36);
+    if (part == 0) s_bad[row] = bad ? 1 : 0;
+    if (bad) mx = 0.0f;
+#pragma unroll
+    for (int o = 4; o <= 32; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0) s_max[wave] = mx;
+    __syncthreads();
+    const double m = fmax((double)fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3])), sqrt(fmax(r2, 0.0)));
+    // scale: m s in [2^13, 2^14); within 2^+-100 of 1 (outside it the margin is infinite)
+    const int ex = m > 0.0 && m < 1e300 ? ilogb(m) : 0;
+    const bool scalable = ex >= -87 && ex <= 113 && m < 1e300;
+    const float scale = scalable ? ldexpf(1.0f, 13 - ex) : 1.0f;
+    const bool real = row < rows;
+    float e = 0.0f;
+    if (real) {
+        const double ed = sm.a * w + sm.f * (w + m * m) + sm.b;
+        e = bad || !scalable || !(ed < 1e37) ? INFINITY : __double2float_ru(ed);
+        if (part == 0) {
+            const double c = 0.25 * r2 - 0.5 * w;
+            caug[R * 64 + row] = (float)c;
+            sc[R * 64 + row] = e < INFINITY ? (float)((c - (double)e) * (double)scale) : 0.0f;
         }
-        e_row = wave_max(a.emarg[R * 64 + lane]);
-    } else {
+    } else if (part == 0) {
+        caug[R * 64 + row] = 0.0f;
+        sc[R * 64 + row] = -3e37f;
+    }
 #pragma unroll
-        for (int g = 0; g < G; ++g) A0[g] = A1[g] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int o = 4; o <= 32; o <<= 1) e = fmaxf(e, __shfl_xor(e, o, 64));
+    if (lane == 0) s_e[wave] = e;
+    __syncthreads();
+    if (tid == 0) {
+        se[R] = fmaxf(fmaxf(s_e[0], s_e[1]), fmaxf(s_e[2], s_e[3]));
+        ss[R] = scale;
     }
-    const float4 *__restrict__ xb = (const float4 *)a.xca;
+    const bool zero = !scalable;
+    for (int t = tid; t < KS * 128; t += 256) {
+        const int l = t & 63, b = (t >> 6) & 1, s = t >> 7;
+        const int r = 32 * b + (l & 31), k0 = 16 * s + 8 * (l >> 5);
+        v8h h, lo;
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-        const int q = threadIdx.x + 256 * u;
-        if (q < kTileF4) sB[0][q] = xb[C0 * kTileF4 + q];
+        for (int q = 0; q < 8; ++q) {
+            const float x = zero || s_bad[r] ? 0.0f : sxr[r * (kD + 1) + k0 + q] * scale;
+            h[q] = (_Float16)x;
+            lo[q] = (_Float16)(x - (float)h[q]);
+        }
+        uint4 *dst = sx + R * (KS * 256) + l;
+        dst[split_at<KS>(s, 0, b)] = __builtin_bit_cast(uint4, h);
+        dst[split_at<KS>(s, 1, b)] = __builtin_bit_cast(uint4, lo);
     }
-    if (wave == 0) {
-        const float e = wave_max(a.emarg[C0 * 64 + lane]);
-        if (lane == 0) sE[0] = e;
+}
+
+__device__ __forceinline__ v16f mfma_f16(const uint4 &a, const uint4 &b, const v16f &c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
+}
+
+// Row operands of one wave: both parts of both 32-row blocks, and the FP32
+// step's row side [c_i s, s] (lanes 0-31: dimension 0, lanes 32-63: dimension 1).
+template <int KS>
+struct SplitRows {
+    uint4 h0[KS], h1[KS], l0[KS], l1[KS];
+    float c0, c1;
+};
+
+template <int KS>
+__device__ __forceinline__ void split_load_rows(const DistArgs &a, int64_t R, SplitRows<KS> &A) {
+    const int lane = threadIdx.x & 63;
+    const uint4 *__restrict__ p = a.sx + R * (KS * 256) + lane;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        A.h0[s] = p[split_at<KS>(s, 0, 0)];
+        A.h1[s] = p[split_at<KS>(s, 0, 1)];
+        A.l0[s] = p[split_at<KS>(s, 1, 0)];
+        A.l1[s] = p[split_at<KS>(s, 1, 1)];
     }
+    const float sr = a.ss[R];
+    A.c0 = lane < 32 ? a.sc[R * 64 + lane] : sr;
+    A.c1 = lane < 32 ? a.sc[R * 64 + 32 + lane] : sr;
+}
+
+// U = T - e_i - e_j (scaled by both tiles' scales) of a 64x64 tile pair; the
+// column operands at pb (lane offset included), cb0 / cb1 the FP32 step's
+// column side [s', c_j s'].  The small products first, then c, then h.h'.
+template <int KS>
+__device__ __forceinline__ void split_tile(const SplitRows<KS> &A, const uint4 *pb, float cb0, float cb1, MfmaTile &t) {
+    mfma_zero(t);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        const uint4 h0 = pb[split_at<KS>(s, 0, 0)], h1 = pb[split_at<KS>(s, 0, 1)];
+        const uint4 l0 = pb[split_at<KS>(s, 1, 0)], l1 = pb[split_at<KS>(s, 1, 1)];
+        t.c00 = mfma_f16(A.l0[s], h0, t.c00);
+        t.c01 = mfma_f16(A.l0[s], h1, t.c01);
+        t.c10 = mfma_f16(A.l1[s], h0, t.c10);
+        t.c11 = mfma_f16(A.l1[s], h1, t.c11);
+        t.c00 = mfma_f16(A.h0[s], l0, t.c00);
+        t.c01 = mfma_f16(A.h0[s], l1, t.c01);
+        t.c10 = mfma_f16(A.h1[s], l0, t.c10);
+        t.c11 = mfma_f16(A.h1[s], l1, t.c11);
+    }
+    mfma_step(t, A.c0, A.c1, cb0, cb1);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        const uint4 h0 = pb[split_at<KS>(s, 0, 0)], h1 = pb[split_at<KS>(s, 0, 1)];
+        t.c00 = mfma_f16(A.h0[s], h0, t.c00);
+        t.c01 = mfma_f16(A.h0[s], h1, t.c01);
+        t.c10 = mfma_f16(A.h1[s], h0, t.c10);
+        t.c11 = mfma_f16(A.h1[s], h1, t.c11);
+    }
+}
+
+// Sign bits of a lane's values x(v, first block), x(v, second block) in the
+// layout of pack_halves: one v_alignbit per value, highest bit first.
+template <typename F>
+__device__ __forceinline__ uint32_t sign_bits(F &&x) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int q = 31; q >= 0; --q) {
+        const int v = 4 * (q >> 3) + (q & 3);
+        w = __builtin_amdgcn_alignbit(w, __float_as_uint(x(v, (q >> 2) & 1)), 31);
+    }
+    return w;
+}
+
+// Decides and stores one tile pair from U.  A clear sign bit proves a
+// neighbour, U < -E2 with E2 >= 2 (e_i + e_j) proves none; the elements in
+// between are queued.  As signed integers the negative floats ascend with
+// their magnitude from INT_MIN (-0), so the integer minimum over the values is
+// the negative one nearest zero: one v_min3 per two values tells whether the
+// lane has a band element.  E2 not finite: every element is settled in FP64.
+// km: the mirror pair's index, -1 without one.
+__device__ __forceinline__ int split_settle_store(const DistArgs &a, const MfmaTile &t, int64_t k, int64_t R,
+                                                  int64_t C, float E2, BandSlots &bs, int64_t km) {
+    const int lane = threadIdx.x & 63;
+    const bool finite = E2 < INFINITY;
+    const float nE = -E2;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        mx = fmaxf(fmaxf(mx, t.c00[v]), t.c01[v]);
+        mx = fmaxf(fmaxf(mx, t.c10[v]), t.c11[v]);
+    }
+    uint64_t word = 0, colword = 0;
+    bool queued = false;
+    if (!finite || __ballot(!(mx < nE))) {
+        uint32_t pa = 0xffffffffu, pb = 0xffffffffu;  // not in
+        uint64_t flags = 0ull;
+        if (finite) {
+            pa = sign_bits([&](int v, int blk) { return blk ? t.c10[v] : t.c00[v]; });
+            pb = sign_bits([&](int v, int blk) { return blk ? t.c11[v] : t.c01[v]; });
+            int mi = INT_MAX;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                mi = min(min(mi, __float_as_int(t.c00[v])), __float_as_int(t.c01[v]));
+                mi = min(min(mi, __float_as_int(t.c10[v])), __float_as_int(t.c11[v]));
+            }
+            if (__ballot(mi <= __float_as_int(nE))) {
+                const uint32_t na = sign_bits([&](int v, int blk) { return (blk ? t.c10[v] : t.c00[v]) + E2; });
+                const uint32_t nb = sign_bits([&](int v, int blk) { return (blk ? t.c11[v] : t.c01[v]) + E2; });
+                flags = (uint64_t)(pa & ~na) | ((uint64_t)(pb & ~nb) << 32);
+            }
+        } else {
+            flags = ~0ull;
+        }
+        if (__ballot(flags != 0ull)) {
+            // (padding rows and columns have no flags unless every element has)
+            if (!finite) {
+                for (int e = 0; e < 64; ++e) {
+                    int row, col;
+                    band_element(lane, e, row, col);
+                    if (R * 64 + row >= a.n || C * 64 + col >= a.n) flags &= ~(1ull << e);
+                }
+            }
+            if (__ballot(flags != 0ull)) {
+                queued = true;
+                queue_band(a, k, R, flags, bs);
+            }
+        }
+        pa = ~pa;
+        pb = ~pb;
+        colword = merge_col_words(pa & 0x0f0f0f0fu, (pa >> 4) & 0x0f0f0f0fu, pb & 0x0f0f0f0fu,
+                                  (pb >> 4) & 0x0f0f0f0fu);
+        word = transpose_bits(colword);
+    }
+    // as store_pair; padding rows and columns hold no bits here
+    const bool any = __ballot(word != 0ull) != 0ull;
+    const bool mirrored = km >= 0;
+    if (lane == 0) {
+        a.pair_nz[k - a.k_base] = any ? 1 : 0;
+        if (mirrored) a.pair_nz[km - a.k_base] = any ? 1 : 0;
+    }
+    if (!any && !queued) return 0;
+    a.mask[(k - a.k_base) * 64 + lane] = word;
+    if (mirrored) {
+        a.mask[(km - a.k_base) * 64 + lane] = colword;
+        const int cd = __popcll(colword);
+        if (cd) atomicAdd(&a.deg[C * 64 + lane], cd);
+    }
+    return __popcll(word);
+}
+
+// E2 of a tile pair in scaled units: 2 (largest margin of the row tile + of
+// the column tile), rounded up.
+__device__ __forceinline__ float split_e2(float e_row, float e_col, float s_row, float s_col) {
+    return 2.0f * (e_row + e_col) * (1.0f + 0x1p-20f) * s_row * s_col;
+}
+
+// Distance kernel of the split form, dense layout.  A workgroup takes 4
+// consecutive row tiles (one per wave, operands in registers) and a chunk of at
+// most 64 column tiles within one word of the live bitmap: each wave takes its
+// row's live bits, pair index and mirrors once, so the column loop depends on
+// no index loads.  The columns live for any of the 4 rows are staged through
+// two LDS buffers; a column's global loads are issued one whole iteration
+// before they are written to LDS (between the MFMAs and the stores of the
+// current pair, so that waiting for them waits for no recent store), the next
+// column's behind them.
+// n = 2e5, d = 64 (859,000 tile pairs): 1.72 ms against 6.1 to 6.4 ms of the FP32
+// MFMA form with one column of look-ahead and its index loads in the loop;
+// n = 1e5, d = 16 (758,000 pairs): 0.53 against 2.0 ms.  At d = 64 the matrix
+// units are busy 0.46 of the time (a bare loop of this MFMA reaches 1750
+// TFLOP/s here; without the epilogue the launch takes 1.40 ms, without any
+// staging 1.30), at d = 16 the vector instructions of the epilogue bound it.
+// Chunks of 16, 32 and 64 columns: 1.84, 1.77 and 1.76 ms.
+template <int KS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, KS <= 1 ? 3 : 2))) void k_dist_split(DistArgs a, int64_t n_rt,
+                                                                                               int64_t n_rb) {
+    constexpr int kTile = KS * 256;  // uint4 per tile
+    __shared__ uint4 sB[2][kTile];
+    __shared__ uint64_t s_live[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t cc = blockIdx.x / n_rb, rb = blockIdx.x - cc * n_rb;
+    const int64_t R_lo = a.R0 + 4 * rb, R = R_lo + wave;
+    const int64_t c_lo = cc * a.col_chunk;
+    if (a.sym && c_lo + a.col_chunk <= R_lo) return;  // the whole workgroup
+    const bool rvalid = R < a.R0 + n_rt;
+    // this row's columns: bit b = column tile 64 cw + b
+    const int64_t cw = c_lo >> 6, cbase = cw << 6;
+    uint64_t row_live = 0ull, mine = 0ull;
+    int64_t kbase = 0;
+    if (rvalid) {
+        const int64_t left = a.n_tiles - cbase;
+        const uint64_t exist = left >= 64 ? ~0ull : (1ull << left) - 1ull;
+        if (a.live) {
+            row_live = a.live[R * a.live_words + cw];
+            kbase = a.tp_ptr[R] + a.live_pre[R * a.live_words + cw];
+        } else {
+            row_live = exist;
+            kbase = R * a.n_tiles + cbase;
+        }
+        const uint64_t part = a.col_chunk >= 64 ? ~0ull : ((1ull << a.col_chunk) - 1ull) << (c_lo & 63);
+        mine = row_live & exist & part;
+        if (a.sym && R > cbase) mine &= R - cbase >= 64 ? 0ull : ~((1ull << (R - cbase)) - 1ull);
+    }
+    if (lane == 0) s_live[wave] = mine;
+    __syncthreads();
+    uint64_t cols = uniform64(s_live[0] | s_live[1] | s_live[2] | s_live[3]);
+    if (cols == 0ull) return;  // the whole workgroup
+    mine = (uint64_t)uniform64((int64_t)mine);
+    row_live = (uint64_t)uniform64((int64_t)row_live);
+    kbase = uniform64(kbase);
+    // mirrors, lane b for column bit b
+    int64_t mir = -1;
+    if (a.sym && ((mine >> lane) & 1ull) && cbase + lane != R)
+        mir = mirror_of(a, kbase + __popcll(row_live & ((1ull << lane) - 1ull)), R, cbase + lane);
+    SplitRows<KS> A;
+    split_load_rows<KS>(a, rvalid ? R : R_lo, A);
+    const float e_row = a.se[rvalid ? R : R_lo], s_row = a.ss[rvalid ? R : R_lo];
+    int cur = __ffsll((unsigned long long)cols) - 1;
+    cols &= cols - 1;
+    int nxt = cols ? __ffsll((unsigned long long)cols) - 1 : cur;
+    // named registers, not an array: the compiler places a private array here
+    // in LDS and waits for its loads at once
+    uint4 g0, g1, g2, g3, g4, g5, g6, g7;
+#define CNN_SPLIT_FETCH(b)                                                              \
+    {                                                                                   \
+        const uint4 *__restrict__ src = a.sx + (cbase + (b)) * kTile + threadIdx.x;     \
+        g0 = src[0];                                                                    \
+        if constexpr (KS > 1) g1 = src[256];                                            \
+        if constexpr (KS > 2) g2 = src[512];                                            \
+        if constexpr (KS > 3) g3 = src[768];                                            \
+        if constexpr (KS > 4) g4 = src[1024];                                           \
+        if constexpr (KS > 5) g5 = src[1280];                                           \
+        if constexpr (KS > 6) g6 = src[1536];                                           \
+        if constexpr (KS > 7) g7 = src[1792];                                           \
+    }
+#define CNN_SPLIT_PLACE(buf_)                                                           \
+    {                                                                                   \
+        uint4 *dst = sB[buf_] + threadIdx.x;                                            \
+        dst[0] = g0;                                                                    \
+        if constexpr (KS > 1) dst[256] = g1;                                            \
+        if constexpr (KS > 2) dst[512] = g2;                                            \
+        if constexpr (KS > 3) dst[768] = g3;                                            \
+        if constexpr (KS > 4) dst[1024] = g4;                                           \
+        if constexpr (KS > 5) dst[1280] = g5;                                           \
+        if constexpr (KS > 6) dst[1536] = g6;                                           \
+        if constexpr (KS > 7) dst[1792] = g7;                                           \
+    }
+    auto col_term = [&](int b, float &c0, float &c1) {
+        const int64_t C = cbase + b;
+        const float s = a.ss[C];
+        const float x0 = a.sc[C * 64 + (lane & 31)], x1 = a.sc[C * 64 + 32 + (lane & 31)];
+        c0 = lane < 32 ? s : x0;
+        c1 = lane < 32 ? s : x1;
+    };
+    float cb0, cb1, nb0, nb1;
+    CNN_SPLIT_FETCH(cur)
+    col_term(cur, cb0, cb1);
+    float e_col = a.se[cbase + cur], s_col = a.ss[cbase + cur];
+    CNN_SPLIT_PLACE(0)
+    CNN_SPLIT_FETCH(nxt)
     __syncthreads();
     const int64_t i = R * 64 + lane;
-    int mydeg = 0;
+    int mydeg = 0, buf = 0;
     BandSlots bs;
-    for (int idx = 0; idx < n_col; ++idx) {
-        const int64_t C = col_at(idx);
-        const int buf = idx & 1;
-        const bool more = idx + 1 < n_col;
-        // the next tile's operands and margins (the last tile reloads itself, in
-        // bounds, unused): loads in flight during this tile's MFMAs, no branch
-        const int64_t Cn = more ? col_at(idx + 1) : C;
-        // named registers, not an array: a private array here is placed in LDS or
-        // scratch memory by the compiler, which waits for the loads right away
-        static_assert(kPer <= 5, "staging registers");
-        const float4 *src = xb + Cn * kTileF4;
-        float4 n0, n1, n2, n3, n4;
-        n0 = src[min((int)threadIdx.x, kTileF4 - 1)];
-        if constexpr (kPer > 1) n1 = src[min((int)threadIdx.x + 256, kTileF4 - 1)];
-        if constexpr (kPer > 2) n2 = src[min((int)threadIdx.x + 512, kTileF4 - 1)];
-        if constexpr (kPer > 3) n3 = src[min((int)threadIdx.x + 768, kTileF4 - 1)];
-        if constexpr (kPer > 4) n4 = src[min((int)threadIdx.x + 1024, kTileF4 - 1)];
-        const float e_nx = a.emarg[Cn * 64 + lane];
-        const bool work = rvalid && (!a.sym || C >= R) && pair_live(a, R, C);
-        // the pair's mask index and its mirror's, loaded during the MFMAs
-        int64_t kp = 0, km = -1;
-        if (work) {
-            kp = pair_index(a, R, C);
-            if (a.sym && C != R) km = mirror_of(a, kp, R, C);
-        }
+    for (;;) {
+        const bool more = cols != 0ull;
+        cols &= cols - 1;
+        const int nxt2 = cols ? __ffsll((unsigned long long)cols) - 1 : nxt;
+        col_term(nxt, nb0, nb1);
+        float e_nx = a.se[cbase + nxt], s_nx = a.ss[cbase + nxt];
+        const bool work = ((mine >> cur) & 1ull) != 0ull;
+        const float E2 = split_e2(e_row, e_col, s_row, s_col);
         MfmaTile t;
-        mfma_zero(t);
+        if (work) split_tile<KS>(A, &sB[buf][lane], cb0, cb1, t);
+        asm volatile("" ::: "memory");  // the LDS stores stay behind the MFMAs
+        if (more) CNN_SPLIT_PLACE(buf ^ 1)
+        // the next column's terms are waited for here, behind the MFMAs: taken
+        // at the loop's end, the wait would cover the loads and stores below
+        asm volatile("" : "+v"(nb0), "+v"(nb1), "+v"(e_nx), "+v"(s_nx)::"memory");
+        if (more) CNN_SPLIT_FETCH(nxt2)
+        asm volatile("" ::: "memory");
         if (work) {
-            const float4 *sb = &sB[buf][h * 64 + r];
-            float4 B0 = sb[0], B1 = sb[32];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                float4 nB0 = B0, nB1 = B1;
-                if (g + 1 < G) {
-                    nB0 = sb[(g + 1) * 128];
-                    nB1 = sb[(g + 1) * 128 + 32];
-                }
-                mfma_group(t, A0[g], A1[g], B0, B1, g + 1 < G ? 4 : tail);
-                B0 = nB0;
-                B1 = nB1;
-            }
+            const int64_t k = kbase + __popcll(row_live & ((1ull << cur) - 1ull));
+            const uint32_t mlo = __builtin_amdgcn_readlane((uint32_t)(uint64_t)mir, cur);
+            const uint32_t mhi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)mir >> 32), cur);
+            const int64_t km = (int64_t)(((uint64_t)mhi << 32) | mlo);
+            mydeg += split_settle_store(a, t, k, R, cbase + cur, E2, bs, km);
         }
-        const float e_col = sE[buf];
-        // Stage the next tile between the MFMAs and the epilogue: the loads have
-        // had the MFMAs' time to arrive, and no store of this tile is in flight
-        // yet (waiting for the loads would also wait for those).  The empty asm
-        // keeps the compiler from moving the LDS stores up next to their loads.
-        asm volatile("" ::: "memory");
-        if (more) {
-            float4 *dst = sB[buf ^ 1];
-            const int q = threadIdx.x;
-            dst[q] = n0;  // kTileF4 >= 384
-            if constexpr (kPer > 1) { if (q + 256 < kTileF4) dst[q + 256] = n1; }
-            if constexpr (kPer > 2) { if (q + 512 < kTileF4) dst[q + 512] = n2; }
-            if constexpr (kPer > 3) { if (q + 768 < kTileF4) dst[q + 768] = n3; }
-            if constexpr (kPer > 4) { if (q + 1024 < kTileF4) dst[q + 1024] = n4; }
-            if (wave == 0) {
-                const float e = wave_max(e_nx);
-                if (lane == 0) sE[buf ^ 1] = e;
-            }
-        }
-        asm volatile("" ::: "memory");
-        if (work) mydeg += mfma_settle_store(a, t, kp, R, C, i, pair_margin(e_row, e_col), bs, km);
+        if (!more) break;
         __syncthreads();
+        cur = nxt;
+        nxt = nxt2;
+        cb0 = nb0;
+        cb1 = nb1;
+        e_col = e_nx;
+        s_col = s_nx;
+        buf ^= 1;
     }
+#undef CNN_SPLIT_FETCH
+#undef CNN_SPLIT_PLACE
     band_slots_release(a, bs);
     if (rvalid && mydeg && i < a.n) atomicAdd(&a.deg[i], mydeg);
+}
+
+// Band elements of the tile pairs that found the record list full (one wave per
+// pair, grid-stride, the count read on the device): U is recomputed by the same
+// instructions, every element in the band is decided in FP64 in reference
+// order by its own lane, and its bits are added to the stored words and degrees
+// of the pair and of its mirror.
+template <int KS>
+__global__ __launch_bounds__(64) void k_split_band(DistArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int64_t n_redo = (int64_t)*a.redo_cnt;
+    unsigned hits = 0, flips = 0;
+    double maxerr = 0.0;
+    for (int64_t slot = blockIdx.x; slot < n_redo; slot += gridDim.x) {
+        const int64_t k = a.redo[2 * slot], R = a.redo[2 * slot + 1];
+        int64_t kb, ke;
+        tile_range(a, R, kb, ke);
+        const int64_t C = uniform64(tile_col(a, k, kb));
+        SplitRows<KS> A;
+        split_load_rows<KS>(a, R, A);
+        const float s_col = a.ss[C];
+        const float cb0 = lane < 32 ? s_col : a.sc[C * 64 + (lane & 31)];
+        const float cb1 = lane < 32 ? s_col : a.sc[C * 64 + 32 + (lane & 31)];
+        const float E2 = split_e2(a.se[R], a.se[C], a.ss[R], s_col);
+        const bool finite = E2 < INFINITY;
+        MfmaTile t;
+        split_tile<KS>(A, a.sx + C * (KS * 256) + lane, cb0, cb1, t);
+        uint32_t half[2] = {0u, 0u};  // new bits, layout of pack_halves
+#pragma unroll
+        for (int e = 0; e < 64; ++e) {
+            const int v = 4 * ((e & 31) >> 3) + (e & 3), blk = ((e >> 2) & 1) + 2 * (e >> 5);
+            const float x = blk == 0 ? t.c00[v] : blk == 1 ? t.c10[v] : blk == 2 ? t.c01[v] : t.c11[v];
+            int row, col;
+            band_element(lane, e, row, col);
+            const int64_t gi = R * 64 + row, gj = C * 64 + col;
+            const bool neg = (__float_as_uint(x) >> 31) != 0u;
+            const bool band = !finite || (neg && (__float_as_uint(x + E2) >> 31) == 0u);
+            if (band && gi < a.n && gj < a.n) {
+                const double exd = exact_d2(a.xw64, a.d, gi, gj);
+                const bool in = exd <= a.bp.r2;
+                if (in) half[e >> 5] |= 1u << (e & 31);
+                ++hits;
+                const double d2 = a.bp.r2 - 2.0 * (double)gram_value(a, gi, gj);
+                flips += (in != (d2 <= a.bp.r2));
+                const double err = fabs(d2 - exd);
+                if (err == err) maxerr = fmax(maxerr, err);
+            }
+        }
+        const uint64_t colword = merge_col_words(half[0] & 0x0f0f0f0fu, (half[0] >> 4) & 0x0f0f0f0fu,
+                                                 half[1] & 0x0f0f0f0fu, (half[1] >> 4) & 0x0f0f0f0fu);
+        const uint64_t word = transpose_bits(colword);  // lane i: row i's extra bits
+        const bool any_new = __ballot(word != 0ull) != 0ull;
+        if (a.pair_nz && lane == 0 && any_new) mark_pair_nz(a, k, R, C);
+        if (word) {
+            atomicOr(&a.mask[(k - a.k_base) * 64 + lane], (unsigned long long)word);
+            atomicAdd(&a.deg[R * 64 + lane], __popcll(word));
+        }
+        if (a.sym && C != R && colword) {
+            const int64_t km = mirror_of(a, k, R, C);
+            atomicOr(&a.mask[(km - a.k_base) * 64 + lane], (unsigned long long)colword);
+            atomicAdd(&a.deg[C * 64 + lane], __popcll(colword));
+        }
+    }
+    flush_band(a, hits, flips, maxerr);
+}
+
+// Calls f(std::integral_constant<int, KS>) for the steps of d dimensions.
+template <typename F>
+static void split_dispatch(int d, F &&f) {
+    switch ((d + 15) / 16) {
+        case 1: f(std::integral_constant<int, 1>{}); break;
+        case 2: f(std::integral_constant<int, 2>{}); break;
+        case 3: f(std::integral_constant<int, 3>{}); break;
+        case 4: f(std::integral_constant<int, 4>{}); break;
+        case 5: f(std::integral_constant<int, 5>{}); break;
+        case 6: f(std::integral_constant<int, 6>{}); break;
+        case 7: f(std::integral_constant<int, 7>{}); break;
+        default: f(std::integral_constant<int, 8>{}); break;
+    }
+}
+
+// Column tiles per workgroup of k_dist_split: at most the tuned chunk and one
+// word of the live bitmap; fewer while the launch has fewer than four
+// workgroups per compute unit.
+static int split_chunk(int64_t n_rb, int64_t n_tiles, bool sym, int tuned) {
+    int chunk = 64;
+    while (chunk > 8 && (chunk > tuned || n_rb * ceil_div(n_tiles, chunk) < (sym ? 2 : 1) * 1024)) chunk >>= 1;
+    return chunk;
 }
 
 // Band elements of the queued tile pairs (one wave per pair): the FP32 values
@@ -1947,62 +2347,63 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // decided in FP64 in reference order (one wave-wide evaluation per element),
 // and its bits are added to the stored words (and to the degrees) of the pair
 // and of its mirror.
-__global__ __launch_bounds__(64) void k_dist_mfma_band(DistArgs a, int64_t n_redo) {
-    const int64_t slot = blockIdx.x;
-    if (slot >= n_redo) return;
+__global__ __launch_bounds__(64) void k_dist_mfma_band(DistArgs a) {
     const int lane = threadIdx.x & 63;
     const int r = lane & 31, h = lane >> 5;
-    const int64_t k = a.redo[2 * slot], R = a.redo[2 * slot + 1];
-    int64_t kb, ke;
-    tile_range(a, R, kb, ke);
-    const int64_t C = uniform64(tile_col(a, k, kb));
-    const float e_row = wave_max(a.emarg[R * 64 + lane]);
-    const float E = pair_margin(e_row, wave_max(a.emarg[C * 64 + lane]));
-    const float nE = -E;
-    const MfmaTile t = mfma_tile(a, R, C);
+    const int64_t n_redo = (int64_t)*a.redo_cnt;
     unsigned hits = 0, flips = 0;
     double maxerr = 0.0;
-    const uint64_t cm = valid_cols(a.n, C);
-    const bool col_a = (cm >> r) & 1ull, col_b = (cm >> (32 + r)) & 1ull;
-    uint32_t a_lo = 0, a_hi = 0, b_lo = 0, b_hi = 0;
-    // element (row 4h + rr + rb, column cb + r) of lane (r, h) with value x,
-    // settled by its own lane: the exact FP64 distance in reference order
-    auto settle = [&](float x, int rr, int rb, int cb, bool col_ok, uint32_t &part) {
-        const bool band = !(x >= E) && !(x < nE) && col_ok && (R * 64 + 4 * h + rr + rb) < a.n;
-        if (band) {
-            const int64_t gi = R * 64 + 4 * h + rr + rb;
-            const int64_t gj = C * 64 + cb + r;
-            const double e = exact_d2(a.xw64, a.d, gi, gj);
-            const bool in = e <= a.bp.r2;
-            if (in) part |= 1u << rr;
-            ++hits;
-            const double d2 = a.bp.r2 - 2.0 * (double)x;
-            flips += (in != (d2 <= a.bp.r2));
-            const double err = fabs(d2 - e);
-            if (err == err) maxerr = fmax(maxerr, err);
+    for (int64_t slot = blockIdx.x; slot < n_redo; slot += gridDim.x) {
+        const int64_t k = a.redo[2 * slot], R = a.redo[2 * slot + 1];
+        int64_t kb, ke;
+        tile_range(a, R, kb, ke);
+        const int64_t C = uniform64(tile_col(a, k, kb));
+        const float e_row = wave_max(a.emarg[R * 64 + lane]);
+        const float E = pair_margin(e_row, wave_max(a.emarg[C * 64 + lane]));
+        const float nE = -E;
+        const MfmaTile t = mfma_tile(a, R, C);
+        const uint64_t cm = valid_cols(a.n, C);
+        const bool col_a = (cm >> r) & 1ull, col_b = (cm >> (32 + r)) & 1ull;
+        uint32_t a_lo = 0, a_hi = 0, b_lo = 0, b_hi = 0;
+        // element (row 4h + rr + rb, column cb + r) of lane (r, h) with value x,
+        // settled by its own lane: the exact FP64 distance in reference order
+        auto settle = [&](float x, int rr, int rb, int cb, bool col_ok, uint32_t &part) {
+            const bool band = !(x >= E) && !(x < nE) && col_ok && (R * 64 + 4 * h + rr + rb) < a.n;
+            if (band) {
+                const int64_t gi = R * 64 + 4 * h + rr + rb;
+                const int64_t gj = C * 64 + cb + r;
+                const double e = exact_d2(a.xw64, a.d, gi, gj);
+                const bool in = e <= a.bp.r2;
+                if (in) part |= 1u << rr;
+                ++hits;
+                const double d2 = a.bp.r2 - 2.0 * (double)x;
+                flips += (in != (d2 <= a.bp.r2));
+                const double err = fabs(d2 - e);
+                if (err == err) maxerr = fmax(maxerr, err);
+            }
+        };
+    #pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int rr = 8 * (v >> 2) + (v & 3);
+            settle(t.c00[v], rr, 0, 0, col_a, a_lo);
+            settle(t.c10[v], rr, 32, 0, col_a, a_hi);
+            settle(t.c01[v], rr, 0, 32, col_b, b_lo);
+            settle(t.c11[v], rr, 32, 32, col_b, b_hi);
         }
-    };
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int rr = 8 * (v >> 2) + (v & 3);
-        settle(t.c00[v], rr, 0, 0, col_a, a_lo);
-        settle(t.c10[v], rr, 32, 0, col_a, a_hi);
-        settle(t.c01[v], rr, 0, 32, col_b, b_lo);
-        settle(t.c11[v], rr, 32, 32, col_b, b_hi);
-    }
-    const uint64_t colword = merge_col_words(a_lo, a_hi, b_lo, b_hi);
-    const uint64_t word = transpose_bits(colword);  // lane i: row i's extra bits
-    const int64_t i = R * 64 + lane;
-    const bool any_new = __ballot(word != 0ull) != 0ull;
-    if (a.pair_nz && lane == 0 && any_new) mark_pair_nz(a, k, R, C);
-    if (word) {
-        atomicOr(&a.mask[(k - a.k_base) * 64 + lane], (unsigned long long)word);
-        atomicAdd(&a.deg[i], __popcll(word));
-    }
-    if (a.sym && C != R && colword) {
-        const int64_t km = a.tp_ptr ? a.mirror[k] : C * a.n_tiles + R;
-        atomicOr(&a.mask[(km - a.k_base) * 64 + lane], (unsigned long long)colword);
-        atomicAdd(&a.deg[C * 64 + lane], __popcll(colword));
+        const uint64_t colword = merge_col_words(a_lo, a_hi, b_lo, b_hi);
+        const uint64_t word = transpose_bits(colword);  // lane i: row i's extra bits
+        const int64_t i = R * 64 + lane;
+        const bool any_new = __ballot(word != 0ull) != 0ull;
+        if (a.pair_nz && lane == 0 && any_new) mark_pair_nz(a, k, R, C);
+        if (word) {
+            atomicOr(&a.mask[(k - a.k_base) * 64 + lane], (unsigned long long)word);
+            atomicAdd(&a.deg[i], __popcll(word));
+        }
+        if (a.sym && C != R && colword) {
+            const int64_t km = a.tp_ptr ? a.mirror[k] : C * a.n_tiles + R;
+            atomicOr(&a.mask[(km - a.k_base) * 64 + lane], (unsigned long long)colword);
+            atomicAdd(&a.deg[C * 64 + lane], __popcll(colword));
+        }
     }
     flush_band(a, hits, flips, maxerr);
 }
@@ -2463,8 +2864,6 @@ __global__ void k_scan_total(int64_t *p, int64_t idx, const int32_t *cnt) { p[id
 
 // ------------------------------------------------------------------ host side
 
-static double gamma_m(int m, double u) { return m * u / (1.0 - m * u); }
-
 // Guard band for the FP32 direct form.  |d2_fp32 - s64| <= E where, near the
 // threshold (magnitudes D <= 2 r2):
 //   FP32 accumulation of d rounded squares of rounded differences: gamma_{d+2}(u32) * D
@@ -2554,59 +2953,26 @@ static void launch_dist(cnn_ctx *ctx, const DistArgs &a, int64_t n_rt, bool band
         b.band_cap = cap;
         b.redo_cnt = (unsigned long long *)(cnt.p + 1);
         b.redo = redo.p;
-        const int G = a.dp / 8;
-        if ((!a.tp_ptr || a.live) && !a.tile_valid && G >= 3 && G <= 10) {
-            // dense pairs, row operands in registers, column tiles shared through LDS
-            b.col_chunk = mfma_col_chunk;
-            // culled items range from no work to the full chunk: round-robin
-            // dealing balances them (measured 5.5 ms against 9.2 ms for
-            // contiguous ranges at n = 2e5, d = 64)
-            b.deal_rr = a.live ? 1 : 0;
-            const int64_t n_rb = ceil_div(n_rt, 4), n_cc = ceil_div(a.n_tiles, b.col_chunk);
-            int64_t n_items = 0;
-            for (int64_t cc = 0; cc < n_cc; ++cc)
-                n_items += mfma_chunk_blocks(b.sym, cc, b.col_chunk, b.n_tiles, b.R0, n_rb);
-            const int64_t per_xcd = ceil_div(n_items, 8);
-            if (8 * per_xcd > (int64_t)INT32_MAX) throw HipFailure{hipErrorInvalidValue, "MFMA grid too large"};
-            const dim3 g8((unsigned)std::max<int64_t>(8 * per_xcd, 1));
-            switch (G) {
-#define CNN_MFMA_LDS(GG) \
-    case GG: k_dist_mfma_lds<GG><<<g8, block, 0, s>>>(b, n_rt, n_rb, n_cc, per_xcd, n_items); break;
-                CNN_MFMA_LDS(3)
-                CNN_MFMA_LDS(4)
-                CNN_MFMA_LDS(5)
-                CNN_MFMA_LDS(6)
-                CNN_MFMA_LDS(7)
-                CNN_MFMA_LDS(8)
-                CNN_MFMA_LDS(9)
-                default: k_dist_mfma_lds<10><<<g8, block, 0, s>>>(b, n_rt, n_rb, n_cc, per_xcd, n_items); break;
-#undef CNN_MFMA_LDS
-            }
+        const unsigned rblocks = (unsigned)std::min<int64_t>(std::max<int64_t>(batch_pairs, 1), 2048);
+        if (a.sx) {
+            const int64_t n_rb = ceil_div(n_rt, 4);
+            b.col_chunk = split_chunk(n_rb, a.n_tiles, a.sym != 0, mfma_col_chunk);
+            const int64_t items = n_rb * ceil_div(a.n_tiles, b.col_chunk);
+            if (items > (int64_t)INT32_MAX) throw HipFailure{hipErrorInvalidValue, "distance grid too large"};
+            split_dispatch(a.d, [&](auto ks) {
+                k_dist_split<decltype(ks)::value><<<(unsigned)items, block, 0, s>>>(b, n_rt, n_rb);
+            });
         } else {
             k_dist_mfma<<<grid, block, 0, s>>>(b);
         }
         CNN_HIP(hipGetLastError());
         CNN_HIP(hipEventRecord(ctx->ev[7], s));
-        PinnedReads rd(ctx);
-        const int64_t *counts = rd.get(cnt.p, 2);
-        rd.wait();
-        const int64_t n_elems = std::min(counts[0], cap), n_redo = counts[1];
-        if (n_redo > batch_pairs) throw HipFailure{hipErrorUnknown, "band pair queue overflow"};
-        if (n_elems > 0) {
-            Scratch<int32_t> rcnt(ctx, n_elems);
-            Scratch<int64_t> roff(ctx, n_elems);
-            k_band_count<<<(unsigned)ceil_div(n_elems, 4), 256, 0, s>>>(list.p, n_elems, rcnt.p);
-            CNN_HIP(hipGetLastError());
-            exclusive_scan_i32_to_i64(ctx, rcnt.p, roff.p, n_elems);
-            const int64_t n_el = read_scalar(ctx, roff.p + (n_elems - 1)) + read_scalar(ctx, rcnt.p + (n_elems - 1));
-            if (n_el > 0) {
-                Scratch<int64_t> elem(ctx, n_el);
-                k_band_list<<<(unsigned)ceil_div(n_elems, 4), 256, 0, s>>>(list.p, n_elems, roff.p, elem.p);
-                k_band_settle<<<(unsigned)std::min<int64_t>(ceil_div(n_el, 256), 4096), 256, 0, s>>>(b, elem.p, n_el);
-                CNN_HIP(hipGetLastError());
-            }
-        }
-        if (n_redo > 0) k_dist_mfma_band<<<(unsigned)n_redo, 64, 0, s>>>(b, n_redo);
+        // both counts are read on the device; every queued pair fits redo
+        k_band_settle<<<(unsigned)std::min<int64_t>(ceil_div(cap, kBandGroup), 2048), 256, 0, s>>>(b);
+        if (a.sx)
+            split_dispatch(a.d, [&](auto ks) { k_split_band<decltype(ks)::value><<<rblocks, 64, 0, s>>>(b); });
+        else
+            k_dist_mfma_band<<<rblocks, 64, 0, s>>>(b);
     } else if (!band && wide_kmax(a) > 0) {
         const int kmax = wide_kmax(a);
         const int64_t n_pad = a.n_tiles * 64;
@@ -2799,18 +3165,33 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
     const int64_t n_pad = T * 64;
     const bool gram = band && d >= kMfmaMinD;
     const int dp = gram ? ((d + 2 + 7) / 8) * 8 : d;  // augmented MFMA rows: d + 2 dims, padded to 8
-    std::unique_ptr<Scratch<float>> xra, xca, emarg;
-    if (gram) {
+    const bool split = gram && d <= kSplitMaxD;
+    std::unique_ptr<Scratch<float>> xra, xca, emarg, caug, sc, se, ss;
+    std::unique_ptr<Scratch<uint4>> sx;
+    if (split) {
+        const int ks = (d + 15) / 16;
+        const SplitMargin sm = split_margin(d, ks, dtype == CNN_F64, g->r2);
+        sx.reset(new Scratch<uint4>(ctx, T * ks * 256));
+        sc.reset(new Scratch<float>(ctx, n_pad));
+        caug.reset(new Scratch<float>(ctx, n_pad));
+        se.reset(new Scratch<float>(ctx, T));
+        ss.reset(new Scratch<float>(ctx, T));
+        split_dispatch(d, [&](auto kc) {
+            k_split_tiles<decltype(kc)::value><<<(unsigned)T, 256, 0, s>>>(g->xw32, n, d, g->r2, sm, sx->p, sc->p,
+                                                                          se->p, ss->p, caug->p);
+        });
+        CNN_HIP(hipGetLastError());
+    } else if (gram) {
         float gka = 0.0f, gkb = 0.0f;
         make_band_gram(d, dp, dtype == CNN_F64, g->r2, gka, gkb);
         xra.reset(new Scratch<float>(ctx, n_pad * dp));
         xca.reset(new Scratch<float>(ctx, n_pad * dp));
         emarg.reset(new Scratch<float>(ctx, n_pad));
-        Scratch<float> caug(ctx, n_pad);
+        caug.reset(new Scratch<float>(ctx, n_pad));
         k_augment_rows<<<(unsigned)ceil_div(n_pad, 256), 256, 0, s>>>(g->xw32, n, n_pad, d, (float)(0.25 * g->r2), gka,
-                                                                      gkb, emarg->p, caug.p);
+                                                                      gkb, emarg->p, caug->p);
         k_augment_pack<<<(unsigned)ceil_div(n_pad * 2 * (dp / 8), 256), 256, 0, s>>>(
-            g->xw32, n, n_pad, d, dp / 8, caug.p, (float4 *)xra->p, (float4 *)xca->p);
+            g->xw32, n, n_pad, d, dp / 8, caug->p, (float4 *)xra->p, (float4 *)xca->p);
         CNN_HIP(hipGetLastError());
     }
 
@@ -3051,6 +3432,13 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
         a.xra = xra ? xra->p : nullptr;
         a.xca = xca ? xca->p : nullptr;
         a.emarg = emarg ? emarg->p : nullptr;
+        if (split) {
+            a.sx = sx->p;
+            a.sc = sc->p;
+            a.se = se->p;
+            a.ss = ss->p;
+        }
+        a.caug = caug ? caug->p : nullptr;
         a.col_chunk = g->tune.wide_col_chunk;
         a.pair_nz = pair_nz_p;
         a.pair_groups = gmask ? gmask->p : nullptr;

@@ -1,0 +1,87 @@
+"""The split FP16 Gram form (banded precision, 16 <= d <= 128): neighbour lists
+equal the oracle's FP64 ones at every number of MFMA steps and its remainders,
+ragged tiles, the ordered and the plain layout, tiles of very different scales,
+subnormal FP16 parts, non-finite and huge points, and with the record list full."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle as C
+from commonnnclustering_amd import engine
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(x, r):
+    want_rp, want_col = C.neighbours_csr(x, r, use_grid=False)
+    X = torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    rp, col, st = engine.radius_csr(X, float(r) ** 2, "f32_band")
+    assert (rp.cpu().numpy() == want_rp).all()
+    assert (col.cpu().numpy() == want_col).all()
+    return st
+
+
+def _quantile_radius(x, q):
+    y = x[np.random.default_rng(0).permutation(len(x))[:300]].astype(np.float64)
+    d2 = ((y[:, None] - y[None]) ** 2).sum(-1)
+    return float(np.sqrt(np.quantile(d2[np.triu_indices(len(y), 1)], q)))
+
+
+@pytest.mark.parametrize("d", [16, 17, 31, 32, 33, 48, 49, 64, 65, 79, 80, 81, 96, 100, 112, 113, 127, 128, 129])
+@pytest.mark.parametrize("n,dtype", [(130, np.float32), (2113, np.float64)])
+def test_every_step_count(cuda, d, n, dtype):
+    rng = np.random.default_rng(d * n)
+    x = (2.0 * rng.normal(size=(5, d)))[rng.integers(0, 5, n)] + rng.normal(size=(n, d))
+    _check(x.astype(dtype), _quantile_radius(x, 0.1))
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1.0, 1e6, 1e15])
+@pytest.mark.parametrize("d", [16, 40])
+def test_scales(cuda, d, scale):
+    rng = np.random.default_rng(3)
+    x = rng.normal(size=(700, d))
+    x[::7] *= 1e-4          # small next to large in one tile
+    x[64:128] *= 1e-6       # whole tiles small
+    x[130] = 0.0
+    x = (x * scale).astype(np.float32)
+    for q in (0.02, 0.3):
+        _check(x, _quantile_radius(x, q))
+    _check(x, 1e-7 * scale)  # far below the coordinates: zero and duplicate distances only
+    _check(x, 1e3 * scale)   # far above them: all pairs
+
+
+def test_offset_and_boundary(cuda):
+    rng = np.random.default_rng(4)
+    x = (rng.integers(-3, 4, size=(900, 24)) + 100.0).astype(np.float32)  # many pairs at exactly r
+    st = _check(x, np.sqrt(150.0))
+    assert st["band_hits"] > 0
+    x = (rng.normal(size=(900, 20)) + 1e4).astype(np.float32)  # far from the origin: most pairs in the band
+    _check(x, _quantile_radius(x, 0.1))
+
+
+def test_nonfinite_and_huge(cuda):
+    rng = np.random.default_rng(5)
+    x = rng.normal(size=(400, 18)).astype(np.float32)
+    x[3, 2], x[70, 0], x[140, 17], x[200], x[399, 1] = np.nan, np.inf, -np.inf, 3e37, 2e18
+    _check(x, 4.0)
+
+
+@pytest.mark.parametrize("records", ["1", "9"])
+@pytest.mark.parametrize("d", [16, 64, 100])
+def test_full_record_list(cuda, monkeypatch, records, d):
+    """Pairs beyond the record list recompute their values and settle them."""
+    monkeypatch.setenv("CNN_HIP_BAND_RECORDS", records)
+    rng = np.random.default_rng(d)
+    x = (rng.integers(-2, 3, size=(1500, d)) + 10.0).astype(np.float32)
+    st = _check(x, np.sqrt(4.0 * d))
+    assert st["band_hits"] > 0
+
+
+def test_row_tile_batches(cuda, monkeypatch):
+    """Several row-tile batches: every pair evaluated from both sides."""
+    monkeypatch.setenv("CNN_HIP_MASK_BUDGET", str(512 * 200))
+    rng = np.random.default_rng(8)
+    for n in (1500, 2500):
+        x = rng.normal(size=(n, 33)).astype(np.float32)
+        _check(x, _quantile_radius(x, 0.05))
