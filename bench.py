@@ -144,8 +144,10 @@ def distance_roofline(gs, d, precision, workload_name):
         if kernel == "k_dist_split":  # three FP16 products per FP32 product
             peak = FP16_PEAK_TFLOPS / 3
     else:
-        kernel = "k_dist_f64_cols" if d <= 8 else "k_dist_f64_wide"
-        bound, peak = "valu", FP64_PEAK_TFLOPS
+        kernel = "k_dist_f64_cols" if d <= 8 else "k_dist_gram64" if d <= 120 else "k_dist_f64_generic"
+        bound, peak = ("mfma" if kernel == "k_dist_gram64" else "valu"), FP64_PEAK_TFLOPS
+        if kernel == "k_dist_gram64":  # one FMA per dimension
+            flops = 2.0 * d * pairs
     achieved = flops / (ms * 1e-3) / 1e12
     traffic = None
     path = TRAFFIC_FILES.get((kernel, workload_name))

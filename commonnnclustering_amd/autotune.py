@@ -9,7 +9,7 @@ the tuner checks that every candidate gives the same labels.
 Tuned here (``cnn_tune_params``):
   mfma_col_chunk  column tiles per workgroup of the dense MFMA distance kernel
                   (FP32-banded form, d >= 16)
-  wide_col_chunk  column tiles per workgroup of the dense plain-FP64 kernel
+  wide_col_chunk  tile pairs per workgroup, at most, of the dense plain-FP64 kernel
   emit_waves      waves per workgroup of the neighbour-list emission
   root_passes     root-hooking passes before the full round of a labelling on lists
   words_min_fill  lists with at least this many entries per 64-bit word are

@@ -780,7 +780,7 @@ struct DistArgs {
     const float *xra;
     const float *xca;
     const float *emarg;
-    // column chunking of the dense wide FP64 kernel (tiles per workgroup)
+    // column tiles (k_dist_split) or pairs (k_dist_gram64) per workgroup
     int64_t col_chunk;
     // packed batches: radius and FP32 band per row tile (nullptr: bp for all)
     const double *tile_r2;
@@ -2024,6 +2024,30 @@ __device__ __forceinline__ uint32_t sign_bits(F &&x) {
     return w;
 }
 
+// Stores pair k's row words and the mirror pair's (km, -1: none), which are the
+// column words, and adds the column side's degrees; returns the row word's
+// popcount.  As store_pair, for column words without bits in padding rows and
+// columns.  force: store empty words too.
+__device__ __forceinline__ int store_words(const DistArgs &a, int64_t k, int64_t km, int64_t C, uint64_t colword,
+                                           bool force = false) {
+    const int lane = threadIdx.x & 63;
+    const bool any = __ballot(colword != 0ull) != 0ull;
+    const bool mirrored = km >= 0;
+    if (lane == 0) {
+        a.pair_nz[k - a.k_base] = any ? 1 : 0;
+        if (mirrored) a.pair_nz[km - a.k_base] = any ? 1 : 0;
+    }
+    if (!any && !force) return 0;
+    const uint64_t word = any ? transpose_bits(colword) : 0ull;
+    a.mask[(k - a.k_base) * 64 + lane] = word;
+    if (mirrored) {
+        a.mask[(km - a.k_base) * 64 + lane] = colword;
+        const int cd = __popcll(colword);
+        if (cd) atomicAdd(&a.deg[C * 64 + lane], cd);
+    }
+    return __popcll(word);
+}
+
 // Decides and stores one tile pair from U.  A clear sign bit proves a
 // neighbour, U < -E2 with E2 >= 2 (e_i + e_j) proves none; the elements in
 // between are queued.  As signed integers the negative floats ascend with
@@ -2042,7 +2066,7 @@ __device__ __forceinline__ int split_settle_store(const DistArgs &a, const MfmaT
         mx = fmaxf(fmaxf(mx, t.c00[v]), t.c01[v]);
         mx = fmaxf(fmaxf(mx, t.c10[v]), t.c11[v]);
     }
-    uint64_t word = 0, colword = 0;
+    uint64_t colword = 0;
     bool queued = false;
     if (!finite || __ballot(!(mx < nE))) {
         uint32_t pa = 0xffffffffu, pb = 0xffffffffu;  // not in
@@ -2082,23 +2106,8 @@ __device__ __forceinline__ int split_settle_store(const DistArgs &a, const MfmaT
         pb = ~pb;
         colword = merge_col_words(pa & 0x0f0f0f0fu, (pa >> 4) & 0x0f0f0f0fu, pb & 0x0f0f0f0fu,
                                   (pb >> 4) & 0x0f0f0f0fu);
-        word = transpose_bits(colword);
     }
-    // as store_pair; padding rows and columns hold no bits here
-    const bool any = __ballot(word != 0ull) != 0ull;
-    const bool mirrored = km >= 0;
-    if (lane == 0) {
-        a.pair_nz[k - a.k_base] = any ? 1 : 0;
-        if (mirrored) a.pair_nz[km - a.k_base] = any ? 1 : 0;
-    }
-    if (!any && !queued) return 0;
-    a.mask[(k - a.k_base) * 64 + lane] = word;
-    if (mirrored) {
-        a.mask[(km - a.k_base) * 64 + lane] = colword;
-        const int cd = __popcll(colword);
-        if (cd) atomicAdd(&a.deg[C * 64 + lane], cd);
-    }
-    return __popcll(word);
+    return store_words(a, k, km, C, colword, queued);
 }
 
 // E2 of a tile pair in scaled units: 2 (largest margin of the row tile + of
@@ -2408,59 +2417,201 @@ __global__ __launch_bounds__(64) void k_dist_mfma_band(DistArgs a) {
     flush_band(a, hits, flips, maxerr);
 }
 
-// Plain FP64 for the dense layout with 4 < d <= KMAX, on a copy of the
-// coordinates zero-padded to KMAX dims: the padded terms add (0 - 0)^2 = +0 at
-// the end of the reference-order sum, which leaves every s_ij unchanged.  The
-// row point lives in VGPRs, column points stream through wave-uniform (scalar)
-// loads.  A workgroup covers 4 consecutive row tiles (one per wave) and a chunk
-// of column tiles, so the 4 waves read the same column rows (scalar-cache
-// reuse); the chunking balances the triangle of the symmetric evaluation.
-// Degrees are accumulated atomically (several chunks contribute to a row).
-template <int KMAX>
-__global__ __launch_bounds__(256) void k_dist_f64_wide(DistArgs a, const double *__restrict__ xp, int64_t n_chunks,
-                                                       int64_t n_rt) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t rg = blockIdx.x / n_chunks, cc = blockIdx.x % n_chunks;
-    const int64_t R = a.R0 + rg * 4 + wave;  // row tiles R0 .. R0 + n_rt - 1 of this batch
-    const int64_t T = a.n_tiles;
-    if (R >= a.R0 + n_rt) return;
-    const int64_t i = R * 64 + lane;
-    double xi[KMAX];
-#pragma unroll
-    for (int k = 0; k < KMAX; ++k) xi[k] = xp[i * KMAX + k];
-    const int64_t c_lo = cc * a.col_chunk, c_hi = min(T, (cc + 1) * a.col_chunk);
-    const int64_t c_begin = a.sym ? max(c_lo, R) : c_lo;
-    int mydeg = 0;
-    for (int64_t C = c_begin; C < c_hi; ++C) {
-        if (!pair_live(a, R, C)) continue;
-        const double *__restrict__ xc = xp + uniform64(C) * 64 * KMAX;
-        uint64_t m = 0;
-#pragma unroll 2
-        for (int jj = 0; jj < 64; jj += 2) {
-            const double *__restrict__ x0 = xc + jj * KMAX;
-            const double *__restrict__ x1 = x0 + KMAX;
-            double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-            for (int k = 0; k < KMAX; ++k) {
-                const double t0 = xi[k] - x0[k];
-                const double t1 = xi[k] - x1[k];
-                s0 = s0 + t0 * t0;
-                s1 = s1 + t1 * t1;
-            }
-            m |= (uint64_t)(s0 <= a.bp.r2) << jj;
-            m |= (uint64_t)(s1 <= a.bp.r2) << (jj + 1);
-        }
-        mydeg += store_pair<true>(a, pair_index(a, R, C), R, i, C, m, false, 0);
-    }
-    if (i < a.n && mydeg) atomicAdd(&a.deg[i], mydeg);
+// ------------------------------------------------------------------ plain FP64, dense layout (8 < d <= 120)
+//
+// T = x_i . x_j + c_i + c_j = (r2 - s_ij)/2 in FP64 on v_mfma_f64_16x16x4_f64:
+// one FMA per pair and dimension on the matrix units, against a separately
+// rounded subtraction, product and addition on the vector units in the
+// reference's order.  T differs from the reference's s_ij by FP64 rounding
+// only, at most e_i + e_j below; a pair whose T lies within that of zero is
+// evaluated in the reference's order by its own lane, so every decision is the
+// reference's.
+constexpr int kGram64MaxD = 120;  // the row tile's operands take at most 60 KB of LDS
+
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// Margin e_i = a w_i + b, w = |x|^2, u = 2^-53: d products and two terms c, each
+// addition at most 2u of Sabs <= (w_i + w_j) + r2/2; w itself (gamma_d w/2) and
+// rounding c; the reference's own rounding near the threshold.
+struct Gram64Margin {
+    double a, b;
+};
+static Gram64Margin gram64_margin(int d, double r2) {
+    const double u = std::ldexp(1.0, -53), g = gamma_m(d + 8, 2.0 * u);
+    Gram64Margin m;
+    m.a = 1.001 * (g + 0.5 * gamma_m(d, u) + 2.0 * u);
+    m.b = 1.001 * (0.25 * g + 2.0 * u + 0.5 * gamma_m(2 * d + 2, u)) * r2 + 1e-300;
+    return m;
 }
 
-__global__ void k_pad_rows(const double *__restrict__ xw64, int64_t n_pad, int d, int kmax, double *__restrict__ xp) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n_pad * kmax) return;
-    const int64_t w = idx / kmax;
-    const int k = (int)(idx - w * kmax);
-    xp[idx] = k < d ? xw64[w * d + k] : 0.0;
+// Packed operands, one workgroup per tile: the double2 at ((t SP + s) 4 + b) 64 + l
+// holds dimensions 8s + l/16 and 8s + 4 + l/16 of point 64t + 16b + l%16, so a
+// wave-wide load of a 16-point block is one contiguous KiB and feeds two MFMA
+// steps.  Also c_i - e_i per point and the largest margin per tile (infinite,
+// with zero operands, where a point is non-finite or huge: such tiles' pairs
+// are evaluated in the reference's order throughout).
+__global__ __launch_bounds__(256) void k_gram64_tiles(const double *__restrict__ xw64, int64_t n, int d, int SP,
+                                                      double r2, Gram64Margin gm, double2 *__restrict__ gx,
+                                                      double *__restrict__ gc, double *__restrict__ ge) {
+    __shared__ double s_e[4];
+    __shared__ int s_bad[64];
+    const int64_t R = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = tid >> 2, part = tid & 3;  // four threads a row
+    const bool real = R * 64 + row < n;
+    const double *__restrict__ x = xw64 + (R * 64 + row) * d;
+    double w = 0.0;
+    if (real)
+        for (int k = part; k < d; k += 4) w += x[k] * x[k];
+    w += __shfl_xor(w, 1, 64);
+    w += __shfl_xor(w, 2, 64);
+    double e = real ? gm.a * w + gm.b : 0.0;
+    const bool bad = !(w <= 1e300) || !(e <= 1e300);
+    if (bad) e = INFINITY;
+    if (part == 0) {
+        s_bad[row] = bad ? 1 : 0;
+        gc[R * 64 + row] = !real ? -1e300 : bad ? 0.0 : (0.25 * r2 - 0.5 * w) - e;
+    }
+#pragma unroll
+    for (int o = 4; o <= 32; o <<= 1) e = fmax(e, __shfl_xor(e, o, 64));
+    if (lane == 0) s_e[wave] = e;
+    __syncthreads();
+    if (tid == 0) ge[R] = fmax(fmax(s_e[0], s_e[1]), fmax(s_e[2], s_e[3]));
+    for (int t = tid; t < SP * 256; t += 256) {
+        const int l = t & 63, b = (t >> 6) & 3, sp = t >> 8;
+        const int r = 16 * b + (l & 15), k = 8 * sp + (l >> 4);
+        double2 v = make_double2(0.0, 0.0);
+        if (R * 64 + r < n && !s_bad[r]) {
+            const double *__restrict__ xr = xw64 + (R * 64 + r) * d;
+            if (k < d) v.x = xr[k];
+            if (k + 4 < d) v.y = xr[k + 4];
+        }
+        gx[R * SP * 256 + t] = v;
+    }
+}
+
+// Lane l of accumulator (rb, cb) holds rows 16 rb + 4 v + l/16 (v = 0..3) of
+// column 16 cb + l%16.
+struct Gram64Tile {
+    v4d c[4][4];
+};
+
+// One workgroup per part of a row tile's candidate pairs (`split` parts): the row
+// operands sit in LDS, each of the 4 waves takes every fourth pair of the part
+// with its column operands straight from global memory, the next step's loads
+// in flight during a step's 32 MFMAs; no barrier inside the loop.
+// Bound by the FP64 matrix units (4096 d FMAs per tile pair, 16 a cycle and SIMD):
+// n = 5e4, d = 64 (63,700 tile pairs) 0.66 ms, 0.43 ms of it MFMA time at full
+// rate; the vector form (three separately rounded operations per pair and
+// dimension, columns through scalar loads, up to 32 columns of 4 row tiles one
+// after another in a workgroup) took 4.1 ms.  n = 5e4, d = 100, which had only
+// the runtime-d form: 39.2 -> 1.36 ms a fit.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_dist_gram64(
+    DistArgs a, const double2 *__restrict__ gx, const double *__restrict__ gc, const double *__restrict__ ge, int SP,
+    int split) {
+    extern __shared__ double2 s_rows[];
+    double *s_c = (double *)(s_rows + SP * 256);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int g = lane >> 4, c15 = lane & 15;
+    const int64_t R = a.R0 + blockIdx.x / split;
+    const int part = blockIdx.x % split;
+    int64_t kb, ke;
+    tile_range(a, R, kb, ke);
+    int64_t k0 = kb;  // symmetric evaluation: from the tile's own pair on
+    if (a.sym) k0 = pair_index(a, R, R);
+    if (k0 + part * 4 >= ke) return;  // the whole workgroup
+    for (int t = threadIdx.x; t < SP * 256; t += 256) s_rows[t] = gx[R * SP * 256 + t];
+    if (threadIdx.x < 64) s_c[threadIdx.x] = gc[R * 64 + threadIdx.x];
+    __syncthreads();
+    const double e_row = ge[R];
+    int mydeg = 0;
+    for (int64_t k = k0 + part * 4 + wave; k < ke; k += 4 * split) {
+        const int64_t C = uniform64(tile_col(a, k, kb));
+        const int64_t km = a.sym && C != R ? mirror_of(a, k, R, C) : -1;
+        const double2 *__restrict__ pb = gx + C * SP * 256 + lane;
+        Gram64Tile t;
+        double2 b[4];
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) b[cb] = pb[cb * 64];
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            const double cc = gc[C * 64 + 16 * cb + c15];
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) t.c[rb][cb][v] = s_c[16 * rb + 4 * v + g] + cc;
+        }
+        const double e_col = ge[C];
+        for (int sp = 0; sp < SP; ++sp) {
+            const int nx = sp + 1 < SP ? sp + 1 : sp;  // (the last step reloads itself, unused)
+            double2 nb[4], ar[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) nb[q] = pb[nx * 256 + q * 64];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) ar[q] = s_rows[sp * 256 + q * 64 + lane];
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < 4; ++cb)
+                    t.c[rb][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[rb].x, b[cb].x, t.c[rb][cb], 0, 0, 0);
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < 4; ++cb)
+                    t.c[rb][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[rb].y, b[cb].y, t.c[rb][cb], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) b[q] = nb[q];
+        }
+        // U = T - e_i - e_j: sign clear proves a neighbour, U < -E2 proves none
+        const double E2 = 2.0 * (e_row + e_col) * (1.0 + 0x1p-40);
+        const bool finite = E2 < INFINITY;
+        // the negative value nearest zero by its high word (signed integers of
+        // negative doubles ascend with their magnitude)
+        int mi = INT_MAX;
+        uint64_t in[4];
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            uint32_t half[2] = {0u, 0u};
+#pragma unroll
+            for (int z = 15; z >= 0; --z) {
+                const int hi = __double2hiint(t.c[z >> 2][cb][z & 3]);
+                mi = min(mi, hi);
+                half[z >> 3] = (half[z >> 3] << 4) | ((uint32_t)~hi >> 31);
+            }
+            in[cb] = finite ? ((uint64_t)half[1] << 32) | half[0] : 0ull;
+        }
+        if (!finite || __ballot(mi <= __double2hiint(-E2))) {
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) {
+                // not out: the sign of U + E2 is clear (the sum's sign is exact)
+                uint32_t half[2] = {0u, 0u};
+#pragma unroll
+                for (int z = 15; z >= 0; --z) {
+                    const int hi = __double2hiint(t.c[z >> 2][cb][z & 3] + E2);
+                    half[z >> 3] = (half[z >> 3] << 4) | ((uint32_t)~hi >> 31);
+                }
+                uint64_t f = finite ? (((uint64_t)half[1] << 32) | half[0]) & ~in[cb] : 0x1111111111111111ull;
+                const int64_t gj = C * 64 + 16 * cb + c15;
+                while (f) {
+                    const int p = __ffsll((unsigned long long)f) - 1;
+                    f &= f - 1;
+                    const int64_t gi = R * 64 + p + g;
+                    if (gi < a.n && gj < a.n && exact_d2(a.xw64, a.d, gi, gj) <= a.bp.r2) in[cb] |= 1ull << p;
+                }
+            }
+        }
+        // column words: bit 4 z + g from each of the four lanes of a column
+        uint64_t colword = 0ull;
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            uint64_t x = in[cb] << g;
+            x |= __shfl_xor(x, 16, 64);
+            x |= __shfl_xor(x, 32, 64);
+            if (g == cb) colword = x;
+        }
+        mydeg += store_words(a, k, km, C, colword);
+    }
+    if (mydeg && R * 64 + lane < a.n) atomicAdd(&a.deg[R * 64 + lane], mydeg);
 }
 
 // Pairs per wave of k_pair_info in one-sided builds, and the count of such
@@ -2920,10 +3071,10 @@ static void make_band_gram(int d, int dp, bool rounded_coords, double r2, float 
     kb = (float)(S * B * 0.5 * r2 + 1e-30);
 }
 
-// Padded width of the wide FP64 kernel (dense layout), 0 if unused.
-static int wide_kmax(const DistArgs &a) {
-    if ((a.tp_ptr && !a.live) || a.d <= 8 || a.d > 64) return 0;
-    return a.d <= 8 ? 8 : a.d <= 16 ? 16 : a.d <= 32 ? 32 : 64;
+// Whether the plain FP64 build takes the matrix-unit form: the dense layout's
+// dimensions up to kGram64MaxD (lists only where they are the live pairs).
+static bool uses_gram64(const DistArgs &a) {
+    return (!a.tp_ptr || a.live) && !a.tile_valid && a.d > kSpatialMaxD && a.d <= kGram64MaxD;
 }
 
 // Events 6 and 7 bracket the main distance kernel (without guard-band settling).
@@ -2973,18 +3124,19 @@ static void launch_dist(cnn_ctx *ctx, const DistArgs &a, int64_t n_rt, bool band
             split_dispatch(a.d, [&](auto ks) { k_split_band<decltype(ks)::value><<<rblocks, 64, 0, s>>>(b); });
         else
             k_dist_mfma_band<<<rblocks, 64, 0, s>>>(b);
-    } else if (!band && wide_kmax(a) > 0) {
-        const int kmax = wide_kmax(a);
-        const int64_t n_pad = a.n_tiles * 64;
-        Scratch<double> xp(ctx, n_pad * kmax);
-        k_pad_rows<<<(unsigned)ceil_div(n_pad * kmax, 256), 256, 0, s>>>(a.xw64, n_pad, a.d, kmax, xp.p);
-        const int64_t n_rg = ceil_div(n_rt, 4);
-        const int64_t n_chunks = ceil_div(a.n_tiles, a.col_chunk);
-        dim3 g2((unsigned)(n_rg * n_chunks));
-        if (kmax == 8) k_dist_f64_wide<8><<<g2, block, 0, s>>>(a, xp.p, n_chunks, n_rt);
-        else if (kmax == 16) k_dist_f64_wide<16><<<g2, block, 0, s>>>(a, xp.p, n_chunks, n_rt);
-        else if (kmax == 32) k_dist_f64_wide<32><<<g2, block, 0, s>>>(a, xp.p, n_chunks, n_rt);
-        else k_dist_f64_wide<64><<<g2, block, 0, s>>>(a, xp.p, n_chunks, n_rt);
+    } else if (!band && uses_gram64(a)) {
+        const int SP = (a.d + 7) / 8;
+        const int64_t T = a.n_tiles;
+        Scratch<double2> gx(ctx, T * SP * 256);
+        Scratch<double> gc(ctx, T * 64), ge(ctx, T);
+        k_gram64_tiles<<<(unsigned)T, 256, 0, s>>>(a.xw64, a.n, a.d, SP, a.bp.r2, gram64_margin(a.d, a.bp.r2), gx.p,
+                                                  gc.p, ge.p);
+        // parts of a row tile's pairs: at most the tuned number of pairs each, and
+        // about 4096 workgroups of at least 4 pairs
+        const int64_t per_row = ceil_div(batch_pairs, std::max<int64_t>(n_rt, 1)) / (a.sym ? 2 : 1) + 1;
+        const int split = (int)std::max(ceil_div(per_row, a.col_chunk), std::min(ceil_div(per_row, 4), ceil_div(4096, n_rt)));
+        k_dist_gram64<<<(unsigned)(n_rt * split), block, SP * 256 * sizeof(double2) + 64 * sizeof(double), s>>>(
+            a, gx.p, gc.p, ge.p, SP, split);
     } else if (!band) {
         switch (a.d) {
             case 1: k_dist_f64_cols<1><<<grid, block, 0, s>>>(a); break;
