@@ -272,8 +272,8 @@ cnn_graph *graph_build(cnn_ctx *ctx, const void *X, int64_t n, int32_t d, int32_
 void graph_free(cnn_graph *g);
 void graph_export(cnn_ctx *ctx, const cnn_graph *g, int64_t *row_ptr, int32_t *col);
 // Throws InvalidArg unless row_ptr (n+1, from 0) is non-decreasing and every
-// row of col is strictly ascending within [0, n).
-void validate_csr(cnn_ctx *ctx, const int64_t *row_ptr, const int32_t *col, int64_t n);
+// row of col is strictly ascending within [0, n).  Returns row_ptr[n].
+int64_t validate_csr(cnn_ctx *ctx, const int64_t *row_ptr, const int32_t *col, int64_t n);
 cnn_graph *graph_rethreshold(cnn_ctx *ctx, const cnn_graph *g, double r2, int32_t precision);
 // Emits the neighbour lists (col, selfpos) of a graph that holds only its row
 // words; no-op when they exist.  Safe to call from several contexts at once;
@@ -338,6 +338,7 @@ struct LabelRequest {
     // tuned switches (graph requests take the graph's; caller lists the d = 0 class)
     int root_passes = 2;
     int64_t words_min_fill = 8;
+    int64_t nnz = -1;   // row_ptr[n] when the caller knows it
 };
 
 // Sort key layout of a packed batch: dataset << ds_shift | (size_max - size)

@@ -1474,24 +1474,40 @@ __global__ __launch_bounds__(256) void k_row_word_count(const int64_t *__restric
 }
 
 // Entries and words of every stride-th row, summed into sums[0] / sums[1]:
-// the automatic similarity choice estimates the lists' fill from them.
+// the automatic similarity choice estimates the lists' fill from them.  A few
+// hundred workgroups add their sums once each (two updates of the same
+// addresses per row took 220 us for 9000 rows and 15 us for 500, the latter 5 us
+// as here).
 __global__ __launch_bounds__(256) void k_row_word_sample(const int64_t *__restrict__ row_ptr,
                                                          const int32_t *__restrict__ col, int64_t n, int64_t stride,
                                                          unsigned long long *__restrict__ sums) {
-    const int lane = threadIdx.x & 63;
-    const int64_t w = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * stride;
-    if (w >= n) return;
-    const int64_t b = row_ptr[w], e = row_ptr[w + 1];
-    int total = 0;
-    for (int64_t t0 = b; t0 < e; t0 += 64) {
-        const int64_t t = t0 + lane;
-        bool head = false;
-        if (t < e) head = t == b || (col[t - 1] >> 6) != (col[t] >> 6);
-        total += __popcll(__ballot(head));
+    __shared__ unsigned long long s_entries[4], s_words[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long entries = 0, words = 0;
+    for (int64_t w = ((int64_t)blockIdx.x * 4 + wave) * stride; w < n; w += (int64_t)gridDim.x * 4 * stride) {
+        const int64_t b = row_ptr[w], e = row_ptr[w + 1];
+        int total = 0;
+        for (int64_t t0 = b; t0 < e; t0 += 64) {
+            const int64_t t = t0 + lane;
+            bool head = false;
+            if (t < e) head = t == b || (col[t - 1] >> 6) != (col[t] >> 6);
+            total += __popcll(__ballot(head));
+        }
+        entries += (unsigned long long)(e - b);
+        words += (unsigned long long)total;
     }
-    if (lane == 0 && total) {
-        atomicAdd(&sums[0], (unsigned long long)(e - b));
-        atomicAdd(&sums[1], (unsigned long long)total);
+    if (lane == 0) {
+        s_entries[wave] = entries;
+        s_words[wave] = words;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        entries = s_entries[0] + s_entries[1] + s_entries[2] + s_entries[3];
+        words = s_words[0] + s_words[1] + s_words[2] + s_words[3];
+        if (words) {
+            atomicAdd(&sums[0], entries);
+            atomicAdd(&sums[1], words);
+        }
     }
 }
 
@@ -1595,12 +1611,12 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
         if (!build && req.words_min_fill > 0 && req.words_min_fill <= (int64_t)1 << 24) {
             // automatic choice: the fill of every stride-th row decides, the
             // stride at least 16 and large enough to sample about 2^21 entries
-            const int64_t nnz = read_scalar(ctx, req.row_ptr + n);
+            const int64_t nnz = req.nnz >= 0 ? req.nnz : read_scalar(ctx, req.row_ptr + n);
             const int64_t stride = std::max<int64_t>(16, ceil_div(nnz, (int64_t)1 << 21));
             Scratch<unsigned long long> sums(ctx, 2);
             fill_u64(ctx, sums.p, 0, 2);
             const int64_t rows = ceil_div(n, stride);
-            k_row_word_sample<<<blocks_for(rows, 4), 256, 0, s>>>(req.row_ptr, req.col, n, stride, sums.p);
+            k_row_word_sample<<<(unsigned)std::min<int64_t>(blocks_for(rows, 4), 512), 256, 0, s>>>(req.row_ptr, req.col, n, stride, sums.p);
             CNN_HIP(hipGetLastError());
             PinnedReads rd(ctx);
             const unsigned long long *h = rd.get(sums.p, 2);
@@ -1952,35 +1968,44 @@ void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabe
 // ------------------------------------------------------------------ caller CSR validation
 
 // Flags rows that are not strictly ascending or hold indices outside [0, n),
-// and offsets that decrease.  Precondition (caller contract): col holds at
-// least row_ptr[n] entries and row_ptr is n+1 long.
-__global__ void k_validate_csr(const int64_t *__restrict__ row_ptr, const int32_t *__restrict__ col, int64_t n,
-                               int64_t nnz_cap, unsigned long long *bad) {
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// offsets that decrease, and a bad first or last offset; one wave per row (one
+// thread per row took 90 us for 8001 rows of 640 entries, 4 us as here).
+// Precondition (caller contract): col holds at least row_ptr[n] entries and
+// row_ptr is n+1 long.
+__global__ __launch_bounds__(256) void k_validate_csr(const int64_t *__restrict__ row_ptr,
+                                                      const int32_t *__restrict__ col, int64_t n,
+                                                      unsigned long long *bad) {
+    const int lane = threadIdx.x & 63;
+    const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (w >= n) return;
-    const int64_t b = row_ptr[w], e = row_ptr[w + 1];
-    if (b < 0 || e < b || e > nnz_cap) { atomicOr(bad, 1ull); return; }
-    int32_t prev = -1;
-    for (int64_t t = b; t < e; ++t) {
-        const int32_t j = col[t];
-        if (j <= prev || (int64_t)j >= n) { atomicOr(bad, 2ull); return; }
-        prev = j;
+    const int64_t b = row_ptr[w], e = row_ptr[w + 1], nnz = row_ptr[n];
+    if (w == 0 && lane == 0 && (b != 0 || nnz < 0)) atomicOr(bad, 4ull);
+    if (b < 0 || e < b || e > nnz) {
+        if (lane == 0) atomicOr(bad, 1ull);
+        return;
     }
+    bool wrong = false;
+    for (int64_t t = b + lane; t < e; t += 64) {
+        const int32_t j = col[t], prev = t > b ? col[t - 1] : -1;
+        wrong = wrong || j <= prev || (int64_t)j >= n;
+    }
+    if (__ballot(wrong) != 0ull && lane == 0) atomicOr(bad, 2ull);
 }
 
-void validate_csr(cnn_ctx *ctx, const int64_t *row_ptr, const int32_t *col, int64_t n) {
-    if (n == 0) return;
-    hipStream_t s = ctx->stream;
-    const int64_t first = read_scalar(ctx, row_ptr);
-    const int64_t nnz = read_scalar(ctx, row_ptr + n);
-    if (first != 0 || nnz < 0) throw InvalidArg{"row_ptr must start at 0 and end at nnz >= 0"};
+int64_t validate_csr(cnn_ctx *ctx, const int64_t *row_ptr, const int32_t *col, int64_t n) {
+    if (n == 0) return 0;
     Scratch<unsigned long long> bad(ctx, 1);
-    CNN_HIP(hipMemsetAsync(bad.p, 0, sizeof(unsigned long long), s));
-    k_validate_csr<<<(unsigned)ceil_div(n, 256), 256, 0, s>>>(row_ptr, col, n, nnz, bad.p);
+    fill_u64(ctx, bad.p, 0ull, 1);
+    k_validate_csr<<<(unsigned)ceil_div(n, 4), 256, 0, ctx->stream>>>(row_ptr, col, n, bad.p);
     CNN_HIP(hipGetLastError());
-    const unsigned long long flags = read_scalar(ctx, bad.p);
-    if (flags & 1ull) throw InvalidArg{"row_ptr is not non-decreasing within [0, nnz]"};
-    if (flags & 2ull) throw InvalidArg{"neighbour rows must be strictly ascending with indices in [0, n)"};
+    PinnedReads rd(ctx);
+    const unsigned long long *flags = rd.get(bad.p);
+    const int64_t *nnz = rd.get(row_ptr + n);
+    rd.wait();
+    if (*flags & 4ull) throw InvalidArg{"row_ptr must start at 0 and end at nnz >= 0"};
+    if (*flags & 1ull) throw InvalidArg{"row_ptr is not non-decreasing within [0, nnz]"};
+    if (*flags & 2ull) throw InvalidArg{"neighbour rows must be strictly ascending with indices in [0, n)"};
+    return *nnz;
 }
 
 // ------------------------------------------------------------------ generic sort_by_size
@@ -2034,10 +2059,86 @@ __global__ void k_seg_write(const int32_t *vals, const int32_t *segid, const int
     labels[vals[t]] = seglab[segid[t] - 1];
 }
 
+// sort_by_size through a table over the labels 0 .. n (what the fits assign):
+// members and first index per label (runs of equal labels combined before the
+// atomics), the clusters collected and ranked by k_rank_clusters_small, labels
+// rewritten.  flags[0] clusters, [1] a label outside the table, [2] more
+// clusters than that kernel ranks: nothing is written then.
+__global__ __launch_bounds__(256) void k_label_table(const int64_t *__restrict__ labels, int64_t n,
+                                                     int32_t *__restrict__ cnt, int32_t *__restrict__ first,
+                                                     unsigned long long *__restrict__ flags, int steps) {
+    const int64_t base = run_base(steps);
+    KeyRun run;
+    bool outside = false;
+    for (int it = 0; it < steps; ++it) {
+        const int64_t i = base + it * 64 + __lane_id();
+        const int64_t l = i < n ? labels[i] : 0;
+        const bool in = l >= 0 && l <= n;
+        outside = outside || !in;
+        run_add(run, cnt, first, in && l != 0, in ? (int)l : 0, (int)i);
+    }
+    run_flush(run, cnt, first);
+    if (__ballot(outside) != 0ull && __lane_id() == 0) flags[1] = 1ull;
+}
+
+__global__ void k_label_clusters(const int32_t *__restrict__ cnt, const int32_t *__restrict__ first, int64_t n,
+                                 int64_t member_cutoff, unsigned long long *__restrict__ K, uint64_t *__restrict__ keys,
+                                 int32_t *__restrict__ vals) {
+    const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (l > n || cnt[l] == 0 || (int64_t)cnt[l] < member_cutoff) return;
+    const unsigned long long idx = atomicAdd(K, 1ull);
+    keys[idx] = ((uint64_t)(uint32_t)(0x7fffffff - cnt[l]) << 32) | (uint32_t)first[l];
+    vals[idx] = (int32_t)l;
+}
+
+__global__ void k_label_rewrite(int64_t *__restrict__ labels, int64_t n, const int32_t *__restrict__ newlab,
+                                const unsigned long long *__restrict__ flags) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && !flags[1] && !flags[2]) labels[i] = newlab[labels[i]];
+}
+
+__global__ void k_label_clear(int32_t *cnt, int32_t *first, int32_t *newlab, int64_t count,
+                              unsigned long long *flags) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < 3) flags[i] = 0ull;
+    if (i >= count) return;
+    cnt[i] = 0;
+    first[i] = INT_MAX;
+    newlab[i] = 0;
+}
+
+// The number of clusters kept, or -1 when the table does not cover the labels
+// (they are unchanged then).
+static int64_t sort_by_size_table(cnn_ctx *ctx, int64_t *labels, int64_t n, int64_t member_cutoff,
+                                  int64_t max_clusters) {
+    hipStream_t s = ctx->stream;
+    Scratch<int32_t> cnt(ctx, n + 1), first(ctx, n + 1), newlab(ctx, n + 1), vals(ctx, n + 1);
+    Scratch<uint64_t> keys(ctx, n + 1);
+    Scratch<unsigned long long> flags(ctx, 3);
+    const int steps = run_steps(n);
+    k_label_clear<<<blocks_for(n + 1), 256, 0, s>>>(cnt.p, first.p, newlab.p, n + 1, flags.p);
+    k_label_table<<<blocks_for(n, 256 * steps), 256, 0, s>>>(labels, n, cnt.p, first.p, flags.p, steps);
+    k_label_clusters<<<blocks_for(n + 1), 256, 0, s>>>(cnt.p, first.p, n, member_cutoff, flags.p, keys.p, vals.p);
+    k_rank_clusters_small<<<1, kSmallClusters, 0, s>>>(keys.p, vals.p, flags.p, max_clusters, newlab.p, flags.p + 2);
+    k_label_rewrite<<<blocks_for(n), 256, 0, s>>>(labels, n, newlab.p, flags.p);
+    CNN_HIP(hipGetLastError());
+    PinnedReads rd(ctx);
+    const unsigned long long *h = rd.get(flags.p, 3);
+    rd.wait();
+    if (h[1] || h[2]) return -1;
+    const int64_t K = (int64_t)h[0];
+    return max_clusters >= 0 ? std::min<int64_t>(K, max_clusters) : K;
+}
+
 int64_t sort_by_size_generic(cnn_ctx *ctx, int64_t *labels, int64_t n, int64_t member_cutoff, int64_t max_clusters) {
     hipStream_t s = ctx->stream;
     if (n == 0) return 0;
     if (n >= (int64_t)INT32_MAX) throw InvalidArg{"n exceeds the int32 index range"};
+    // labels as the fits assign them (0 .. n, at most 1024 clusters kept) need no
+    // sort: five kernels and one host read against 22 launches and four reads
+    // (n = 8000: 47 against 330 us of a traced call)
+    const int64_t kept_small = sort_by_size_table(ctx, labels, n, member_cutoff, max_clusters);
+    if (kept_small >= 0) return kept_small;
     Scratch<int64_t> keys(ctx, n);
     Scratch<int32_t> vals(ctx, n), segid(ctx, n);
     Scratch<uint8_t> head(ctx, n);
@@ -2095,9 +2196,10 @@ int cnn_labels_from_csr(cnn_ctx *ctx, const int64_t *row_ptr, const int32_t *col
         if (n > 0 && (!row_ptr || !col || !labels)) throw InvalidArg{"null buffer"};
         if (n >= (int64_t)INT32_MAX) throw InvalidArg{"n exceeds the int32 index range"};
         CNN_HIP(hipSetDevice(ctx->device));
-        validate_csr(ctx, row_ptr, col, n);
+        const int64_t nnz = validate_csr(ctx, row_ptr, col, n);
         LabelRequest r{row_ptr, col, n, nullptr, c_sim, m_core, consider, current_start, sim_mode,
                        false, false, 2, -1, labels};
+        r.nnz = nnz;
         const TuneParams t = tune_lookup(0, n, CNN_PLAIN_F64);
         r.root_passes = t.root_passes;
         r.words_min_fill = t.words_min_fill;

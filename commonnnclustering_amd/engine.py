@@ -275,18 +275,24 @@ def labels_from_csr(row_ptr: torch.Tensor, col: torch.Tensor, c_sim: int, m_core
     if not (row_ptr.is_cuda and col.is_cuda and row_ptr.is_contiguous() and col.is_contiguous()):
         raise ValueError("row_ptr and col must be contiguous CUDA tensors")
     if n > 0:
-        if int(row_ptr[0]) != 0 or bool((row_ptr[1:] < row_ptr[:-1]).any()):
+        first, last = row_ptr[::n].tolist()  # (the order in between is checked with the lists)
+        if first != 0 or last < 0:
             raise ValueError("row_ptr must start at 0 and be non-decreasing")
-        if int(row_ptr[-1]) > col.numel():
-            raise ValueError(f"row_ptr[-1] = {int(row_ptr[-1])} exceeds len(col) = {col.numel()}")
+        if last > col.numel():
+            raise ValueError(f"row_ptr[-1] = {last} exceeds len(col) = {col.numel()}")
     if labels is None:
         labels = torch.zeros(n, dtype=torch.int64, device=device)
     _check_labels(labels, n, consider)
     col_arg = col if col.numel() else torch.zeros(1, dtype=torch.int32, device=device)
     st = LabelStats()
-    ctx.check(_lib.lib().cnn_labels_from_csr(ctx.handle, ptr(row_ptr), ptr(col_arg), n, int(c_sim), int(m_core),
-                                             ptr(consider), int(current_start), int(sim_mode), ptr(labels),
-                                             ctypes.byref(st)), "cnn_labels_from_csr")
+    try:
+        ctx.check(_lib.lib().cnn_labels_from_csr(ctx.handle, ptr(row_ptr), ptr(col_arg), n, int(c_sim), int(m_core),
+                                                 ptr(consider), int(current_start), int(sim_mode), ptr(labels),
+                                                 ctypes.byref(st)), "cnn_labels_from_csr")
+    except _lib.CNNError as e:
+        if e.code == _lib.CNN_ERR_INVALID and "row_ptr is not non-decreasing" in str(e):
+            raise ValueError("row_ptr must start at 0 and be non-decreasing") from None
+        raise
     return labels, st.to_dict()
 
 
@@ -426,15 +432,14 @@ def precomputed_csr(D: torch.Tensor, r: float):
     row_ptr = torch.empty(n + 1, dtype=torch.int64, device=D.device)
     nnz, asym = ctypes.c_int64(0), ctypes.c_int64(0)
     L = _lib.lib()
-    rc = L.cnn_precomputed_csr(ctx.handle, ptr(D), n, dt, float(r), ptr(row_ptr), None, 0,
-                               ctypes.byref(nnz), ctypes.byref(asym))
-    if rc == _lib.CNN_ERR_CAPACITY and nnz.value > 0:
+    h = ctypes.c_void_p()
+    ctx.check(L.cnn_precomputed_create(ctx.handle, ptr(D), n, dt, float(r), ptr(row_ptr), ctypes.byref(h),
+                                       ctypes.byref(nnz), ctypes.byref(asym)), "cnn_precomputed_csr")
+    try:
         col = torch.empty(nnz.value, dtype=torch.int32, device=D.device)
-        rc = L.cnn_precomputed_csr(ctx.handle, ptr(D), n, dt, float(r), ptr(row_ptr), ptr(col), nnz.value,
-                                   ctypes.byref(nnz), ctypes.byref(asym))
-    else:
-        col = torch.empty(0, dtype=torch.int32, device=D.device)
-    ctx.check(rc, "cnn_precomputed_csr")
+        ctx.check(L.cnn_precomputed_emit(ctx.handle, h, ptr(row_ptr), ptr(col), nnz.value), "cnn_precomputed_csr")
+    finally:
+        L.cnn_precomputed_destroy(h)
     return row_ptr, col, int(asym.value)
 
 

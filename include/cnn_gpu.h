@@ -301,6 +301,19 @@ int cnn_precomputed_csr(cnn_ctx *ctx, const void *D, int64_t n, int32_t dtype, d
                         int64_t *row_ptr, int32_t *col, int64_t col_cap, int64_t *nnz_out,
                         int64_t *asymmetric_out);
 
+/* The same in two steps that read D once, for callers that size col from the
+ * count: create thresholds D (row_ptr complete, counts on the host) and keeps
+ * the decisions in the context's working memory; emit writes the lists (stream-
+ * ordered on the context's stream; CNN_ERR_CAPACITY when col_cap < nnz).  Use and
+ * destroy the handle on the context's thread, before the context. */
+typedef struct cnn_precomputed cnn_precomputed;
+int cnn_precomputed_create(cnn_ctx *ctx, const void *D, int64_t n, int32_t dtype, double r,
+                           int64_t *row_ptr, cnn_precomputed **out, int64_t *nnz_out,
+                           int64_t *asymmetric_out);
+int cnn_precomputed_emit(cnn_ctx *ctx, const cnn_precomputed *p, const int64_t *row_ptr, int32_t *col,
+                         int64_t col_cap);
+int cnn_precomputed_destroy(cnn_precomputed *p);
+
 /* Radius graph under the periodic reduced metric, replacing
  * NeighboursGetterExtBruteForce._get (_types.pyx:1692-1710) over
  * MetricExtEuclideanPeriodicReduced._calc_distance (_types.pyx:2296-2317): per

@@ -1,0 +1,88 @@
+"""List inputs: the check of caller lists, sort_by_size through its label table
+and beyond it, and the two-step precomputed entry at the edges of its words."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle as C
+from commonnnclustering_amd import _lib, engine
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 512, 513, 1000])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_precomputed_words(cuda, n, dtype):
+    rng = np.random.default_rng(n)
+    d = rng.random((n, n)).astype(dtype)
+    d = (d + d.T) / 2
+    np.fill_diagonal(d, 0.0)
+    if n > 2:
+        d[0, 1] = np.nan       # one decision of a pair differs
+        d[1, 0] = 0.0
+    row_ptr, col, asym = engine.precomputed_csr(torch.from_numpy(d).cuda(), 0.3)
+    want = d.astype(np.float64) <= 0.3
+    assert (row_ptr.cpu().numpy() == np.concatenate([[0], np.cumsum(want.sum(1))])).all()
+    assert (col.cpu().numpy() == np.nonzero(want)[1]).all()
+    assert asym == (1 if n > 2 else 0)
+    # the one-call form, sized exactly and one entry short
+    ctx = _lib.get_context(torch.device("cuda", 0))
+    L, D = _lib.lib(), torch.from_numpy(d).cuda()
+    out = torch.full((max(len(col), 1),), -1, dtype=torch.int32, device="cuda")
+    k, a = ctypes.c_int64(), ctypes.c_int64()
+    for cap, rc in ((len(col), _lib.CNN_OK), (len(col) - 1, _lib.CNN_ERR_CAPACITY)):
+        assert L.cnn_precomputed_csr(ctx.handle, D.data_ptr(), n, _lib.dtype_code(D), 0.3, row_ptr.data_ptr(),
+                                     out.data_ptr(), cap, ctypes.byref(k), ctypes.byref(a)) == rc
+        assert k.value == len(col)
+    assert (out[:len(col)] == col).all()
+
+
+def _csr(rows):
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64)
+    return torch.from_numpy(rp).cuda(), torch.tensor([j for r in rows for j in r], dtype=torch.int32, device="cuda")
+
+
+def test_lists_are_checked(cuda):
+    long = list(range(130))
+    good = [long] + [[0, i] for i in range(1, 130)]
+    rp, col = _csr(good)
+    engine.labels_from_csr(rp, col, 2, 1)
+    for at, value in ((1, 0), (64, 63), (65, 64), (129, 130), (128, -1)):  # equal, across lanes, outside
+        bad = col.clone()
+        bad[at] = value
+        with pytest.raises(_lib.CNNError, match="ascending"):
+            engine.labels_from_csr(rp, bad, 2, 1)
+    for at, value in ((0, 1), (3, int(rp[-1]) + 1), (64, 0)):
+        bad = rp.clone()
+        bad[at] = value
+        with pytest.raises(ValueError, match="non-decreasing"):
+            engine.labels_from_csr(bad, col, 2, 1)
+    with pytest.raises(ValueError, match="exceeds"):
+        engine.labels_from_csr(rp, col[:-1], 2, 1)
+
+
+@pytest.mark.parametrize("n", [1, 64, 1000, 200_003])
+@pytest.mark.parametrize("k", [1, 1023, 1024, 1025])
+def test_sort_by_size_table_and_beyond(cuda, n, k):
+    """Labels 0 .. n, up to and above the clusters one workgroup ranks, and
+    labels outside the table (negative, above n)."""
+    rng = np.random.default_rng(n + k)
+    top = min(k, n)
+    lab = np.sort(rng.integers(0, top + 1, n)) if n > 1000 else rng.integers(0, top + 1, n)
+    for extra in (None, -3, n + 1):
+        x = lab.copy()
+        if extra is not None:
+            x[n // 2] = extra
+        for mc, mx in ((None, None), (3, None), (1, 2)):
+            want = x.copy()
+            if extra == -3:
+                # a negative label is a label like any other: ranked by size and first place
+                want[want == -3] = n + 7
+            C.sort_by_size(want, mc, mx)
+            dev = torch.from_numpy(x.copy()).cuda()
+            kept = engine.sort_by_size(dev, mc, mx)
+            assert (dev.cpu().numpy() == want).all(), (extra, mc, mx)
+            assert kept == len(set(want[want > 0].tolist()))
