@@ -639,7 +639,9 @@ __device__ __forceinline__ uint64_t word_at(const WordRow &r, int64_t t) {
 // search; rows sharing one tile list (the rows of one row tile of a spatial
 // graph) pair their words lane by lane.  Early exit once c common neighbours
 // are counted.  Wave-uniform result; every lane must call it.
-__device__ inline bool wave_sim_words(const WordRow &A, const WordRow &B, int c) {
+// keep (nullable): per column tile, the columns that count.
+__device__ inline bool wave_sim_words(const WordRow &A, const WordRow &B, int c,
+                                      const uint64_t *__restrict__ keep = nullptr) {
     if (c <= 0) return true;
     const int lane = __lane_id();
     int count = 0;
@@ -650,7 +652,9 @@ __device__ inline bool wave_sim_words(const WordRow &A, const WordRow &B, int c)
             const int64_t t = t0 + lane, t2 = t + 64;
             const int z2 = t2 < A.len ? (A.nz ? (int)A.nz[t2] : 1) : 0;
             int cnt = 0;
-            if (z) cnt = __popcll(A.word[t * (int64_t)A.stride] & B.word[t * (int64_t)B.stride]);
+            if (z)
+                cnt = __popcll(A.word[t * (int64_t)A.stride] & B.word[t * (int64_t)B.stride] &
+                               (keep ? keep[A.tile[t]] : ~0ull));
             count += wave_sum(cnt);
             if (count >= c) return true;
             z = z2;
@@ -694,7 +698,9 @@ __device__ inline bool wave_sim_words(const WordRow &A, const WordRow &B, int c)
         const int za2 = lane < va2 ? (A.nz ? (int)A.nz[ia2 + lane] : 1) : 0;
         const int zb2 = lane < vb2 ? (B.nz ? (int)B.nz[ib2 + lane] : 1) : 0;
         int cnt = 0;
-        if (hit) cnt = __popcll(A.word[pa * (int64_t)A.stride] & B.word[pb * (int64_t)B.stride]);
+        if (hit)
+            cnt = __popcll(A.word[pa * (int64_t)A.stride] & B.word[pb * (int64_t)B.stride] &
+                           (keep ? keep[tb] : ~0ull));
         count += wave_sum(cnt);
         if (count >= c) return true;
         ia = ia2;

@@ -123,3 +123,18 @@ def test_clustering_predict_frozen_labels_accumulate(cuda):
     ref.predict(other, 0.6, 3, clusters={2}, purge=True)
     want3, _ = O.predict_firstmatch(X, labels, Y, 0.6, 3, clusters={2})
     assert (other.labels == want3).all()
+
+
+# n = 129 and 2048 are where the graphs start to hold words in d = 2 and 16
+@pytest.mark.parametrize("d,n_x,n_y", [(2, 100, 20), (2, 128, 1), (2, 300, 65), (3, 63, 1000), (16, 2000, 47),
+                                       (16, 2000, 48), (16, 2100, 63)])
+def test_predict_on_words_and_lists(cuda, d, n_x, n_y):
+    X, Y = _split(n_x, n_y, d, n_x + n_y)
+    r, c = {2: 0.9, 3: 1.4, 16: 3.8}[d], 2
+    labels_x, _ = O.fit(X, r, c, member_cutoff=3)
+    want_l, want_c = O.predict_firstmatch(X, labels_x, Y, r, c)
+    lx = torch.from_numpy(labels_x).cuda()
+    lab, con, _ = engine.predict(torch.from_numpy(X).cuda(), lx, torch.from_numpy(Y).cuda(), r * r, c + 2, c + 1,
+                                 set(labels_x.tolist()) - {0})
+    assert (lab.cpu().numpy() == want_l).all()
+    assert (con.cpu().numpy() == want_c).all()
