@@ -206,18 +206,16 @@ void scan_free(cnn_scan *sc) {
     if (sc->graph) (void)hipGraphDestroy(sc->graph);
     for (auto &e : sc->ev)
         if (e) (void)hipEventDestroy(e);
-    for (void *p : sc->bufs) (void)hipFree(p);
+    if (!sc->bufs.empty()) (void)hipDeviceSynchronize();
+    for (void *p : sc->bufs) pool_free(sc->device, p, true);
     delete sc;
 }
 
 template <typename T>
 T *scan_alloc(cnn_scan *sc, int64_t count) {
-    void *p = nullptr;
     const size_t bytes = (size_t)std::max<int64_t>(count, 1) * sizeof(T);
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        throw OutOfMemory{"scan buffer of " + std::to_string(bytes) + " bytes"};
-    }
+    void *p = pool_alloc(sc->device, bytes);
+    if (!p) throw OutOfMemory{"scan buffer of " + std::to_string(bytes) + " bytes"};
     sc->bufs.push_back(p);
     return (T *)p;
 }

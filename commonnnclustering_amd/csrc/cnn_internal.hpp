@@ -55,6 +55,20 @@ private:
     int64_t total_ = 0;
 };
 
+// Device memory of objects that outlive a call (resident graphs, recorded
+// scans).  A freed block waits in a pool of its device for the next object:
+// hipMalloc and hipFree of a graph's words (230 MB) take 85 and 280 us here.
+// The pool is shared by all threads, holds at most kPoolBytes in kPoolBlocks
+// blocks (the oldest are freed first), and is given back by cnn_ctx_trim, when
+// an allocation fails and with the device's last context.  pool_free waits for
+// the device before a block becomes available, as hipFree does, so a block may
+// be reused on any stream; `waited`: the caller has done so.
+constexpr size_t kPoolBytes = (size_t)1 << 30;
+constexpr size_t kPoolBlocks = 64;
+void *pool_alloc(int device, size_t bytes);  // nullptr: out of memory
+void pool_free(int device, void *p, bool waited = false);
+void pool_trim(int device);
+
 // A fixed device buffer handed out front to back (entry points that may not
 // allocate).  Blocks are 256-byte aligned; releasing the most recent block
 // makes its bytes available again (Scratch buffers die in reverse order).
@@ -116,12 +130,17 @@ struct cnn_graph {
     // pairs tp_ptr[R] .. tp_ptr[R+1]), mask[64k + r] holds row 64R+r's bits over
     // the 64 points of column tile tp_col[k], valid where pair_nz[k] != 0
     uint64_t *mask = nullptr;
-    uint8_t *pair_nz = nullptr;
+    uint8_t *pair_nz = nullptr;  // in mask's allocation, behind the words
     int64_t n_tile_pairs = 0;
     int32_t *diag = nullptr;     // spatial layout: per row tile, its own pair's place in its list (nullable)
     // spatial one-batch builds: the row tiles, heavy ones first (nullable)
     int32_t *tile_order = nullptr;
     int64_t bytes = 0;
+    // resident graphs: one allocation that holds the arrays whose sizes are known
+    // before the build (graph_reserve)
+    char *slab = nullptr;
+    size_t slab_size = 0, slab_used = 0;
+    double max_norm2 = -1.0;     // largest squared norm of the points (-1: not computed)
     cnn_graph_stats stats{};
     cnn::TuneParams tune{};      // launch shapes of the graph's class
     // a graph that keeps its words emits its lists (col, selfpos) only when a

@@ -3168,26 +3168,58 @@ static void launch_dist(cnn_ctx *ctx, const DistArgs &a, int64_t n_rt, bool band
 
 // Graph memory: from the building context's arena for a graph that lives only
 // inside one call on that context (stream-ordered reuse, no hipMalloc/hipFree
-// per fit), else hipMalloc.
+// per fit), else from the device's pool.
 static void *graph_mem(cnn_graph *g, size_t bytes) {
     void *p = nullptr;
+    const size_t rounded = (bytes + 255) & ~(size_t)255;
     if (g->arena) {
         p = g->arena->get(bytes);
+    } else if (g->slab && rounded <= g->slab_size - g->slab_used) {
+        p = g->slab + g->slab_used;
+        g->slab_used += rounded;
     } else {
-        hipError_t e = hipMalloc(&p, bytes);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            p = nullptr;
-        }
+        p = pool_alloc(g->device, bytes);
     }
     if (!p) throw OutOfMemory{"graph allocation of " + std::to_string(bytes) + " bytes failed"};
     return p;
 }
 
-static void graph_mem_free(cnn_graph *g, void *p) {
+// waited: nothing on the device uses the memory any more.
+static void graph_mem_free(cnn_graph *g, void *p, bool waited = false) {
     if (!p) return;
     if (g->arena) g->arena->put(p);
-    else (void)hipFree(p);
+    else if (!g->slab || (char *)p < g->slab || (char *)p >= g->slab + g->slab_size) pool_free(g->device, p, waited);
+}
+
+// One allocation for a resident graph's arrays of known size (offsets, order,
+// coordinates, per-tile arrays).  Without it (no memory in one piece) they are
+// allocated one by one.
+static void graph_reserve(cnn_graph *g) {
+    if (g->arena || g->n == 0) return;
+    const size_t n = (size_t)g->n, T = (size_t)g->n_tiles, d = (size_t)std::max(g->d, 1), rows = T * 64;
+    size_t total = 0;
+    for (size_t b : {(n + 1) * sizeof(int64_t), n * sizeof(int32_t), rows * d * sizeof(double),
+                     g->precision == CNN_F32_BAND ? rows * d * sizeof(float) : size_t(0), (T + 1) * sizeof(int64_t),
+                     T * sizeof(int32_t), T * sizeof(int32_t)})
+        total += (b + 255) & ~(size_t)255;
+    g->slab = (char *)pool_alloc(g->device, total);
+    g->slab_size = g->slab ? total : 0;
+}
+
+// The words of `pairs` tile pairs and their flags, in one allocation.
+static void words_alloc(cnn_graph *g, int64_t pairs) {
+    const int64_t count = std::max<int64_t>(pairs, 1);
+    const size_t bytes = (size_t)count * (64 * sizeof(uint64_t) + 1);
+    g->mask = (uint64_t *)graph_mem(g, bytes);
+    g->pair_nz = (uint8_t *)(g->mask + count * 64);
+    g->bytes += (int64_t)bytes;
+}
+
+static void words_free(cnn_graph *g, int64_t pairs) {
+    graph_mem_free(g, g->mask);
+    g->bytes -= std::max<int64_t>(pairs, 1) * (int64_t)(64 * sizeof(uint64_t) + 1);
+    g->mask = nullptr;
+    g->pair_nz = nullptr;
 }
 
 template <typename T>
@@ -3201,19 +3233,12 @@ static T *dev_alloc(cnn_graph *g, int64_t count) {
 void graph_free(cnn_graph *g) {
     if (!g) return;
     (void)hipSetDevice(g->device);
-    graph_mem_free(g, g->perm);
-    graph_mem_free(g, g->xw64);
-    graph_mem_free(g, g->xw32);
-    graph_mem_free(g, g->row_ptr);
-    graph_mem_free(g, g->col);
-    graph_mem_free(g, g->tp_ptr);
-    graph_mem_free(g, g->tp_col);
-    graph_mem_free(g, g->diag);
-    graph_mem_free(g, g->tile_order);
-    graph_mem_free(g, g->selfpos);
-    graph_mem_free(g, g->mask);
-    graph_mem_free(g, g->pair_nz);
-    graph_mem_free(g, g->bounds);
+    if (!g->arena) (void)hipDeviceSynchronize();  // as hipFree: no kernel reads the graph any more
+    for (void *p : {(void *)g->perm, (void *)g->xw64, (void *)g->xw32, (void *)g->row_ptr, (void *)g->col,
+                    (void *)g->tp_ptr, (void *)g->tp_col, (void *)g->diag, (void *)g->tile_order, (void *)g->selfpos,
+                    (void *)g->mask, (void *)g->bounds})
+        graph_mem_free(g, p, true);
+    pool_free(g->device, g->slab, true);
     delete g;
 }
 
@@ -3532,8 +3557,9 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
     std::unique_ptr<Scratch<uint64_t>> mask_s;
     std::unique_ptr<Scratch<uint8_t>> pair_nz_s;
     if (sym && tp_ptr) {
-        mask_p = g->mask = dev_alloc<uint64_t>(g, std::max<int64_t>(max_batch_pairs, 1) * 64);
-        pair_nz_p = g->pair_nz = dev_alloc<uint8_t>(g, std::max<int64_t>(max_batch_pairs, 1));
+        words_alloc(g, max_batch_pairs);
+        mask_p = g->mask;
+        pair_nz_p = g->pair_nz;
     } else {
         mask_s.reset(new Scratch<uint64_t>(ctx, std::max<int64_t>(max_batch_pairs, 1) * 64));
         pair_nz_s.reset(new Scratch<uint8_t>(ctx, std::max<int64_t>(max_batch_pairs, 1)));
@@ -3684,12 +3710,7 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
     }
     if (!words_only && g->mask) {
         // the lists are the smaller form: drop the words
-        graph_mem_free(g, g->mask);
-        graph_mem_free(g, g->pair_nz);
-        g->bytes -= std::max<int64_t>(max_batch_pairs, 1) * 64 * (int64_t)sizeof(uint64_t) +
-                    std::max<int64_t>(max_batch_pairs, 1);
-        g->mask = nullptr;
-        g->pair_nz = nullptr;
+        words_free(g, max_batch_pairs);
     }
     if (!words_deferred) set_i64(ctx, g->row_ptr + n, nnz_total);
     PinnedReads rd(ctx);
@@ -3727,12 +3748,7 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
     if (words_deferred && !keeps_words(g, total_pairs, nnz_total)) {
         // the lists are the smaller form: emit them from the words, then drop the words
         graph_lists(ctx, g);
-        graph_mem_free(g, g->mask);
-        graph_mem_free(g, g->pair_nz);
-        g->bytes -= std::max<int64_t>(max_batch_pairs, 1) * 64 * (int64_t)sizeof(uint64_t) +
-                    std::max<int64_t>(max_batch_pairs, 1);
-        g->mask = nullptr;
-        g->pair_nz = nullptr;
+        words_free(g, max_batch_pairs);
     }
 }
 
@@ -3767,6 +3783,7 @@ cnn_graph *graph_build(cnn_ctx *ctx, const void *X, int64_t n, int32_t d, int32_
     const bool band = precision == CNN_F32_BAND;
 
     CNN_HIP(hipEventRecord(ctx->ev[0], s));
+    graph_reserve(g);
     g->row_ptr = dev_alloc<int64_t>(g, n + 1);
     if (n == 0) {
         fill_i64(ctx, g->row_ptr, 0, 1);
@@ -3788,7 +3805,10 @@ cnn_graph *graph_build(cnn_ctx *ctx, const void *X, int64_t n, int32_t d, int32_
     // norm); the plain FP64 and MFMA forms of the dense layout need neither
     std::vector<double> lo, hi;
     double max_norm2 = 0.0;
-    if (g->layout == 1 || (band && d < kMfmaMinD)) bbox(ctx, X, n, d, dtype, lo, hi, max_norm2);
+    if (g->layout == 1 || (band && d < kMfmaMinD)) {
+        bbox(ctx, X, n, d, dtype, lo, hi, max_norm2);
+        g->max_norm2 = max_norm2;
+    }
     if (g->layout == 1) {
         const KeySpec ks = make_keyspec(d, lo, hi, 64, n);
         g->perm = dev_alloc<int32_t>(g, n);
@@ -4153,6 +4173,7 @@ static cnn_graph *graph_rebuild(cnn_ctx *ctx, const cnn_graph *src, double r2, i
     const int d = g->d;
     const bool band = precision == CNN_F32_BAND;
     CNN_HIP(hipEventRecord(ctx->ev[0], s));
+    graph_reserve(g);
     g->row_ptr = dev_alloc<int64_t>(g, n + 1);
     if (src->perm) {
         g->perm = dev_alloc<int32_t>(g, n);
@@ -4175,10 +4196,12 @@ static cnn_graph *graph_rebuild(cnn_ctx *ctx, const cnn_graph *src, double r2, i
         }
     }
     g->dp = d;
-    std::vector<double> lo, hi;
-    double max_norm2 = 0.0;
-    if (band && d < kMfmaMinD) bbox(ctx, g->xw64, n, d, CNN_F64, lo, hi, max_norm2);
-    build_pairs_and_csr(ctx, g, band, g->dtype, max_norm2, nullptr, nullptr);
+    g->max_norm2 = src->max_norm2;
+    if (band && d < kMfmaMinD && g->max_norm2 < 0.0) {
+        std::vector<double> lo, hi;
+        bbox(ctx, g->xw64, n, d, CNN_F64, lo, hi, g->max_norm2);
+    }
+    build_pairs_and_csr(ctx, g, band, g->dtype, std::max(g->max_norm2, 0.0), nullptr, nullptr);
     return std::exchange(guard.g, nullptr);
 }
 
@@ -4202,8 +4225,10 @@ cnn_graph *graph_rethreshold(cnn_ctx *ctx, const cnn_graph *src, double r2, int3
     g->layout = src->layout;
     g->n_tiles = src->n_tiles;
     g->tune = src->tune;
+    g->max_norm2 = src->max_norm2;
     const int64_t n = g->n, n_pad = g->n_tiles * 64;
     const int dd = std::max(g->d, 1);
+    graph_reserve(g);
     g->row_ptr = dev_alloc<int64_t>(g, n + 1);
     if (src->perm) {
         g->perm = dev_alloc<int32_t>(g, n);

@@ -7,6 +7,8 @@
 #include <rocprim/iterator/transform_iterator.hpp>
 
 #include <algorithm>
+#include <mutex>
+#include <unordered_map>
 
 #include "cnn_internal.hpp"
 
@@ -39,6 +41,7 @@ void *Arena::get(size_t bytes) {
                 ++i;
             }
         }
+        pool_trim(device_);
         e = hipMalloc(&p, bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -65,6 +68,98 @@ void Arena::trim() {
             ++i;
         }
     }
+}
+
+// ------------------------------------------------------------------ device pool
+namespace {
+
+struct PoolBlock {
+    void *p;
+    size_t size;
+};
+struct DevicePool {
+    std::vector<PoolBlock> free;                  // oldest first
+    std::unordered_map<void *, size_t> in_use;    // sizes of the blocks handed out
+    size_t free_bytes = 0;
+    int contexts = 0;
+};
+std::mutex pool_mu;
+std::unordered_map<int, DevicePool> pools;
+
+// (pool_mu held)
+void pool_drop(DevicePool &d, size_t at) {
+    (void)hipFree(d.free[at].p);
+    d.free_bytes -= d.free[at].size;
+    d.free.erase(d.free.begin() + (std::ptrdiff_t)at);
+}
+
+}  // namespace
+
+void *pool_alloc(int device, size_t bytes) {
+    bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+    {
+        std::lock_guard<std::mutex> lock(pool_mu);
+        DevicePool &d = pools[device];
+        int best = -1;  // the smallest block that wastes at most a quarter (or 64 KiB)
+        for (size_t i = 0; i < d.free.size(); ++i) {
+            const size_t sz = d.free[i].size;
+            if (sz >= bytes && sz <= bytes + bytes / 4 + ((size_t)64 << 10) && (best < 0 || sz < d.free[best].size))
+                best = (int)i;
+        }
+        if (best >= 0) {
+            const PoolBlock b = d.free[best];
+            d.free_bytes -= b.size;
+            d.free.erase(d.free.begin() + best);
+            d.in_use[b.p] = b.size;
+            return b.p;
+        }
+    }
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        pool_trim(device);
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
+    std::lock_guard<std::mutex> lock(pool_mu);
+    pools[device].in_use[p] = bytes;
+    return p;
+}
+
+void pool_free(int device, void *p, bool waited) {
+    if (!p) return;
+    if (!waited) (void)hipDeviceSynchronize();
+    std::lock_guard<std::mutex> lock(pool_mu);
+    DevicePool &d = pools[device];
+    auto it = d.in_use.find(p);
+    const size_t size = it == d.in_use.end() ? 0 : it->second;
+    if (it != d.in_use.end()) d.in_use.erase(it);
+    if (size == 0 || size > kPoolBytes || d.contexts == 0) {
+        (void)hipFree(p);
+        return;
+    }
+    while (!d.free.empty() && (d.free_bytes + size > kPoolBytes || d.free.size() >= kPoolBlocks)) pool_drop(d, 0);
+    d.free.push_back({p, size});
+    d.free_bytes += size;
+}
+
+void pool_trim(int device) {
+    std::lock_guard<std::mutex> lock(pool_mu);
+    DevicePool &d = pools[device];
+    while (!d.free.empty()) pool_drop(d, d.free.size() - 1);
+}
+
+static void pool_contexts(int device, int change) {
+    bool last = false;
+    {
+        std::lock_guard<std::mutex> lock(pool_mu);
+        DevicePool &d = pools[device];
+        d.contexts += change;
+        last = d.contexts == 0;
+    }
+    if (last) pool_trim(device);
 }
 
 // ------------------------------------------------------------------ fills
@@ -223,6 +318,7 @@ int cnn_ctx_create(int device, cnn_ctx **out) {
         ctx->arena = new Arena(device);
         CNN_HIP(hipHostMalloc((void **)&ctx->pinned, cnn_ctx::kPinnedBytes, hipHostMallocDefault));
         noalloc_setup(device);
+        pool_contexts(device, 1);
         return (int)CNN_OK;
     });
     if (rc != CNN_OK) {
@@ -246,6 +342,7 @@ int cnn_ctx_destroy(cnn_ctx *ctx) {
     for (auto &e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
+    pool_contexts(ctx->device, -1);
     delete ctx;
     return CNN_OK;
 }
@@ -283,6 +380,7 @@ int cnn_ctx_trim(cnn_ctx *ctx) {
         CNN_HIP(hipSetDevice(ctx->device));
         CNN_HIP(hipStreamSynchronize(ctx->stream));
         ctx->arena->trim();
+        pool_trim(ctx->device);
         return (int)CNN_OK;
     });
 }

@@ -139,7 +139,8 @@ void *cnn_ctx_get_stream(cnn_ctx *ctx);
 int cnn_ctx_synchronize(cnn_ctx *ctx);
 /* Device bytes currently held by the context's workspace arena. */
 int cnn_ctx_workspace_bytes(const cnn_ctx *ctx, int64_t *bytes);
-/* Release the workspace arena (kept between calls otherwise). */
+/* Release the workspace arena and the device's pool of freed graph memory (kept
+ * between calls otherwise; the pool holds at most 1 GiB). */
 int cnn_ctx_trim(cnn_ctx *ctx);
 
 /* ------------------------------------------------------------------ phase N */
