@@ -181,7 +181,14 @@ struct ComponentArrays {
 };
 
 __global__ void k_init(LabelArgs a, const uint8_t *__restrict__ consider, const int32_t *__restrict__ perm,
-                       ComponentArrays ca) {
+                       ComponentArrays ca, ClearList clear) {
+    if (blockIdx.y == 0) {
+        const int64_t step = (int64_t)gridDim.x * blockDim.x;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < clear.count[q]; t += step)
+                clear.p[q][t] = 0ull;
+    }
     a = slice(a);
     int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= a.n) return;
@@ -1578,12 +1585,11 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
     Scratch<uint8_t> core(ctx, n);
     Scratch<uint64_t> rank(ctx, n);
     Scratch<int> parent(ctx, n);
-    // the pass's small counters in one buffer, zeroed by one fill kernel:
+    // the pass's small counters in one buffer, zeroed by k_init:
     // counters (8), striped test statistics (4 per slot), the hook and the round
     // queue length, then one root count per root hooking pass
     const int64_t kSmallSlots = 8 + 4 * kStatSlots + 2 + std::max(req.root_passes, 0);
     Scratch<unsigned long long> small(ctx, kSmallSlots);
-    fill_u64(ctx, small.p, 0ull, kSmallSlots);
     unsigned long long *const counters_p = small.p, *const tstats_p = small.p + 8;
     unsigned long long *const slot_p = small.p + 8 + 4 * kStatSlots;
     LabelArgs a{req.row_ptr, req.col, n, req.c_sim, req.m_core, core.p, parent.p, tstats_p, rank.p, nullptr,
@@ -1652,7 +1658,8 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
     if (req.sort) snewlab.reset(new Scratch<int32_t>(ctx, n));
     std::unique_ptr<Scratch<int32_t>> cnt(new Scratch<int32_t>(ctx, n));  // until the snapshot
     k_init<<<blocks_for(n), 256, 0, s>>>(a, req.consider, req.perm,
-                                         ComponentArrays{cnt->p, cmin.p, csize.p, req.sort ? snewlab->p : nullptr});
+                                         ComponentArrays{cnt->p, cmin.p, csize.p, req.sort ? snewlab->p : nullptr},
+                                         ClearList{{small.p}, {kSmallSlots}});
     CNN_HIP(hipGetLastError());
     CNN_HIP(hipEventRecord(ctx->ev[8], s));
     if (words && a.mask) {
@@ -1918,10 +1925,6 @@ void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabe
     const int64_t n = b.n, T = b.n_tiles;
     const unsigned nc = (unsigned)b.n_c;
     if (n == 0 || nc == 0) return;
-    fill_u64(ctx, counters, 0, 8 * (int64_t)nc);
-    fill_u64(ctx, b.rq_len, 0, nc);
-    fill_u64(ctx, tstats, 0, 4 * (int64_t)kStatSlots * nc);
-    fill_i32(ctx, (int32_t *)b.lens, 0, 2 * (int64_t)nc);
     unsigned int *const hq_len = b.lens, *const ccount = b.lens + nc;
     LabelArgs a{};
     a.n = n;
@@ -1939,7 +1942,10 @@ void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabe
     a.tiles = T;
     auto g2 = [&](int64_t items, int per) { return dim3(blocks_for(items, per), nc); };
     const unsigned waves = (unsigned)std::min<int64_t>(blocks_for(n, 4), 4096);
-    k_init<<<g2(n, 256), 256, 0, s>>>(a, nullptr, src.perm, ComponentArrays{b.cnt, b.cmin, b.csize, b.newlab});
+    k_init<<<g2(n, 256), 256, 0, s>>>(a, nullptr, src.perm, ComponentArrays{b.cnt, b.cmin, b.csize, b.newlab},
+                                         ClearList{{counters, b.rq_len, tstats, (unsigned long long *)b.lens},
+                                                   {8 * (int64_t)nc, (int64_t)nc, 4 * (int64_t)kStatSlots * nc,
+                                                    (int64_t)nc}});
     k_hook_tile<<<g2(T, 4), 256, 0, s>>>(a, T, b.hq, hq_len);
     k_hook_queue<<<dim3(waves, nc), 256, 0, s>>>(a, b.hq, hq_len, 2);
     CNN_HIP(hipGetLastError());

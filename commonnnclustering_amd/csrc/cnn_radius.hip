@@ -3011,7 +3011,18 @@ __global__ void k_set_last(int64_t *p, int64_t idx, const int64_t *prev_excl, co
 }
 
 // p[idx] = p[idx - 1] + cnt[idx - 1]: the total after an exclusive scan of counts.
-__global__ void k_scan_total(int64_t *p, int64_t idx, const int32_t *cnt) { p[idx] = p[idx - 1] + cnt[idx - 1]; }
+
+// The build's arrays that start from a constant, in one launch (each nullable).
+__global__ void k_clear_build(int32_t *deg, int64_t n_deg, int32_t *diag, int64_t n_diag, unsigned long long *rows,
+                              int64_t n_rows, unsigned long long *stats, int n_stats) {
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (int64_t t = t0; t < n_deg; t += step) deg[t] = 0;
+    if (diag)
+        for (int64_t t = t0; t < n_diag; t += step) diag[t] = -1;
+    if (rows)
+        for (int64_t t = t0; t < n_rows; t += step) rows[t] = 0ull;
+    for (int64_t t = t0; t < n_stats; t += step) stats[t] = 0ull;
+}
 
 // ------------------------------------------------------------------ host side
 
@@ -3378,6 +3389,22 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
     if (const char *ev = std::getenv("CNN_HIP_MASK_BUDGET")) mask_budget = std::max<int64_t>(512, std::atoll(ev));
     const int64_t max_pairs_per_batch = std::max<int64_t>(mask_budget / 512, T);
 
+    // per-row degrees (one more entry than rows: the offsets' scan covers it, so
+    // that it ends with the total), band statistics, live pair counts, per-tile
+    // rows to evaluate: cleared together
+    Scratch<int32_t> deg(ctx, n + 1);
+    Scratch<unsigned long long> bstats(ctx, 6);
+    unsigned long long *const lcnt = bstats.p + 4;
+    std::unique_ptr<Scratch<unsigned long long>> rows_part;
+    if (g->layout == 1) {
+        rows_part.reset(new Scratch<unsigned long long>(ctx, 2 * T));
+        // kept with the graph: the label pass's tile hooking starts at it
+        g->diag = dev_alloc<int32_t>(g, T);
+    }
+    k_clear_build<<<(unsigned)std::min<int64_t>(ceil_div(n + 1, 256), 2048), 256, 0, s>>>(
+        deg.p, n + 1, g->layout == 1 ? g->diag : nullptr, T, rows_part ? rows_part->p : nullptr, 2 * T, bstats.p, 6);
+    CNN_HIP(hipGetLastError());
+
     // candidate tile pairs
     int64_t *tp_ptr = nullptr;
     int32_t *tp_col = nullptr;
@@ -3398,14 +3425,12 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
         Scratch<double> slo(ctx, NS * d), shi(ctx, NS * d);
         k_super_boxes<<<(unsigned)ceil_div(NS, 4), 256, 0, s>>>(blo.p, bhi.p, d, T, NS, slo.p, shi.p);
         CNN_HIP(hipGetLastError());
-        Scratch<int32_t> cnt(ctx, T);
+        Scratch<int32_t> cnt(ctx, T + 1);
         const double *tthr = pk ? pk->tile_thr : nullptr;
         const int32_t *sl = pk ? pk->seg_lo : nullptr, *sh = pk ? pk->seg_hi : nullptr;
         // one search: counts and lists (in per-tile buckets), then the lists
         // move to their places once the counts are scanned
-        // kept with the graph: the label pass's tile hooking starts at it
-        int32_t *diag = g->diag = dev_alloc<int32_t>(g, T);
-        fill_i32(ctx, diag, -1, T);
+        int32_t *const diag = g->diag;
         {
             int B = (int)std::max<int64_t>(
                 16, std::min<int64_t>(kPairBucketMax, kPairBucketBytes / (4 * std::max<int64_t>(T, 1))));
@@ -3415,8 +3440,7 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
                                                                   sl, sh, cnt.p, bucket.p, B, diag);
             CNN_HIP(hipGetLastError());
             tp_ptr = g->tp_ptr = dev_alloc<int64_t>(g, T + 1);
-            exclusive_scan_i32_to_i64(ctx, cnt.p, tp_ptr, T);
-            k_scan_total<<<1, 1, 0, s>>>(tp_ptr, T, cnt.p);
+            exclusive_scan_i32_to_i64(ctx, cnt.p, tp_ptr, T + 1);
             total_pairs = read_scalar(ctx, tp_ptr + T);
             tp_col = g->tp_col = dev_alloc<int32_t>(g, total_pairs);
             k_tile_pairs_place<<<(unsigned)ceil_div(T, 4), 256, 0, s>>>(blo.p, bhi.p, slo.p, shi.p, d, T, NS, thr,
@@ -3426,9 +3450,7 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
         }
         gmask.reset(new Scratch<GroupMask>(ctx, std::max<int64_t>(total_pairs, 1)));
         mirror.reset(new Scratch<int64_t>(ctx, std::max<int64_t>(total_pairs, 1)));
-        Scratch<unsigned long long> rows_part(ctx, 2 * T);
         rows_eval.reset(new Scratch<unsigned long long>(ctx, 2));
-        fill_u64(ctx, rows_part.p, 0ull, 2 * T);
         if (total_pairs <= max_pairs_per_batch) {
             // one-sided: chunks of kPairChunk pairs from each row tile's own pair on
             Scratch<int32_t> ccnt(ctx, T);
@@ -3438,24 +3460,28 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
             exclusive_scan_i32_to_i64(ctx, ccnt.p, coff.p, T);
             const int64_t waves = T + total_pairs / kPairChunk + 1;  // bounds the chunks
             k_pair_info<<<(unsigned)ceil_div(waves, 4), 256, 0, s>>>(tp_ptr, tp_col, T, mirror->p, glo->p, ghi->p,
-                                                                   blo.p, bhi.p, d, thr, tthr, gmask->p, rows_part.p,
+                                                                   blo.p, bhi.p, d, thr, tthr, gmask->p, rows_part->p,
                                                                    diag, 1, coff.p, ccnt.p);
         } else {
             k_pair_info<<<(unsigned)ceil_div(2 * T, 4), 256, 0, s>>>(tp_ptr, tp_col, T, mirror->p, glo->p, ghi->p,
-                                                                   blo.p, bhi.p, d, thr, tthr, gmask->p, rows_part.p,
+                                                                   blo.p, bhi.p, d, thr, tthr, gmask->p, rows_part->p,
                                                                    diag, 0, nullptr, nullptr);
         }
         CNN_HIP(hipGetLastError());
-        k_sum_pairs_u64<<<1, 256, 0, s>>>(rows_part.p, T, rows_eval->p);
+        k_sum_pairs_u64<<<1, 256, 0, s>>>(rows_part->p, T, rows_eval->p);
         CNN_HIP(hipGetLastError());
-        if (total_pairs <= max_pairs_per_batch) {
-            // kept with the graph: the label pass's per-tile kernels take the same order
+        // kept with the graph: the label pass's per-tile kernels take the same order.
+        // Up to kOrderMinT tiles all workgroups are resident at once and the order
+        // changes nothing (its three launches cost 35 of 470 us at n = 3e4, d = 3)
+        constexpr int64_t kOrderMinT = 1024;
+        if (total_pairs <= max_pairs_per_batch && T > kOrderMinT) {
             g->tile_order = dev_alloc<int32_t>(g, T);
             Scratch<uint32_t> okey(ctx, T);
-            k_row_order_keys<<<(unsigned)ceil_div(T, 256), 256, 0, s>>>(rows_part.p, T, okey.p, g->tile_order,
+            Scratch<int32_t> iota(ctx, T);
+            k_row_order_keys<<<(unsigned)ceil_div(T, 256), 256, 0, s>>>(rows_part->p, T, okey.p, iota.p,
                                                                        rows_eval->p);
             CNN_HIP(hipGetLastError());
-            sort_pairs_u32_i32(ctx, okey.p, g->tile_order, T, 32);
+            sort_pairs_u32_i32(ctx, okey.p, iota.p, g->tile_order, T, 32);
         }
     }
     // dense layout in nearest-pivot order: tile pairs out of reach by the pivot
@@ -3473,18 +3499,16 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
         CNN_HIP(hipGetLastError());
         live_words = ceil_div(T, 64);
         live.reset(new Scratch<uint64_t>(ctx, T * live_words));
-        Scratch<unsigned long long> lcnt(ctx, 2);
-        fill_u64(ctx, lcnt.p, 0ull, 2);
         const double rr = std::sqrt(g->r2) * (1.0 + 1e-6);
         float rc = (float)rr;
         if ((double)rc < rr) rc = std::nextafter(rc, INFINITY);
         k_dense_live<<<(unsigned)std::min<int64_t>(ceil_div(T * live_words, 4), 2048), 256, 0, s>>>(
-            bnd.p, home.p, T, live_words, rc, live->p, lcnt.p);
+            bnd.p, home.p, T, live_words, rc, live->p, lcnt);
         k_live_mirror<<<(unsigned)ceil_div(live_words * live_words, 4), 256, 0, s>>>(live->p, T, live_words);
         CNN_HIP(hipGetLastError());
         {
             PinnedReads rd(ctx);
-            const unsigned long long *lc = rd.get(lcnt.p, 2);
+            const unsigned long long *lc = rd.get(lcnt, 2);
             rd.wait();
             live_count[1] = lc[1];
             live_count[0] = 2 * lc[1] - (unsigned long long)T;  // the diagonal pairs are live and counted once
@@ -3493,12 +3517,11 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
         // words of culled pairs are never stored, and the label pass can test
         // similarities on the words as for the spatial layout
         live_pre.reset(new Scratch<int32_t>(ctx, T * live_words));
-        Scratch<int32_t> cnt(ctx, T);
+        Scratch<int32_t> cnt(ctx, T + 1);
         k_live_rows<<<(unsigned)ceil_div(T, 4), 256, 0, s>>>(live->p, T, live_words, live_pre->p, cnt.p);
         CNN_HIP(hipGetLastError());
         tp_ptr = g->tp_ptr = dev_alloc<int64_t>(g, T + 1);
-        exclusive_scan_i32_to_i64(ctx, cnt.p, tp_ptr, T);
-        k_scan_total<<<1, 1, 0, s>>>(tp_ptr, T, cnt.p);
+        exclusive_scan_i32_to_i64(ctx, cnt.p, tp_ptr, T + 1);
         total_pairs = (int64_t)live_count[0];
         tp_col = g->tp_col = dev_alloc<int32_t>(g, std::max<int64_t>(total_pairs, 1));
         mirror.reset(new Scratch<int64_t>(ctx, std::max<int64_t>(total_pairs, 1)));
@@ -3533,9 +3556,6 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
         bp.lo = 0.0f;
         bp.hi = 0.0f;
     }
-    Scratch<unsigned long long> bstats(ctx, 4);
-    fill_u64(ctx, bstats.p, 0ull, 4);
-    Scratch<int32_t> deg(ctx, n);
 
     std::vector<std::pair<int64_t, int64_t>> batches;
     if (one_batch) batches.push_back({0, T});
@@ -3633,7 +3653,7 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
             a.tile_hi = pk->tile_hi;
             a.tile_valid = pk->tile_valid;
         }
-        fill_i32(ctx, deg.p, 0, n);
+        if (b.first > 0) fill_i32(ctx, deg.p, 0, n);
         CNN_HIP(hipEventRecord(ctx->ev[2], s));
         launch_dist(ctx, a, b.second - b.first, band, pair_begin(b.second) - pair_begin(b.first),
                     g->tune.mfma_col_chunk);
@@ -3641,14 +3661,12 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
         // row_ptr for this batch's rows: exclusive scan + running offset
         const int64_t row_lo = b.first * 64, row_hi = std::min<int64_t>(b.second * 64, n);
         const int64_t rows = row_hi - row_lo;
-        exclusive_scan_i32_to_i64(ctx, deg.p + row_lo, g->row_ptr + row_lo, rows);
+        // (one batch: up to and with row_ptr[n])
+        exclusive_scan_i32_to_i64(ctx, deg.p + row_lo, g->row_ptr + row_lo, words_deferred ? rows + 1 : rows);
         if (words_deferred) {
-            // one batch that may keep its words: row_ptr[n] is completed on the
-            // device and the entry count read with the final statistics (no
-            // synchronisation here); the lists are emitted after it only if
-            // they are the smaller form
-            k_scan_total<<<1, 1, 0, s>>>(g->row_ptr, n, deg.p);
-            CNN_HIP(hipGetLastError());
+            // one batch that may keep its words: the entry count is read with the
+            // final statistics (no synchronisation here); the lists are emitted
+            // after it only if they are the smaller form
             words_only = true;
             emitted = false;
             continue;
@@ -3817,12 +3835,13 @@ cnn_graph *graph_build(cnn_ctx *ctx, const void *X, int64_t n, int32_t d, int32_
         if (key_bits <= 32) {
             // 32-bit keys: half the key traffic, and the sort's 32-bit configuration
             Scratch<uint32_t> keys(ctx, n);
+            Scratch<int32_t> iota(ctx, n);
             if (dtype == CNN_F32)
-                k_curve_keys<float, uint32_t><<<blocks, 256, 0, s>>>((const float *)X, n, d, ks, keys.p, g->perm);
+                k_curve_keys<float, uint32_t><<<blocks, 256, 0, s>>>((const float *)X, n, d, ks, keys.p, iota.p);
             else
-                k_curve_keys<double, uint32_t><<<blocks, 256, 0, s>>>((const double *)X, n, d, ks, keys.p, g->perm);
+                k_curve_keys<double, uint32_t><<<blocks, 256, 0, s>>>((const double *)X, n, d, ks, keys.p, iota.p);
             CNN_HIP(hipGetLastError());
-            sort_pairs_u32_i32(ctx, keys.p, g->perm, n, key_bits);
+            sort_pairs_u32_i32(ctx, keys.p, iota.p, g->perm, n, key_bits);
         } else {
             Scratch<uint64_t> keys(ctx, n);
             if (dtype == CNN_F32)
@@ -3837,6 +3856,7 @@ cnn_graph *graph_build(cnn_ctx *ctx, const void *X, int64_t n, int32_t d, int32_
         const int S = std::min(kSuperPivots, L);
         g->perm = dev_alloc<int32_t>(g, n);
         Scratch<uint32_t> keys(ctx, n);
+        Scratch<int32_t> iota(ctx, n);
         Scratch<int32_t> super_of(ctx, L);
         const unsigned blocks = (unsigned)ceil_div(n, 256);
         const int Lp = (L + 31) / 32 * 32;
@@ -3846,15 +3866,15 @@ cnn_graph *graph_build(cnn_ctx *ctx, const void *X, int64_t n, int32_t d, int32_
             k_pivot_super<float><<<1, 256, 0, s>>>((const float *)X, n, d, L, S, super_of.p);
             k_pivot_table<float><<<(unsigned)Lp, 64, 0, s>>>((const float *)X, n, d, L, piv.p, phalf.p);
             k_pivot_cells_mfma<float, uint32_t><<<mblocks, 256, 0, s>>>((const float *)X, n, d, L, piv.p, phalf.p,
-                                                                       super_of.p, keys.p, g->perm);
+                                                                       super_of.p, keys.p, iota.p);
         } else {
             k_pivot_super<double><<<1, 256, 0, s>>>((const double *)X, n, d, L, S, super_of.p);
             k_pivot_table<double><<<(unsigned)Lp, 64, 0, s>>>((const double *)X, n, d, L, piv.p, phalf.p);
             k_pivot_cells_mfma<double, uint32_t><<<mblocks, 256, 0, s>>>((const double *)X, n, d, L, piv.p,
-                                                                        phalf.p, super_of.p, keys.p, g->perm);
+                                                                        phalf.p, super_of.p, keys.p, iota.p);
         }
         CNN_HIP(hipGetLastError());
-        sort_pairs_u32_i32(ctx, keys.p, g->perm, n, 12);
+        sort_pairs_u32_i32(ctx, keys.p, iota.p, g->perm, n, 12);
     }
     g->xw64 = dev_alloc<double>(g, n_pad * std::max(d, 1));
     if (band) g->xw32 = dev_alloc<float>(g, n_pad * std::max(d, 1));
