@@ -1281,7 +1281,7 @@ __device__ __forceinline__ uint32_t band_value(const float *srow, int i, const f
 // that are not finite in FP32 take the compares (their sign says nothing).
 // Bound by vector issue and the LDS broadcasts of the rows (16 bytes to 64 lanes
 // a row): n = 1e6, d = 3 (2.91e9 pairs) 825 us, 912 us with the compares; n = 8e4,
-// d = 8 262 against 290 us.
+// d = 8 262 against 271 us.
 template <int D>
 __global__ __launch_bounds__(256) void k_dist_f32_cols(DistArgs a) {
     constexpr int DP = lds_row_stride<float, D>();

@@ -359,7 +359,8 @@ int cnn_similarity_mst(cnn_ctx *ctx, const int64_t *row_ptr, const int32_t *col,
  * autotuner (commonnnclustering_amd/autotune.py).  No counterpart in the
  * reference.  Every value is exact-result neutral: it changes speed only. */
 typedef struct {
-    int32_t mfma_col_chunk;  /* column tiles per workgroup of the dense MFMA distance kernel (8..1024; 64) */
+    int32_t mfma_col_chunk;  /* column tiles per workgroup of the dense MFMA distance kernel (8..1024; 64; the
+                                split FP16 form takes at most 64) */
     int32_t wide_col_chunk;  /* tile pairs per workgroup, at most, of the dense plain-FP64 kernel (1..1024; 32) */
     int32_t emit_waves;      /* waves per workgroup of the neighbour-list emission (4 or 8; 8) */
     int32_t root_passes;     /* root-hooking passes before the full round of a labelling on lists (0..8; 2) */
