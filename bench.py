@@ -52,6 +52,7 @@ FP64_PEAK_TFLOPS = 78.6      # FMA-counted; separately rounded sub/mul/add reach
 # scaled by a copy kernel of known size (profiles/*_traffic.json).
 TRAFFIC_FILES = {
     ("k_dist_f32_cols", "md_basins_3d"): "profiles/k_dist_f32_cols_md_basins_3d_traffic.json",
+    ("k_dist_split", "features_64d"): "profiles/k_dist_split_features_64d_traffic.json",
     ("round", "md_basins_3d"): "profiles/round_md_basins_3d_traffic.json",
     ("hook", "md_basins_3d"): "profiles/hook_md_basins_3d_traffic.json",
     ("round", "features_64d"): "profiles/round_features_64d_traffic.json",
