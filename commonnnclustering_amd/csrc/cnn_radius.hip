@@ -3149,8 +3149,11 @@ static void launch_dist(cnn_ctx *ctx, const DistArgs &a, int64_t n_rt, bool band
     }
     if (band && a.d >= kMfmaMinD) {
         // guard-band elements are listed (and, when the list is full, whole tile pairs,
-        // at most once each) and settled afterwards
-        int64_t cap = std::min<int64_t>(std::max<int64_t>(batch_pairs / 4, 1 << 14), (int64_t)1 << 21);
+        // at most once each) and settled afterwards.  Half a record per pair: a wave
+        // reserves slots 8 at a time and leaves some empty, so at a quarter the list
+        // was full at 5.5e5 elements (n = 2e5, d = 64) and the recomputing kernel took
+        // 820 us, now 4; reserving 2 at a time instead cost k_dist_split 1.59 -> 2.28 ms.
+        int64_t cap = std::min<int64_t>(std::max<int64_t>(batch_pairs / 2, 1 << 14), (int64_t)1 << 21);
         if (const char *ev = std::getenv("CNN_HIP_BAND_RECORDS")) cap = std::max<int64_t>(1, std::atoll(ev));
         Scratch<int64_t> cnt(ctx, 2);
         Scratch<int64_t> list(ctx, 66 * cap);
