@@ -2073,11 +2073,13 @@ __device__ __forceinline__ uint32_t sign_bits(F &&x) {
 
 // Stores pair k's row words and the mirror pair's (km, -1: none), which are the
 // column words, and adds the column side's degrees; returns the row word's
-// popcount.  As store_pair, for column words without bits in padding rows and
-// columns.  force: store empty words too.
-__device__ __forceinline__ int store_words(const DistArgs &a, int64_t k, int64_t km, int64_t C, uint64_t colword,
-                                           bool force = false) {
+// popcount.  As store_pair, which also clears padding rows and columns: their
+// values follow from a term that no radius bounds.  force: store empty words too.
+__device__ __forceinline__ int store_words(const DistArgs &a, int64_t k, int64_t km, int64_t R, int64_t C,
+                                           uint64_t colword, bool force = false) {
     const int lane = threadIdx.x & 63;
+    colword &= valid_cols(a.n, R);
+    if (C * 64 + lane >= a.n) colword = 0ull;
     const bool any = __ballot(colword != 0ull) != 0ull;
     const bool mirrored = km >= 0;
     if (lane == 0) {
@@ -2154,7 +2156,7 @@ __device__ __forceinline__ int split_settle_store(const DistArgs &a, const MfmaT
         colword = merge_col_words(pa & 0x0f0f0f0fu, (pa >> 4) & 0x0f0f0f0fu, pb & 0x0f0f0f0fu,
                                   (pb >> 4) & 0x0f0f0f0fu);
     }
-    return store_words(a, k, km, C, colword, queued);
+    return store_words(a, k, km, R, C, colword, queued);
 }
 
 // E2 of a tile pair in scaled units: 2 (largest margin of the row tile + of
@@ -2656,7 +2658,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             x |= __shfl_xor(x, 32, 64);
             if (g == cb) colword = x;
         }
-        mydeg += store_words(a, k, km, C, colword);
+        mydeg += store_words(a, k, km, R, C, colword);
     }
     if (mydeg && R * 64 + lane < a.n) atomicAdd(&a.deg[R * 64 + lane], mydeg);
 }

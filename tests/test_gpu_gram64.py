@@ -52,6 +52,21 @@ def test_nonfinite_huge_and_tiny(cuda):
     _check(rng.normal(size=(300, 10)), np.inf)
 
 
+@pytest.mark.parametrize("r", [1e150, 2.1e150, 1e151, 1.3e154])
+@pytest.mark.parametrize("n,d", [(1, 9), (65, 9), (130, 64), (2113, 17)])
+def test_radius_beyond_the_padding_term(cuda, monkeypatch, n, d, r):
+    """r^2 up to the largest double: padding rows and columns of the ragged tile are
+    never neighbours, in one batch and in several."""
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(n, d))
+    x[::5] *= 1e149
+    _check(x, r)
+    lab = engine.fit(torch.from_numpy(x).cuda(), r * r, 3, 2, precision="f64", member_cutoff=1)[0].cpu().numpy()
+    assert (lab == C.fit(x, r, 1, member_cutoff=1)).all()
+    monkeypatch.setenv("CNN_HIP_MASK_BUDGET", "512")
+    _check(x, r)
+
+
 def test_row_tile_batches(cuda, monkeypatch):
     monkeypatch.setenv("CNN_HIP_MASK_BUDGET", str(512 * 200))
     rng = np.random.default_rng(8)
