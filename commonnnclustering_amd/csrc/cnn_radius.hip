@@ -2138,8 +2138,9 @@ __device__ __forceinline__ int split_settle_store(const DistArgs &a, const MfmaT
             flags = ~0ull;
         }
         if (__ballot(flags != 0ull)) {
-            // (padding rows and columns have no flags unless every element has)
-            if (!finite) {
+            // padding rows and columns are out of every radius, but tiles of very
+            // different scales can put their values inside the band
+            if (max(R, C) * 64 + 64 > a.n) {
                 for (int e = 0; e < 64; ++e) {
                     int row, col;
                     band_element(lane, e, row, col);

@@ -1,7 +1,8 @@
 """The split FP16 Gram form (banded precision, 16 <= d <= 128): neighbour lists
 equal the oracle's FP64 ones at every number of MFMA steps and its remainders,
 ragged tiles, the ordered and the plain layout, tiles of very different scales,
-subnormal FP16 parts, non-finite and huge points, and with the record list full."""
+subnormal FP16 parts, non-finite and huge points, padding next to far points, and
+with the record list full."""
 
 import numpy as np
 import pytest
@@ -65,6 +66,25 @@ def test_nonfinite_and_huge(cuda):
     x = rng.normal(size=(400, 18)).astype(np.float32)
     x[3, 2], x[70, 0], x[140, 17], x[200], x[399, 1] = np.nan, np.inf, -np.inf, 3e37, 2e18
     _check(x, 4.0)
+
+
+@pytest.mark.parametrize("records", [None, "1"])
+@pytest.mark.parametrize("budget", [None, "512"])
+@pytest.mark.parametrize("n,d", [(69, 64), (69, 16), (130, 128)])
+def test_padding_next_to_a_far_tile(cuda, monkeypatch, n, d, budget, records):
+    """A tile with a coordinate near 1e18 and the origin next to a ragged tile of
+    tiny scale: padding values fall inside the pair's band, in one batch and in
+    several, with room in the record list and without."""
+    for name, value in (("CNN_HIP_MASK_BUDGET", budget), ("CNN_HIP_BAND_RECORDS", records)):
+        if value is not None:
+            monkeypatch.setenv(name, value)
+    rng = np.random.default_rng(n)
+    for small in (1e-3, 1e-5):
+        x = (rng.uniform(-1.0, 1.0, size=(n, d)) * small).astype(np.float32)
+        x[0] = 0.0
+        x[1, 0] = 9e17
+        _check(x, small)
+        _check(x, 0.3 * small * np.sqrt(d))
 
 
 @pytest.mark.parametrize("records", ["1", "9"])
