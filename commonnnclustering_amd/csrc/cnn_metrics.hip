@@ -176,6 +176,9 @@ int cnn_precomputed_emit(cnn_ctx *ctx, const cnn_precomputed *p, const int64_t *
     return guarded(ctx, [&]() {
         CNN_HIP(hipSetDevice(ctx->device));
         pre_emit(ctx, *p, row_ptr, col, col_cap);
+        // the words go back to the context's working memory with the handle, and the
+        // context's next call may run on another stream
+        CNN_HIP(hipStreamSynchronize(ctx->stream));
         return (int)CNN_OK;
     });
 }

@@ -304,9 +304,10 @@ int cnn_precomputed_csr(cnn_ctx *ctx, const void *D, int64_t n, int32_t dtype, d
 
 /* The same in two steps that read D once, for callers that size col from the
  * count: create thresholds D (row_ptr complete, counts on the host) and keeps
- * the decisions in the context's working memory; emit writes the lists (stream-
- * ordered on the context's stream; CNN_ERR_CAPACITY when col_cap < nnz).  Use and
- * destroy the handle on the context's thread, before the context. */
+ * the decisions in the context's working memory; emit writes the lists
+ * (CNN_ERR_CAPACITY when col_cap < nnz).  Each ends with its work on the context's
+ * stream complete.  Use and destroy the handle on the context's thread, before the
+ * context. */
 typedef struct cnn_precomputed cnn_precomputed;
 int cnn_precomputed_create(cnn_ctx *ctx, const void *D, int64_t n, int32_t dtype, double r,
                            int64_t *row_ptr, cnn_precomputed **out, int64_t *nnz_out,

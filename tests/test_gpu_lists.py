@@ -40,6 +40,25 @@ def test_precomputed_words(cuda, n, dtype):
     assert (out[:len(col)] == col).all()
 
 
+@pytest.mark.parametrize("n", [65, 4001])
+def test_precomputed_is_complete_on_return(cuda, n):
+    """No work is left on the call's stream, so the thread's next call may take the
+    context's working memory on another stream."""
+    x = np.random.default_rng(n).normal(size=(n, 2))
+    d = np.sqrt(((x[:, None] - x[None]) ** 2).sum(-1))
+    D, X = torch.from_numpy(d).cuda(), torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    want_rp, want_col = np.concatenate([[0], np.cumsum((d <= 0.9).sum(1))]), np.nonzero(d <= 0.9)[1]
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(3):
+        with torch.cuda.stream(a):
+            row_ptr, col, _ = engine.precomputed_csr(D, 0.9)
+            assert a.query()
+        with torch.cuda.stream(b):
+            engine.fit(X, 0.25, 5, 4)
+        assert (row_ptr.cpu().numpy() == want_rp).all() and (col.cpu().numpy() == want_col).all()
+
+
 def _csr(rows):
     rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64)
     return torch.from_numpy(rp).cuda(), torch.tensor([j for r in rows for j in r], dtype=torch.int32, device="cuda")
