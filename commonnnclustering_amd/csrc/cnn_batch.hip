@@ -206,8 +206,8 @@ void scan_free(cnn_scan *sc) {
     if (sc->graph) (void)hipGraphDestroy(sc->graph);
     for (auto &e : sc->ev)
         if (e) (void)hipEventDestroy(e);
-    if (!sc->bufs.empty()) (void)hipDeviceSynchronize();
-    for (void *p : sc->bufs) pool_free(sc->device, p, true);
+    const bool waited = sc->bufs.empty() || device_wait();
+    for (void *p : sc->bufs) pool_free(sc->device, p, waited);
     delete sc;
 }
 

@@ -62,9 +62,11 @@ private:
 // blocks (the oldest are freed first), and is given back by cnn_ctx_trim, when
 // an allocation fails and with the device's last context.  pool_free waits for
 // the device before a block becomes available, as hipFree does, so a block may
-// be reused on any stream; `waited`: the caller has done so.
+// be reused on any stream; `waited`: the caller has done so.  Where the wait is
+// refused (a stream is being captured) the block is freed instead.
 constexpr size_t kPoolBytes = (size_t)1 << 30;
 constexpr size_t kPoolBlocks = 64;
+bool device_wait();                          // for the current device; false: refused
 void *pool_alloc(int device, size_t bytes);  // nullptr: out of memory
 void pool_free(int device, void *p, bool waited = false);
 void pool_trim(int device);

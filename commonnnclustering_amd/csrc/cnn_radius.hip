@@ -3297,12 +3297,12 @@ static T *dev_alloc(cnn_graph *g, int64_t count) {
 void graph_free(cnn_graph *g) {
     if (!g) return;
     (void)hipSetDevice(g->device);
-    if (!g->arena) (void)hipDeviceSynchronize();  // as hipFree: no kernel reads the graph any more
+    const bool waited = g->arena || device_wait();  // as hipFree: no kernel reads the graph any more
     for (void *p : {(void *)g->perm, (void *)g->xw64, (void *)g->xw32, (void *)g->row_ptr, (void *)g->col,
                     (void *)g->tp_ptr, (void *)g->tp_col, (void *)g->diag, (void *)g->tile_order, (void *)g->selfpos,
                     (void *)g->mask, (void *)g->bounds})
-        graph_mem_free(g, p, true);
-    pool_free(g->device, g->slab, true);
+        graph_mem_free(g, p, waited);
+    pool_free(g->device, g->slab, waited);
     delete g;
 }
 

@@ -128,16 +128,27 @@ void *pool_alloc(int device, size_t bytes) {
     return p;
 }
 
+bool device_wait() {
+    if (hipDeviceSynchronize() == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 void pool_free(int device, void *p, bool waited) {
     if (!p) return;
-    if (!waited) (void)hipDeviceSynchronize();
+    waited = waited || device_wait();
     std::lock_guard<std::mutex> lock(pool_mu);
     DevicePool &d = pools[device];
     auto it = d.in_use.find(p);
     const size_t size = it == d.in_use.end() ? 0 : it->second;
     if (it != d.in_use.end()) d.in_use.erase(it);
-    if (size == 0 || size > kPoolBytes || d.contexts == 0) {
+    if (!waited || size == 0 || size > kPoolBytes || d.contexts == 0) {
+        // hipFree waits for the device itself; while a stream is captured it is
+        // let through in the relaxed mode only
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
         (void)hipFree(p);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
         return;
     }
     while (!d.free.empty() && (d.free_bytes + size > kPoolBytes || d.free.size() >= kPoolBlocks)) pool_drop(d, 0);

@@ -1,7 +1,8 @@
 """Graphs built, fitted and released again and again on several threads and
-streams share freed device memory: results stay right, and the memory is given
-back on trim."""
+streams share freed device memory: results stay right, the memory is given
+back on trim, and a release is safe while a stream is captured."""
 
+import ctypes
 import threading
 
 import numpy as np
@@ -54,3 +55,34 @@ def test_trim_gives_the_memory_back(cuda):
     engine.build_graph(X, 0.04).release()
     ctx.trim()
     assert torch.cuda.mem_get_info()[0] >= before - (64 << 20)
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_release_while_a_stream_is_captured(cuda, mode):
+    """A thread that captures a stream (globally, or for itself) may not wait for the
+    device.  A graph released then is freed: it must not enter the pool unwaited.
+    (The refused wait invalidates the capture, as documented for HIP.)"""
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
+    hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
+    ctx = _lib.get_context(torch.device("cuda", 0))
+    X = torch.from_numpy(np.random.default_rng(3).normal(size=(200_000, 3))).cuda()
+    engine.build_graph(X, 0.04).release()
+    ctx.trim()
+    graph = engine.build_graph(X, 0.04)
+    ctx.trim()
+    size = graph.nbytes
+    assert size > 64 << 20
+    stream, recorded = torch.cuda.Stream(), ctypes.c_void_p()
+    torch.cuda.synchronize()
+    held = torch.cuda.mem_get_info()[0]
+    assert hip.hipStreamBeginCapture(stream.cuda_stream, mode) == 0
+    graph.release()
+    if hip.hipStreamEndCapture(stream.cuda_stream, ctypes.byref(recorded)) == 0:
+        hip.hipGraphDestroy(recorded)
+    hip.hipGetLastError()
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] > held + size // 2
+    want = engine.fit(X, 0.04, 5, 4)[0]
+    assert (engine.build_graph(X, 0.04).fit(5, 4)[0] == want).all()
