@@ -1573,25 +1573,58 @@ __device__ __forceinline__ uint64_t pack_halves(uint32_t a_lo, uint32_t a_hi, ui
 // in registers -- flattens their elements into an LDS list (record, lane, bit)
 // and decides each in FP64 in reference order, or-ing its bit into the stored
 // words of the pair and of its mirror and counting it in both degrees.  The
-// number of records is read on the device.  The FP32 statistics add the FP32
-// products along the way (statistics only).
+// number of records is read on the device.
 // Bound by the latency of the record and row reads: with the records read one
 // after another, 68 KB of LDS and whole-row loads it took 508 us for 443,000
-// elements of 64 dimensions, as here 218 us.
+// elements of 64 dimensions, as here 236 us (18 of it the split form's value).
 constexpr int kBandGroup = 64;     // records a workgroup flattens at a time
 constexpr int kBandElems = 4096;   // elements of its list; one record has at most as many
+
+// The FP32 value that a Gram form finds for a pair, formed along the FP64
+// evaluation (statistics only): add() per dimension, end() after every eight
+// and after the last.
+struct GramValue {  // FP32 products, one after another
+    float p = 0.0f;
+    __device__ __forceinline__ void add(double x, double y) { p = __builtin_fmaf((float)x, (float)y, p); }
+    __device__ __forceinline__ void end() {}
+};
+
+// The split form's: the parts of both sides, the products of eight dimensions
+// summed together and rounded into the FP32 sum as k_dist_split's instructions
+// do; only the small products' sum is added last here.
+struct SplitValue {
+    float sr, sc;           // the tiles' scales
+    float big, small = 0.0f;  // h h' on top of the terms c; h l' and l h'
+    double hh = 0.0, lh = 0.0, hl = 0.0;
+    __device__ __forceinline__ SplitValue(const DistArgs &a, int64_t gi, int64_t gj, float sr_, float sc_)
+        : sr(sr_), sc(sc_), big((a.caug[gi] * sr_) * sc_ + (a.caug[gj] * sc_) * sr_) {}
+    __device__ __forceinline__ void add(double x, double y) {
+        const float xs = (float)x * sr, ys = (float)y * sc;
+        const _Float16 xh = (_Float16)xs, yh = (_Float16)ys;
+        const double xl = (double)(_Float16)(xs - (float)xh), yl = (double)(_Float16)(ys - (float)yh);
+        hh += (double)xh * (double)yh;
+        lh += xl * (double)yh;
+        hl += (double)xh * yl;
+    }
+    __device__ __forceinline__ void end() {
+        small = (float)((double)small + lh);
+        small = (float)((double)small + hl);
+        big = (float)((double)big + hh);
+        hh = lh = hl = 0.0;
+    }
+    __device__ __forceinline__ double value() const { return (double)(big + small) / ((double)sr * (double)sc); }
+};
 
 // exact_d2 with the row reads grouped: eight dimensions of both rows loaded
 // together as 16-byte pairs (rows start 16-byte aligned when d is even), so a
 // thread's accesses to a row's cache lines come close together; the sum is
-// the same sequence of separately rounded steps in ascending k.  prod: the FP32
-// products' sum.
+// the same sequence of separately rounded steps in ascending k.
+template <typename V>
 __device__ __forceinline__ double exact_d2_grouped(const double *__restrict__ xw64, int d, int64_t i, int64_t j,
-                                                   float &prod) {
+                                                   V &val) {
     const double *a = xw64 + i * d;
     const double *b = xw64 + j * d;
     double s = 0.0;
-    float p = 0.0f;
     int k = 0;
     if ((d & 1) == 0) {
         for (; k + 8 <= d; k += 8) {
@@ -1604,32 +1637,35 @@ __device__ __forceinline__ double exact_d2_grouped(const double *__restrict__ xw
             for (int q = 0; q < 8; ++q) {
                 const double t = av[q] - bv[q];
                 s = s + t * t;
-                p = __builtin_fmaf((float)av[q], (float)bv[q], p);
+                val.add(av[q], bv[q]);
             }
+            val.end();
         }
     }
     for (; k < d; ++k) {
         const double t = a[k] - b[k];
         s = s + t * t;
-        p = __builtin_fmaf((float)a[k], (float)b[k], p);
+        val.add(a[k], b[k]);
+        if ((k & 7) == 7) val.end();
     }
-    prod = p;
+    val.end();
     return s;
 }
 
-// FP32 Gram value of points gi, gj from the plain FP32 rows (statistics only).
-__device__ __forceinline__ float gram_value(const DistArgs &a, int64_t gi, int64_t gj) {
-    const float *x = a.xw32 + gi * a.d, *y = a.xw32 + gj * a.d;
-    float prod = 0.0f;
-    for (int k = 0; k < a.d; ++k) prod = __builtin_fmaf(x[k], y[k], prod);
-    return prod + a.caug[gi] + a.caug[gj];
+// Statistics of one settled pair: d2 the FP32 form's value, ex the FP64 one.
+__device__ __forceinline__ void band_pair_stats(double d2, double ex, double r2, unsigned &flips, double &maxerr) {
+    flips += (ex <= r2) != (d2 <= r2);
+    const double err = fabs(d2 - ex);
+    if (err == err) maxerr = fmax(maxerr, err);
 }
 
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void k_band_settle(DistArgs a) {
     __shared__ uint32_t s_elem[kBandElems];
     __shared__ int s_cnt[kBandGroup];
     __shared__ int64_t s_k[kBandGroup];
     __shared__ int2 s_rc[kBandGroup];
+    __shared__ float2 s_scale[kBandGroup];  // the tiles' scales; 0: no finite margin, so no FP32 value
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t n_rec = min((int64_t)*a.band_cnt, a.band_cap);
     unsigned hits = 0, flips = 0;
@@ -1655,6 +1691,9 @@ __global__ __launch_bounds__(256) void k_band_settle(DistArgs a) {
             }
             s_k[wave * kRec + lane] = k_rec;
             s_rc[wave * kRec + lane] = make_int2((int)R, (int)C);
+            if constexpr (SPLIT)
+                s_scale[wave * kRec + lane] =
+                    a.se[R] + a.se[C] < INFINITY ? make_float2(a.ss[R], a.ss[C]) : make_float2(0.0f, 0.0f);
         }
         const uint64_t used = __ballot(k_rec >= 0);
         int incl[kRec];
@@ -1692,14 +1731,20 @@ __global__ __launch_bounds__(256) void k_band_settle(DistArgs a) {
                 int row, col;
                 band_element((int)((v >> 6) & 63), (int)(v & 63), row, col);
                 const int64_t gi = R * 64 + row, gj = C * 64 + col;
-                float prod;
-                const double ex = exact_d2_grouped(a.xw64, a.d, gi, gj, prod);
+                double ex;
+                if constexpr (SPLIT) {
+                    const float2 sc = s_scale[v >> 12];
+                    SplitValue val(a, gi, gj, sc.x, sc.y);
+                    ex = exact_d2_grouped(a.xw64, a.d, gi, gj, val);
+                    if (sc.x > 0.0f) band_pair_stats(a.bp.r2 - 2.0 * val.value(), ex, a.bp.r2, flips, maxerr);
+                } else {
+                    GramValue val;
+                    ex = exact_d2_grouped(a.xw64, a.d, gi, gj, val);
+                    band_pair_stats(a.bp.r2 - 2.0 * (double)(val.p + a.caug[gi] + a.caug[gj]), ex, a.bp.r2, flips,
+                                    maxerr);
+                }
                 const bool in = ex <= a.bp.r2;
-                const double d2 = a.bp.r2 - 2.0 * (double)(prod + a.caug[gi] + a.caug[gj]);
                 ++hits;
-                flips += in != (d2 <= a.bp.r2);
-                const double err = fabs(d2 - ex);
-                if (err == err) maxerr = fmax(maxerr, err);
                 if (in) {
                     atomicOr(&a.mask[(k - a.k_base) * 64 + row], 1ull << col);
                     atomicAdd(&a.deg[gi], 1);
@@ -2338,26 +2383,30 @@ __global__ __launch_bounds__(64) void k_split_band(DistArgs a) {
         const bool finite = E2 < INFINITY;
         MfmaTile t;
         split_tile<KS>(A, a.sx + C * (KS * 256) + lane, cb0, cb1, t);
-        uint32_t half[2] = {0u, 0u};  // new bits, layout of pack_halves
+        uint64_t flags = 0ull;  // elements in the band
 #pragma unroll
         for (int e = 0; e < 64; ++e) {
             const int v = 4 * ((e & 31) >> 3) + (e & 3), blk = ((e >> 2) & 1) + 2 * (e >> 5);
             const float x = blk == 0 ? t.c00[v] : blk == 1 ? t.c10[v] : blk == 2 ? t.c01[v] : t.c11[v];
+            const bool neg = (__float_as_uint(x) >> 31) != 0u;
+            if (!finite || (neg && (__float_as_uint(x + E2) >> 31) == 0u)) flags |= 1ull << e;
+        }
+        uint32_t half[2] = {0u, 0u};  // new bits, layout of pack_halves
+        while (flags) {
+            const int e = __ffsll((unsigned long long)flags) - 1;
+            flags &= flags - 1;
             int row, col;
             band_element(lane, e, row, col);
             const int64_t gi = R * 64 + row, gj = C * 64 + col;
-            const bool neg = (__float_as_uint(x) >> 31) != 0u;
-            const bool band = !finite || (neg && (__float_as_uint(x + E2) >> 31) == 0u);
-            if (band && gi < a.n && gj < a.n) {
-                const double exd = exact_d2(a.xw64, a.d, gi, gj);
-                const bool in = exd <= a.bp.r2;
-                if (in) half[e >> 5] |= 1u << (e & 31);
-                ++hits;
-                const double d2 = a.bp.r2 - 2.0 * (double)gram_value(a, gi, gj);
-                flips += (in != (d2 <= a.bp.r2));
-                const double err = fabs(d2 - exd);
-                if (err == err) maxerr = fmax(maxerr, err);
+            if (gi >= a.n || gj >= a.n) continue;
+            SplitValue val(a, gi, gj, a.ss[R], s_col);
+            const double ex = exact_d2_grouped(a.xw64, a.d, gi, gj, val);
+            if (ex <= a.bp.r2) {
+                if (e < 32) half[0] |= 1u << e;
+                else half[1] |= 1u << (e - 32);
             }
+            ++hits;
+            if (finite) band_pair_stats(a.bp.r2 - 2.0 * val.value(), ex, a.bp.r2, flips, maxerr);
         }
         const uint64_t colword = merge_col_words(half[0] & 0x0f0f0f0fu, (half[0] >> 4) & 0x0f0f0f0fu,
                                                  half[1] & 0x0f0f0f0fu, (half[1] >> 4) & 0x0f0f0f0fu);
@@ -3183,7 +3232,9 @@ static void launch_dist(cnn_ctx *ctx, const DistArgs &a, int64_t n_rt, bool band
         CNN_HIP(hipGetLastError());
         CNN_HIP(hipEventRecord(ctx->ev[7], s));
         // both counts are read on the device; every queued pair fits redo
-        k_band_settle<<<(unsigned)std::min<int64_t>(ceil_div(cap, kBandGroup), 2048), 256, 0, s>>>(b);
+        const unsigned sblocks = (unsigned)std::min<int64_t>(ceil_div(cap, kBandGroup), 2048);
+        if (a.sx) k_band_settle<true><<<sblocks, 256, 0, s>>>(b);
+        else k_band_settle<false><<<sblocks, 256, 0, s>>>(b);
         if (a.sx)
             split_dispatch(a.d, [&](auto ks) { k_split_band<decltype(ks)::value><<<rblocks, 64, 0, s>>>(b); });
         else

@@ -89,7 +89,9 @@ typedef struct {
                                   applied; a symmetric launch computes each unordered pair once) */
     int64_t band_hits;         /* FP32 pairs recomputed in FP64 */
     int64_t band_flips;        /* band pairs whose FP64 decision differed from the FP32 one */
-    double max_abs_err_band;   /* max |d2_fp32 - d2_fp64| over band pairs */
+    double max_abs_err_band;   /* max |d2_fp32 - d2_fp64| over band pairs; 16 <= d <= 128: d2_fp32 is the
+                                  split FP16 form's value (its small products' sum added last), and pairs of
+                                  tiles without a finite margin, which have none, are left out of both */
     int64_t tile_pairs;        /* 64x64 tile pairs evaluated */
     int64_t nnz;               /* neighbour-list entries (self included) */
     float ms_prep;             /* ordering, tiling, candidate tile pairs */

@@ -98,6 +98,56 @@ def test_full_record_list(cuda, monkeypatch, records, d):
     assert st["band_hits"] > 0
 
 
+def _split_d2(x, r2):
+    """The split form's FP32 values of d2 for all pairs: scaled parts, products of
+    eight dimensions summed and rounded into FP32, the small products' sum last."""
+    f32, f64 = np.float32, np.float64
+    x = x.astype(f32)
+    n, d = x.shape
+    tile = np.arange(n) // 64
+    m = np.array([max(np.abs(x[tile == t]).max(), np.sqrt(r2)) for t in range(tile[-1] + 1)])
+    s = (2.0 ** (13 - np.floor(np.log2(m)))).astype(f32)[tile]
+    xs = x * s[:, None]
+    h = xs.astype(np.float16)
+    low = (xs - h.astype(f32)).astype(np.float16).astype(f64)
+    h = h.astype(f64)
+    c = (0.25 * r2 - 0.5 * (x.astype(f64) ** 2).sum(1)).astype(f32)
+    big = (c * s)[:, None] * s[None] + (c * s)[None] * s[:, None]
+    small = np.zeros((n, n), f32)
+    for k0 in range(0, d, 8):
+        hh, lh, hl = np.zeros((n, n)), np.zeros((n, n)), np.zeros((n, n))
+        for k in range(k0, min(k0 + 8, d)):
+            hh += h[:, None, k] * h[None, :, k]
+            lh += low[:, None, k] * h[None, :, k]
+            hl += h[:, None, k] * low[None, :, k]
+        small = (small + lh).astype(f32)
+        small = (small + hl).astype(f32)
+        big = (big + hh).astype(f32)
+    return r2 - 2.0 * ((big + small).astype(f64) / (s[:, None].astype(f64) * s[None].astype(f64)))
+
+
+@pytest.mark.parametrize("records", [None, "1"])
+@pytest.mark.parametrize("n,d", [(200, 16), (257, 33), (190, 64), (130, 128)])
+def test_band_statistics(cuda, monkeypatch, n, d, records):
+    """1000 from the origin every pair lies inside the band: the reported flips and
+    largest error are those of the split form's values over all pairs."""
+    if records is not None:
+        monkeypatch.setenv("CNN_HIP_BAND_RECORDS", records)
+    rng = np.random.default_rng(n)
+    x = (rng.normal(size=(n, d)) + 1000.0).astype(np.float32)
+    r = np.sqrt(2.0 * d)
+    st = _check(x, r)
+    y = x.astype(np.float64)
+    exact = np.zeros((n, n))
+    for k in range(d):
+        exact += (y[:, None, k] - y[None, :, k]) ** 2
+    value = _split_d2(x, r * r)
+    evaluated = np.arange(n)[:, None] // 64 <= np.arange(n)[None] // 64  # a tile pair once
+    assert st["band_hits"] == evaluated.sum()
+    assert st["max_abs_err_band"] == pytest.approx(np.abs(value - exact)[evaluated].max(), rel=1e-9)
+    assert st["band_flips"] == ((value <= r * r) != (exact <= r * r))[evaluated].sum()
+
+
 def test_row_tile_batches(cuda, monkeypatch):
     """Several row-tile batches: every pair evaluated from both sides."""
     monkeypatch.setenv("CNN_HIP_MASK_BUDGET", str(512 * 200))
