@@ -48,6 +48,7 @@ EXPORTED = [
     "cnn_graph_bytes", "cnn_graph_export_csr", "cnn_radius_csr", "cnn_graph_rethreshold",
     "cnn_graph_labels", "cnn_labels_from_csr", "cnn_sort_by_size", "cnn_fit", "cnn_graph_fit",
     "cnn_fit_batch", "cnn_fit_scan", "cnn_predict", "cnn_precomputed_csr", "cnn_graph_build_periodic",
+    "cnn_pool_bytes", "cnn_pool_trim",
     "cnn_precomputed_create", "cnn_precomputed_emit", "cnn_precomputed_destroy",
     "cnn_csr_edge_similarity", "cnn_similarity_mst", "cnn_version", "cnn_labels_from_csr_noalloc",
     "cnn_tune_set", "cnn_tune_get", "cnn_tune_clear", "cnn_graph_scan_create", "cnn_scan_launch",
@@ -143,6 +144,8 @@ def _declare(L):
         "cnn_ctx_synchronize": (c, [_vp]),
         "cnn_ctx_workspace_bytes": (c, [_vp, _i64p]),
         "cnn_ctx_trim": (c, [_vp]),
+        "cnn_pool_bytes": (c, [ctypes.c_int, _i64p]),
+        "cnn_pool_trim": (c, [ctypes.c_int]),
         "cnn_graph_build": (c, [_vp, _vp, _i64, _i32, _i32, _dbl, _i32, ctypes.POINTER(_vp)]),
         "cnn_graph_destroy": (c, [_vp]),
         "cnn_graph_nnz": (c, [_vp, _i64p]),
@@ -260,6 +263,18 @@ class Context:
             self.close()
         except Exception:
             pass
+
+
+def pool_bytes(device: int = 0) -> int:
+    """Device memory of released graphs and scans that waits for the next ones."""
+    v = _i64()
+    lib().cnn_pool_bytes(int(device), ctypes.byref(v))
+    return v.value
+
+
+def trim_pool(device: int = 0) -> None:
+    """Gives that memory back to the device."""
+    lib().cnn_pool_trim(int(device))
 
 
 _contexts: dict = {}

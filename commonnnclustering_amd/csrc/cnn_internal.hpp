@@ -59,17 +59,19 @@ private:
 // scans).  A freed block waits in a pool of its device for the next object:
 // hipMalloc and hipFree of a graph's words (230 MB) take 85 and 280 us here.
 // The pool is shared by all threads, holds at most kPoolBytes in kPoolBlocks
-// blocks (the oldest are freed first), and is given back by cnn_ctx_trim, when
-// an allocation fails and with the device's last context.  pool_free waits for
-// the device before a block becomes available, as hipFree does, so a block may
-// be reused on any stream; `waited`: the caller has done so.  Where the wait is
-// refused (a stream is being captured) the block is freed instead.
+// blocks (the oldest are freed first), and is given back by cnn_ctx_trim and
+// cnn_pool_trim, when an allocation fails and with the device's last context.
+// pool_free waits for the device before a block becomes available, as hipFree
+// does, so a block may be reused on any stream; `waited`: the caller has done so.
+// Where the wait is refused (a stream is being captured) the block is freed
+// instead.
 constexpr size_t kPoolBytes = (size_t)1 << 30;
 constexpr size_t kPoolBlocks = 64;
 bool device_wait();                          // for the current device; false: refused
 void *pool_alloc(int device, size_t bytes);  // nullptr: out of memory
 void pool_free(int device, void *p, bool waited = false);
 void pool_trim(int device);
+size_t pool_bytes(int device);               // held for the next object
 
 // A fixed device buffer handed out front to back (entry points that may not
 // allocate).  Blocks are 256-byte aligned; releasing the most recent block

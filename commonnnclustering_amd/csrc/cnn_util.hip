@@ -158,8 +158,15 @@ void pool_free(int device, void *p, bool waited) {
 
 void pool_trim(int device) {
     std::lock_guard<std::mutex> lock(pool_mu);
-    DevicePool &d = pools[device];
-    while (!d.free.empty()) pool_drop(d, d.free.size() - 1);
+    const auto it = pools.find(device);
+    if (it == pools.end()) return;
+    while (!it->second.free.empty()) pool_drop(it->second, it->second.free.size() - 1);
+}
+
+size_t pool_bytes(int device) {
+    std::lock_guard<std::mutex> lock(pool_mu);
+    const auto it = pools.find(device);
+    return it == pools.end() ? 0 : it->second.free_bytes;
 }
 
 static void pool_contexts(int device, int change) {
@@ -392,6 +399,17 @@ int cnn_ctx_trim(cnn_ctx *ctx) {
         pool_trim(ctx->device);
         return (int)CNN_OK;
     });
+}
+
+int cnn_pool_bytes(int device, int64_t *bytes) {
+    if (!bytes) return CNN_ERR_INVALID;
+    *bytes = (int64_t)pool_bytes(device);
+    return CNN_OK;
+}
+
+int cnn_pool_trim(int device) {
+    pool_trim(device);
+    return CNN_OK;
 }
 
 int cnn_tune_set(int32_t d_lo, int32_t d_hi, int64_t n_lo, int64_t n_hi, int32_t precision,

@@ -31,7 +31,7 @@ from typing import Optional
 import numpy as np
 import torch
 
-from . import engine
+from . import _lib, engine
 
 
 @dataclass
@@ -187,6 +187,7 @@ class Server:
             for res in self._cache.values():
                 res.graph.release()
             self._cache.clear()
+        _lib.trim_pool(self.device.index)
 
     def __enter__(self):
         return self
@@ -214,6 +215,15 @@ class Server:
     def _cache_bytes(self) -> int:
         return sum(r.nbytes for r in self._cache.values())
 
+    def _make_room(self, need: int) -> None:
+        """When `need` more bytes do not fit next to the running requests, the
+        resident graphs and the pool of released graphs' memory: give the pool
+        back, and with it the least recently used resident graphs that are not in
+        use, until they do."""
+        if self._inflight + self._cache_bytes() + _lib.pool_bytes(self.device.index) + need > self.memory_budget:
+            self._evict(need)
+            _lib.trim_pool(self.device.index)
+
     def _evict(self, need: int) -> None:
         """Drop least recently used resident graphs (not in use) until `need`
         more bytes fit next to the running requests."""
@@ -239,8 +249,7 @@ class Server:
                     if p.req.X is None and p.req.dataset_id not in self._cache and \
                             p.req.dataset_id in self._producing:
                         continue  # its dataset is not resident yet
-                    if self._inflight + self._cache_bytes() + p.est > self.memory_budget:
-                        self._evict(p.est)
+                    self._make_room(p.est)
                     fits = self._inflight + self._cache_bytes() + p.est <= self.memory_budget
                     if fits or self._running == 0:
                         del self._pending[k]

@@ -144,6 +144,10 @@ int cnn_ctx_workspace_bytes(const cnn_ctx *ctx, int64_t *bytes);
 /* Release the workspace arena and the device's pool of freed graph memory (kept
  * between calls otherwise; the pool holds at most 1 GiB). */
 int cnn_ctx_trim(cnn_ctx *ctx);
+/* Freed graph and scan memory that the device's pool holds, and giving it back
+ * (the arenas of the contexts are not touched). */
+int cnn_pool_bytes(int device, int64_t *bytes);
+int cnn_pool_trim(int device);
 
 /* ------------------------------------------------------------------ phase N */
 /* Build the radius-r neighbour graph of X (device, row-major n x d, dtype

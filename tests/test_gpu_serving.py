@@ -7,8 +7,8 @@ import pytest
 import torch
 
 from oracle import c_oracle as C
-from commonnnclustering_amd import engine, synthetic
-from commonnnclustering_amd.serving import FitRequest, Server
+from commonnnclustering_amd import _lib, engine, synthetic
+from commonnnclustering_amd.serving import FitRequest, Server, _estimate_bytes
 
 pytestmark = pytest.mark.gpu
 
@@ -70,6 +70,28 @@ def test_tight_budget_serialises_but_agrees(cuda):
         got = [f.result(timeout=120) for f in futs]
     for g, w in zip(got, want):
         assert (g.labels == w).all()
+
+
+def test_released_memory_counts_against_the_budget(cuda):
+    """The pool that keeps released graphs' memory is given back when a request
+    would not fit beside it, and when the server closes."""
+    rng = np.random.default_rng(5)
+    a, b = rng.normal(size=(60_000, 3)).astype(np.float32), rng.normal(size=(20_000, 3)).astype(np.float32)
+    _lib.trim_pool(0)
+    with Server(slots=1) as srv:
+        srv.submit(FitRequest(0.15, 3, X=a, dataset_id="a")).result(timeout=120)
+        for _ in range(2):  # re-fits at a smaller radius: temporary graphs
+            srv.submit(FitRequest(0.12, 3, dataset_id="a")).result(timeout=120)
+        resident = srv.resident_bytes()
+        assert _lib.pool_bytes(0) > 0
+        srv.memory_budget = resident + _estimate_bytes(len(b), 3, 0.4 * 0.4, b, None)
+        got = srv.submit(FitRequest(0.4, 3, X=b)).result(timeout=120)  # (its graph is no pool memory)
+        assert _lib.pool_bytes(0) == 0 and srv.resident_bytes() == resident
+        want = engine.fit(torch.from_numpy(b).cuda(), 0.4 * 0.4, 5, 4, precision="f32_band")[0]
+        assert (got.labels == want.cpu().numpy()).all()
+        again = srv.submit(FitRequest(0.12, 3, dataset_id="a")).result(timeout=120)
+        assert again.graph_reused
+    assert _lib.pool_bytes(0) == 0
 
 
 def test_unknown_dataset_is_rejected(cuda):
