@@ -1956,7 +1956,7 @@ void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabe
     CNN_HIP(hipGetLastError());
     a.cand_max = b.cand_max;
     a.tile_rank = b.tile_common;
-    const int split = round_split(src.n_tile_pairs, T * nc);
+    const int split = round_split(src.n_tile_pairs * nc, T * nc);
     a.rq = b.rq;
     a.rq_len = b.rq_len;
     a.rq_cap = round_queue_cap(src.n_tile_pairs, b.n_c);
