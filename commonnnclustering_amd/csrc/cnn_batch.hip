@@ -265,7 +265,8 @@ cnn_scan *scan_create(cnn_ctx *ctx, const cnn_graph *g, const double *r2, int32_
     b.cnt = scan_alloc<int32_t>(sc.get(), m);
     b.hq = scan_alloc<uint32_t>(sc.get(), m);
     b.lens = scan_alloc<unsigned int>(sc.get(), 2 * (int64_t)n_c);
-    b.rq = scan_alloc<int2>(sc.get(), sz.round_queue);
+    b.rq_cap = sz.round_queue;
+    b.rq = scan_alloc<int2>(sc.get(), b.rq_cap * n_c);
     b.rq_len = scan_alloc<unsigned long long>(sc.get(), n_c);
     b.tmax = scan_alloc<uint64_t>(sc.get(), mt);
     b.cand_max = scan_alloc<uint64_t>(sc.get(), mt);

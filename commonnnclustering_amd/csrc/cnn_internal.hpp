@@ -396,7 +396,8 @@ struct MultiLabelBufs {
     int32_t *cnt = nullptr;
     uint32_t *hq = nullptr;        // hook queues
     unsigned int *lens = nullptr;  // 2 * n_c: hook queue lengths, cluster counts
-    int2 *rq = nullptr;            // round queues
+    int2 *rq = nullptr;            // round queues, rq_cap entries each
+    int64_t rq_cap = 0;
     unsigned long long *rq_len = nullptr;
     uint64_t *tmax = nullptr, *cand_max = nullptr, *tile_common = nullptr;
     int32_t *cmin = nullptr, *csize = nullptr, *newlab = nullptr;
@@ -406,7 +407,8 @@ struct MultiLabelBufs {
     const int32_t *csim = nullptr, *mcore = nullptr;  // device, n_c each
 };
 struct MultiLabelSizes {
-    int64_t per_point = 0, per_tile = 0, round_queue = 0;
+    int64_t per_point = 0, per_tile = 0;  // all pairs
+    int64_t round_queue = 0;              // entries of one pair's queue
 };
 // Counters a labelling pass starts from zero, cleared by its first kernel.
 struct ClearList {

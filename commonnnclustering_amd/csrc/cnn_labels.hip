@@ -27,6 +27,7 @@
 //   k_comp_stats flatten, component statistics; label assignment / sort_by_size
 #include <algorithm>
 #include <climits>
+#include <cstdlib>
 #include <memory>
 
 #include "cnn_internal.hpp"
@@ -1058,6 +1059,7 @@ __global__ __launch_bounds__(256) void k_round_queue(LabelArgs a) {
 
 // Queue entries of one full round over that many tile pairs.
 static int64_t round_queue_cap(int64_t n_tile_pairs, int n_c) {
+    if (const char *ev = std::getenv("CNN_HIP_ROUND_QUEUE")) return std::max<int64_t>(1, std::atoll(ev));  // tests
     return std::min<int64_t>(std::max<int64_t>(n_tile_pairs, 1), ((int64_t)1 << 21) / n_c);
 }
 
@@ -1716,10 +1718,10 @@ void labels_run(cnn_ctx *ctx, const LabelRequest &req, cnn_label_stats *st) {
     CNN_HIP(hipEventRecord(ctx->ev[10], s));
     if (words && a.mask && req.n_tiles > 0) {
         const int split = round_split(req.n_tile_pairs, req.n_tiles);
-        Scratch<int2> rq(ctx, round_queue_cap(req.n_tile_pairs, 1));
+        a.rq_cap = round_queue_cap(req.n_tile_pairs, 1);
+        Scratch<int2> rq(ctx, a.rq_cap);
         a.rq = rq.p;
         a.rq_len = slot_p + 1;  // zeroed with the counters
-        a.rq_cap = round_queue_cap(req.n_tile_pairs, 1);
         k_round_tile<<<blocks_for(req.n_tiles * split, 4), 256, 0, s>>>(a, req.n_tiles, split);
         k_round_queue<<<(unsigned)std::min<int64_t>(blocks_for(a.rq_cap, 4), 2048), 256, 0, s>>>(a);
         a.rq = nullptr;
@@ -1915,7 +1917,7 @@ __global__ __launch_bounds__(256) void k_rank_count(const uint64_t *ckey, const 
 void multi_labels_bytes(int64_t n, int64_t n_tiles, int64_t n_tile_pairs, int n_c, MultiLabelSizes &sz) {
     sz.per_point = n * n_c;
     sz.per_tile = std::max<int64_t>(n_tiles, 1) * n_c;
-    sz.round_queue = round_queue_cap(n_tile_pairs, n_c) * n_c;
+    sz.round_queue = round_queue_cap(n_tile_pairs, n_c);
 }
 
 void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabelSource &src, int64_t member_cutoff,
@@ -1959,7 +1961,7 @@ void labels_enqueue_multi(cnn_ctx *ctx, const MultiLabelBufs &b, const MultiLabe
     const int split = round_split(src.n_tile_pairs * nc, T * nc);
     a.rq = b.rq;
     a.rq_len = b.rq_len;
-    a.rq_cap = round_queue_cap(src.n_tile_pairs, b.n_c);
+    a.rq_cap = b.rq_cap;
     k_round_tile<<<g2(T * split, 4), 256, 0, s>>>(a, T, split);
     k_round_queue<<<dim3((unsigned)std::min<int64_t>(blocks_for(a.rq_cap, 4), 2048), nc), 256, 0, s>>>(a);
     k_comp_stats<<<g2(n, 256 * steps), 256, 0, s>>>(b.core, b.parent, src.perm, n, b.cmin, b.csize, counters + 2,

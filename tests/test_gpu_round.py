@@ -1,7 +1,8 @@
 """The label pass on tile-pair words at the places where its kernels can go
 wrong: tests that fail over many columns (batches of several columns a row, the
-queue of tile pairs), tiles with more common candidate tiles than one chunk of
-the match holds, ragged tiles, a cutoff of zero, mixed components per tile.
+queue of tile pairs, also when it is full), tiles with more common candidate tiles
+than one chunk of the match holds, ragged tiles, a cutoff of zero, mixed
+components per tile.
 Labels are whole numbers: equal to the oracle's."""
 
 import numpy as np
@@ -45,6 +46,29 @@ def test_round_matches_oracle(cuda, n, d, sep, r, cuts):
             lab = engine.fit(X, r * r, 0, 1, precision="f64", member_cutoff=1)[0].cpu().numpy()
             full = C.fit(x, r, 0, member_cutoff=1)
             assert ((lab > 0) >= (full > 0)).all()
+
+
+@pytest.mark.parametrize("capacity", ["1", "70"])
+@pytest.mark.parametrize("n,d,sep,r,cuts", CASES[2:])
+def test_full_queue_matches_oracle(cuda, monkeypatch, n, d, sep, r, cuts, capacity):
+    """Tile pairs beyond the round's queue are tested where they were found: fits,
+    every cutoff of a scan in one launch, and a batch."""
+    monkeypatch.setenv("CNN_HIP_ROUND_QUEUE", capacity)
+    x = _blobs(n, d, sep, n)
+    X = torch.from_numpy(x).cuda()
+    want = [C.fit(x, r, c, member_cutoff=2) for c in cuts]
+    for c, w in zip(cuts, want):
+        lab = engine.fit(X, r * r, c + 2, c + 1, precision="f64", member_cutoff=2)[0].cpu().numpy()
+        assert (lab == w).all(), f"c={c}"
+    if d > 3:
+        return
+    lab = engine.fit_scan(X, [r], list(cuts), precision="f64", member_cutoff=2)[0].cpu().numpy()
+    for ci, w in enumerate(want):
+        assert (lab[0, ci] == w).all(), f"scan c={cuts[ci]}"
+    both, offsets = torch.cat([X, X]), np.array([0, n, 2 * n])
+    lab = engine.fit_batch(both, offsets, np.full(2, r * r), cuts[-1] + 2, cuts[-1] + 1, precision="f64",
+                           member_cutoff=2)[0].cpu().numpy()
+    assert (lab[:n] == want[-1]).all() and (lab[n:] == want[-1]).all()
 
 
 @pytest.mark.parametrize("n,d,sep,r,cuts", [c for c in CASES if c[1] <= 3 and c[0] > 128])
