@@ -116,7 +116,7 @@ struct cnn_graph {
     double radius = 0.0;
     double r2 = 0.0;
     double *bounds = nullptr;    // periodic metric: period per dimension (device, d entries)
-    cnn::Arena *arena = nullptr; // memory owner when the graph lives inside one call (else hipMalloc)
+    cnn::Arena *arena = nullptr; // memory owner when the graph lives inside one call (else the device's pool)
     int32_t layout = 0;          // 0 identity, 1 spatial order
     int32_t dp = 0;              // row stride of xw32 (d, or d padded to 8 for the MFMA form)
     int64_t n_tiles = 0;

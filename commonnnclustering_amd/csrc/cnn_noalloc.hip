@@ -22,13 +22,17 @@
 namespace cnn {
 
 constexpr int64_t kNoAllocMaxPoints = CNN_NOALLOC_MAX_POINTS;
-// The pass needs at most 26 bytes per point at a time (core flags 1, snapshot
-// ranks 8, parents 4, component minima 4 and sizes 4, first-occurrence flags 1
-// and their scan 4; the root counts, 4, are released before the minima), plus
-// the statistics counters (32 KiB), the caller-CSR check (one word) and the
-// scan's temporary storage (a few KiB), each block rounded up to 256 bytes:
-// about 26 MiB at n = 2^20.
+// The pass needs at most 29 bytes per point at a time: core flags 1, snapshot
+// ranks 8, parents 4, component minima 4 and sizes 4, root counts 4 and, during
+// root hooking, the roots 4.  (The root counts and the roots are released before
+// the first-occurrence flags, 1, and their scan, 4, are taken.)  Beside these the
+// statistics counters (33 KiB), the caller-CSR check (one word) and the scan's
+// temporary storage (a few KiB), each block rounded up to 256 bytes: about
+// 29 MiB at n = 2^20.
+constexpr size_t kNoAllocPointBytes = 29, kNoAllocFixedBytes = size_t(1) << 20;
 constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;
+static_assert(kNoAllocPointBytes * kNoAllocMaxPoints + kNoAllocFixedBytes <= kNoAllocScratchBytes,
+              "the labelling pass's temporaries fit the fixed workspace");
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
