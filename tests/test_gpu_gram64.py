@@ -52,6 +52,31 @@ def test_nonfinite_huge_and_tiny(cuda):
     _check(rng.normal(size=(300, 10)), np.inf)
 
 
+@pytest.mark.parametrize("n,d", [(2, 9), (70, 64), (2113, 17)])
+@pytest.mark.parametrize("kind", ["offset", "column", "sampled rows", "no finite sample", "far samples"])
+def test_origin_of_the_coordinates(cuda, n, d, kind):
+    """The form works from a median of nine rows: points far from zero, one far
+    column, and sampled rows that are not finite or far from all others."""
+    rng = np.random.default_rng(n + d)
+    x = rng.normal(size=(n, d))
+    r = _quantile_radius(x, 0.2) if n > 2 else 4.0
+    sampled = np.arange(9) * (n - 1) // 8
+    if kind == "offset":
+        for offset in (1e3, 1e8, -1e15):
+            _check(x + offset, r)
+        return
+    if kind == "column":
+        x[:, -1] = 1.7e9 + np.sort(rng.uniform(0.0, 2.0 * r, n))
+    elif kind == "sampled rows":
+        x[sampled[::2], :3] = np.nan
+        x[sampled[1], 4:] = -np.inf
+    elif kind == "no finite sample":
+        x[sampled, 1] = np.inf
+    else:
+        x[sampled] += 1e14
+    _check(x, r)
+
+
 @pytest.mark.parametrize("r", [1e150, 2.1e150, 1e151, 1.3e154])
 @pytest.mark.parametrize("n,d", [(1, 9), (65, 9), (130, 64), (2113, 17)])
 def test_radius_beyond_the_padding_term(cuda, monkeypatch, n, d, r):
