@@ -813,6 +813,7 @@ struct DistArgs {
     const float *se;
     const float *ss;
     const float *caug;
+    const double *centre;  // split form: origin of its coordinates (gram_centre)
     // spatial layout, one batch: the row tile of workgroup b is row_order[b]
     // (heavy tiles first), nullptr: R0 + b
     const int32_t *row_order;
@@ -1585,7 +1586,7 @@ constexpr int kBandElems = 4096;   // elements of its list; one record has at mo
 // and after the last.
 struct GramValue {  // FP32 products, one after another
     float p = 0.0f;
-    __device__ __forceinline__ void add(double x, double y) { p = __builtin_fmaf((float)x, (float)y, p); }
+    __device__ __forceinline__ void add(int, double x, double y) { p = __builtin_fmaf((float)x, (float)y, p); }
     __device__ __forceinline__ void end() {}
 };
 
@@ -1593,13 +1594,15 @@ struct GramValue {  // FP32 products, one after another
 // summed together and rounded into the FP32 sum as k_dist_split's instructions
 // do; only the small products' sum is added last here.
 struct SplitValue {
-    float sr, sc;           // the tiles' scales
+    const double *__restrict__ centre;
+    float sr, sc;             // the tiles' scales
     float big, small = 0.0f;  // h h' on top of the terms c; h l' and l h'
     double hh = 0.0, lh = 0.0, hl = 0.0;
     __device__ __forceinline__ SplitValue(const DistArgs &a, int64_t gi, int64_t gj, float sr_, float sc_)
-        : sr(sr_), sc(sc_), big((a.caug[gi] * sr_) * sc_ + (a.caug[gj] * sc_) * sr_) {}
-    __device__ __forceinline__ void add(double x, double y) {
-        const float xs = (float)x * sr, ys = (float)y * sc;
+        : centre(a.centre), sr(sr_), sc(sc_), big((a.caug[gi] * sr_) * sc_ + (a.caug[gj] * sc_) * sr_) {}
+    __device__ __forceinline__ void add(int k, double x, double y) {
+        const double c = centre[k];
+        const float xs = (float)(x - c) * sr, ys = (float)(y - c) * sc;
         const _Float16 xh = (_Float16)xs, yh = (_Float16)ys;
         const double xl = (double)(_Float16)(xs - (float)xh), yl = (double)(_Float16)(ys - (float)yh);
         hh += (double)xh * (double)yh;
@@ -1637,7 +1640,7 @@ __device__ __forceinline__ double exact_d2_grouped(const double *__restrict__ xw
             for (int q = 0; q < 8; ++q) {
                 const double t = av[q] - bv[q];
                 s = s + t * t;
-                val.add(av[q], bv[q]);
+                val.add(k + q, av[q], bv[q]);
             }
             val.end();
         }
@@ -1645,7 +1648,7 @@ __device__ __forceinline__ double exact_d2_grouped(const double *__restrict__ xw
     for (; k < d; ++k) {
         const double t = a[k] - b[k];
         s = s + t * t;
-        val.add(a[k], b[k]);
+        val.add(k, a[k], b[k]);
         if ((k & 7) == 7) val.end();
     }
     val.end();
@@ -1902,6 +1905,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // m u / (1 - m u): the relative bound of m rounded operations of unit u.
 static double gamma_m(int m, double u) { return m * u / (1.0 - m * u); }
 
+// ------------------------------------------------------------------ origin of the Gram forms
+
+// Origin of the Gram forms' coordinates, by every thread of a workgroup (at most
+// 256 dimensions): per dimension the median of nine rows spread over the working
+// order (of the finite ones; 0 without any).  The margins grow with |x|^2, the
+// distances do not depend on the origin: without it points around 1e8 in every
+// dimension (n = 2e4, d = 64, plain) left every pair to the exact evaluation,
+// 28.6 ms a fit, as here 1.2 ms; around 1e3 (d = 64, banded) 7.6 ms, as here 0.59.
+template <typename T>
+__device__ __forceinline__ void gram_centre(const T *__restrict__ xw, int64_t n, int d, double *s_centre) {
+    const int k = threadIdx.x;
+    if (k < d) {
+        double v[9];
+        int m = 0;
+#pragma unroll
+        for (int q = 0; q < 9; ++q) v[q] = (double)xw[(q * (n - 1) / 8) * d + k];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const bool finite = fabs(v[q]) < INFINITY;
+            m += finite ? 1 : 0;
+            v[q] = finite ? v[q] : INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int j = i + 1; j < 9; ++j) {
+                const double lo = fmin(v[i], v[j]), hi = fmax(v[i], v[j]);
+                v[i] = lo;
+                v[j] = hi;
+            }
+        double c = 0.0;
+#pragma unroll
+        for (int q = 0; q < 9; ++q)
+            if (m > 0 && q == (m - 1) / 2) c = v[q];
+        s_centre[k] = c;
+    }
+    __syncthreads();
+}
+
 // ------------------------------------------------------------------ split FP16 Gram form on MFMA (16 <= d <= 128)
 //
 // T = x_i . x_j + c_i + c_j = (r2 - d2)/2 as in the FP32 Gram form, with each
@@ -1943,7 +1985,8 @@ __device__ __forceinline__ constexpr int split_at(int s, int p, int b) {
 //     1/s <= 2^-13 m, so 2^-26 sqrt(d) m |y| on either side, at most
 //     2^-27 sqrt(d) (w + m^2) a point;
 //   rounding c and its scaled form, r2/4: u w + u r2/2 (w is summed in FP64);
-//   f64 input rounded to f32: u w + u r2/2;
+//   rounding the centred coordinates: u |x| each, so T moves by at most u
+//     |x_i - x_j| (|x_i| + |x_j|) <= 2u (w_i + w_j);
 //   the reference's FP64 rounding near the threshold: gamma_{2d+2}(2^-53) r2/2.
 // Measured |d2_hat - d2| on 5e5 pairs of unit Gaussians around shared centres of
 // spread 2, split against FP32 form: d = 16 rms 7.6e-6 / 1.2e-5, largest
@@ -1955,37 +1998,40 @@ struct SplitMargin {
     double f;   // times w + m^2
     double b;   // constant
 };
-static SplitMargin split_margin(int d, int ks, bool rounded_coords, double r2) {
+static SplitMargin split_margin(int d, int ks, double r2) {
     const double u = std::ldexp(1.0, -24), u64 = std::ldexp(1.0, -53);
     const double g = gamma_m(16 * ks + 6, 2.0 * u);
     SplitMargin m;
     const double S = 1.0 + 64.0 * u;  // evaluating the margin itself
-    m.a = S * (g + 6.0 * u + u + (rounded_coords ? u : 0.0));
+    m.a = S * (g + 6.0 * u + u + 2.0 * u);
     m.f = S * std::ldexp(std::sqrt((double)d), -27);
-    m.b = S * (0.25 * g + u + 0.5 * gamma_m(2 * d + 2, u64) + (rounded_coords ? 0.5 * u : 0.0)) * r2 + 1e-30;
+    m.b = S * (0.25 * g + u + 0.5 * gamma_m(2 * d + 2, u64)) * r2 + 1e-30;
     return m;
 }
 
 // The split operands, terms and margins of one tile per workgroup, its
-// coordinates staged in LDS (rows padded by one: no bank conflicts).  Points
+// coordinates (from gram_centre's origin) staged in LDS (rows padded by one: no bank conflicts).  Points
 // that are non-finite or have |x|^2 > 1e36 get zero operands and an infinite
 // tile margin, which sends every element of the tile's pairs to the FP64
 // settling; padding rows get a term that is out of every radius.
-template <int KS>
-__global__ __launch_bounds__(256) void k_split_tiles(const float *__restrict__ xw32, int64_t n, int d, double r2,
+template <int KS, typename T>
+__global__ __launch_bounds__(256) void k_split_tiles(const T *__restrict__ xw, int64_t n, int d, double r2,
                                                      SplitMargin sm, uint4 *__restrict__ sx, float *__restrict__ sc,
                                                      float *__restrict__ se, float *__restrict__ ss,
-                                                     float *__restrict__ caug) {
+                                                     float *__restrict__ caug, double *__restrict__ centre) {
     constexpr int kD = 16 * KS;
     __shared__ float sxr[64 * (kD + 1)];
     __shared__ float s_max[4], s_e[4];
+    __shared__ double s_centre[kD];
     __shared__ int s_bad[64];
     const int64_t R = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    gram_centre(xw, n, d, s_centre);
+    if (R == 0 && tid < d) centre[tid] = s_centre[tid];
     for (int t = tid; t < 64 * kD; t += 256) sxr[(t / kD) * (kD + 1) + t % kD] = 0.0f;
     __syncthreads();
     const int rows = (int)min<int64_t>(64, n - R * 64);
-    for (int t = tid; t < rows * d; t += 256) sxr[(t / d) * (kD + 1) + t % d] = xw32[R * 64 * d + t];
+    for (int t = tid; t < rows * d; t += 256) sxr[(t / d) * (kD + 1) + t % d] = (float)((double)xw[R * 64 * d + t] - s_centre[t % d]);
     __syncthreads();
     // four threads a row
     const int row = tid >> 2, part = tid & 3;
@@ -2546,42 +2592,6 @@ struct Gram64Margin {
     double a, b;
 };
 
-// Origin of the Gram forms' coordinates, by every thread of a workgroup (at most
-// 256 dimensions): per dimension the median of nine rows spread over the working
-// order (of the finite ones; 0 without any).  The margins grow with |x|^2, the
-// distances do not depend on the origin: without it points around 1e8 in every
-// dimension (n = 2e4, d = 64) left every pair to the exact evaluation, 28.6 ms a
-// fit (3.3 ms by the vector form), as here 1.2 ms.
-template <typename T>
-__device__ __forceinline__ void gram_centre(const T *__restrict__ xw, int64_t n, int d, double *s_centre) {
-    const int k = threadIdx.x;
-    if (k < d) {
-        double v[9];
-        int m = 0;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) v[q] = (double)xw[(q * (n - 1) / 8) * d + k];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            const bool finite = fabs(v[q]) < INFINITY;
-            m += finite ? 1 : 0;
-            v[q] = finite ? v[q] : INFINITY;
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int j = i + 1; j < 9; ++j) {
-                const double lo = fmin(v[i], v[j]), hi = fmax(v[i], v[j]);
-                v[i] = lo;
-                v[j] = hi;
-            }
-        double c = 0.0;
-#pragma unroll
-        for (int q = 0; q < 9; ++q)
-            if (m > 0 && q == (m - 1) / 2) c = v[q];
-        s_centre[k] = c;
-    }
-    __syncthreads();
-}
 static Gram64Margin gram64_margin(int d, double r2) {
     const double u = std::ldexp(1.0, -53), g = gamma_m(d + 8, 2.0 * u);
     Gram64Margin m;
@@ -3511,17 +3521,24 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
     const bool split = gram && d <= kSplitMaxD;
     std::unique_ptr<Scratch<float>> xra, xca, emarg, caug, sc, se, ss;
     std::unique_ptr<Scratch<uint4>> sx;
+    std::unique_ptr<Scratch<double>> centre;
     if (split) {
         const int ks = (d + 15) / 16;
-        const SplitMargin sm = split_margin(d, ks, dtype == CNN_F64, g->r2);
+        const SplitMargin sm = split_margin(d, ks, g->r2);
         sx.reset(new Scratch<uint4>(ctx, T * ks * 256));
         sc.reset(new Scratch<float>(ctx, n_pad));
         caug.reset(new Scratch<float>(ctx, n_pad));
         se.reset(new Scratch<float>(ctx, T));
         ss.reset(new Scratch<float>(ctx, T));
+        centre.reset(new Scratch<double>(ctx, d));
         split_dispatch(d, [&](auto kc) {
-            k_split_tiles<decltype(kc)::value><<<(unsigned)T, 256, 0, s>>>(g->xw32, n, d, g->r2, sm, sx->p, sc->p,
-                                                                          se->p, ss->p, caug->p);
+            // (FP64 input: rounded to FP32 after centring)
+            if (dtype == CNN_F64)
+                k_split_tiles<decltype(kc)::value><<<(unsigned)T, 256, 0, s>>>(g->xw64, n, d, g->r2, sm, sx->p, sc->p,
+                                                                              se->p, ss->p, caug->p, centre->p);
+            else
+                k_split_tiles<decltype(kc)::value><<<(unsigned)T, 256, 0, s>>>(g->xw32, n, d, g->r2, sm, sx->p, sc->p,
+                                                                              se->p, ss->p, caug->p, centre->p);
         });
         CNN_HIP(hipGetLastError());
     } else if (gram) {
@@ -3790,6 +3807,7 @@ static void build_pairs_and_csr(cnn_ctx *ctx, cnn_graph *g, bool band, int dtype
             a.sc = sc->p;
             a.se = se->p;
             a.ss = ss->p;
+            a.centre = centre->p;
         }
         a.caug = caug ? caug->p : nullptr;
         a.col_chunk = g->tune.wide_col_chunk;

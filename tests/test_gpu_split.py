@@ -129,12 +129,16 @@ def _split_d2(x, r2):
 @pytest.mark.parametrize("records", [None, "1"])
 @pytest.mark.parametrize("n,d", [(200, 16), (257, 33), (190, 64), (130, 128)])
 def test_band_statistics(cuda, monkeypatch, n, d, records):
-    """1000 from the origin every pair lies inside the band: the reported flips and
-    largest error are those of the split form's values over all pairs."""
+    """Points 1000 from the form's origin (the median of nine rows, here all zero):
+    every pair of them lies inside the band, and the reported flips and largest
+    error are those of the split form's values over these pairs."""
     if records is not None:
         monkeypatch.setenv("CNN_HIP_BAND_RECORDS", records)
     rng = np.random.default_rng(n)
     x = (rng.normal(size=(n, d)) + 1000.0).astype(np.float32)
+    far = np.ones(n, bool)
+    far[np.arange(9) * (n - 1) // 8] = False
+    x[~far] = 0.0
     r = np.sqrt(2.0 * d)
     st = _check(x, r)
     y = x.astype(np.float64)
@@ -142,10 +146,49 @@ def test_band_statistics(cuda, monkeypatch, n, d, records):
     for k in range(d):
         exact += (y[:, None, k] - y[None, :, k]) ** 2
     value = _split_d2(x, r * r)
-    evaluated = np.arange(n)[:, None] // 64 <= np.arange(n)[None] // 64  # a tile pair once
-    assert st["band_hits"] == evaluated.sum()
-    assert st["max_abs_err_band"] == pytest.approx(np.abs(value - exact)[evaluated].max(), rel=1e-9)
-    assert st["band_flips"] == ((value <= r * r) != (exact <= r * r))[evaluated].sum()
+    tile = np.arange(n) // 64
+    pairs = (tile[:, None] <= tile[None]) & far[:, None] & far[None]  # a tile pair is evaluated once
+    assert st["band_hits"] == pairs.sum()
+    assert st["max_abs_err_band"] == pytest.approx(np.abs(value - exact)[pairs].max(), rel=1e-9)
+    assert st["band_flips"] == ((value <= r * r) != (exact <= r * r))[pairs].sum()
+
+
+@pytest.mark.parametrize("dtype,shift", [(np.float32, 1024.0), (np.float64, 2.0 ** 30)])
+@pytest.mark.parametrize("n,d", [(1, 16), (700, 16), (2000, 40), (300, 128)])
+def test_translation_changes_nothing(cuda, n, d, dtype, shift):
+    """The form works from a median of the points, so a translation that the input
+    holds exactly leaves lists and band statistics the same (in the caller's order,
+    n < 2048: beyond it the working order depends on the origin)."""
+    rng = np.random.default_rng(n)
+    x = np.rint(rng.normal(size=(n, d)) * 256.0) / 256.0
+    r = _quantile_radius(x, 0.05) if n > 1 else 1.0
+    base = _check(x.astype(dtype), r)
+    moved = (x + shift).astype(dtype)
+    assert (moved.astype(np.float64) == x + shift).all()
+    st = _check(moved, r)
+    for name in ("band_hits", "band_flips", "max_abs_err_band"):
+        assert st[name] == base[name], name
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["column", "sampled rows", "no finite sample", "far samples"])
+def test_origin_of_the_coordinates(cuda, kind, dtype):
+    """One far column, and sampled rows that are not finite or far from the others."""
+    for n, d in ((70, 64), (2113, 17)):
+        rng = np.random.default_rng(n + d)
+        x = rng.normal(size=(n, d))
+        r = _quantile_radius(x, 0.2)
+        sampled = np.arange(9) * (n - 1) // 8
+        if kind == "column":
+            x[:, -1] = 1e5 + np.sort(rng.uniform(0.0, 2.0 * r, n))
+        elif kind == "sampled rows":
+            x[sampled[::2], :3] = np.nan
+            x[sampled[1], 4:] = -np.inf
+        elif kind == "no finite sample":
+            x[sampled, 1] = np.inf
+        else:
+            x[sampled] += 1e14
+        _check(x.astype(dtype), r)
 
 
 def test_row_tile_batches(cuda, monkeypatch):
