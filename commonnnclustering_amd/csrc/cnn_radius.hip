@@ -1138,8 +1138,11 @@ __device__ __forceinline__ void flush_band(const DistArgs &a, unsigned hits, uns
         }
         if (h) {
             atomicAdd(&a.band_stats[0], h);
-            atomicAdd(&a.band_stats[1], f);
-            atomic_max_double(&a.band_stats[2], mx);
+            // (single addresses: no update that changes nothing)
+            if (f) atomicAdd(&a.band_stats[1], f);
+            if ((unsigned long long)__double_as_longlong(mx) >
+                __hip_atomic_load(&a.band_stats[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                atomic_max_double(&a.band_stats[2], mx);
         }
     }
 }
@@ -1582,8 +1585,13 @@ constexpr int kBandGroup = 64;     // records a workgroup flattens at a time
 constexpr int kBandElems = 4096;   // elements of its list; one record has at most as many
 
 // The FP32 value that a Gram form finds for a pair, formed along the FP64
-// evaluation (statistics only): add() per dimension, end() after every eight
-// and after the last.
+// evaluation (statistics only; NoValue: none): add() per dimension, end() after
+// every eight and after the last.
+struct NoValue {
+    __device__ __forceinline__ void add(int, double, double) {}
+    __device__ __forceinline__ void end() {}
+};
+
 struct GramValue {  // FP32 products, one after another
     float p = 0.0f;
     __device__ __forceinline__ void add(int, double x, double y) { p = __builtin_fmaf((float)x, (float)y, p); }
@@ -1605,9 +1613,9 @@ struct SplitValue {
         const float xs = (float)(x - c) * sr, ys = (float)(y - c) * sc;
         const _Float16 xh = (_Float16)xs, yh = (_Float16)ys;
         const double xl = (double)(_Float16)(xs - (float)xh), yl = (double)(_Float16)(ys - (float)yh);
-        hh += (double)xh * (double)yh;
-        lh += xl * (double)yh;
-        hl += (double)xh * yl;
+        hh = __builtin_fma((double)xh, (double)yh, hh);  // (exact products)
+        lh = __builtin_fma(xl, (double)yh, lh);
+        hl = __builtin_fma((double)xh, yl, hl);
     }
     __device__ __forceinline__ void end() {
         small = (float)((double)small + lh);
@@ -1797,18 +1805,27 @@ __device__ __forceinline__ void band_slots_release(const DistArgs &a, BandSlots 
     bs.next = bs.end;
 }
 
-// Queues the guard-band elements of pair k of row tile R (the lane's flags).
+// Queues the guard-band elements of pair k of row tile R (the lane's flags): as a
+// record, or, when the pair has more than kBandDense of them in most lanes or the
+// list is full, the whole pair for the kernels that recompute it.  k_band_settle's workgroups
+// take 64 records whatever they hold: with full pairs among them (64 clusters of
+// 312 points 1e4 radii apart, n = 2e4, d = 64: every pair within a cluster) a fit
+// took 7.2 ms, as here 2.8 (3.4 by the kernels before, which flattened all
+// elements of a launch).
+constexpr int kBandDense = 128;
 __device__ __forceinline__ void queue_band(const DistArgs &a, int64_t k, int64_t R, uint64_t flags, BandSlots &bs) {
     const int lane = threadIdx.x & 63;
-    if (bs.next == bs.end) {
+    // (few pairs have flags in most lanes: the others skip the sum)
+    const bool dense = __popcll(__ballot(flags != 0ull)) > 32 && wave_sum(__popcll(flags)) > kBandDense;
+    if (!dense && bs.next == bs.end) {
         unsigned long long base = 0;
         if (lane == 0) base = atomicAdd(a.band_cnt, (unsigned long long)kBandSlotChunk);
         base = __shfl(base, 0, 64);
         bs.next = base;
         bs.end = base + kBandSlotChunk;
     }
-    const unsigned long long slot = bs.next++;
-    if ((int64_t)slot < a.band_cap) {
+    const unsigned long long slot = dense ? ~0ull : bs.next++;
+    if (!dense && (int64_t)slot < a.band_cap) {
         int64_t *p = a.band_list + (int64_t)slot * 66;
         if (lane == 0) {
             p[0] = k;
@@ -1968,17 +1985,16 @@ __device__ __forceinline__ constexpr int split_at(int s, int p, int b) {
 
 // Margin of a point in the split form.  |T_hat - T| <= e_i + e_j with, for
 // w = |x|^2, u = 2^-24 and m the tile's largest |coordinate| or r if larger:
-//   accumulation: gamma_{16 KS + 6}(2u) of Sabs <= (w_i + w_j) + r2/2, that is
-//     32 KS + 12 units u.  What it has to cover: v_mfma_f32_32x32x16_f16 adds two
-//     groups of eight products; the products of a group are cut below 2^-24 of
-//     its largest exponent (less than u of Sabs each), then their sum joins the
-//     FP32 accumulator with one rounding (at most u, and u for what the
-//     accumulator loses when it is the smaller): 20 u an instruction, 20 KS for
-//     h.h'.  (Measured against exact sums over 65,536 results of eight kinds --
-//     mixed exponents, cancelling and dominating accumulators, subnormal parts:
-//     at most 6.4 u.)  The 2 KS instructions of the small products see sums of
-//     2^-10 Sabs: 0.04 KS.  The FP32 step is two FMAs rounded to nearest: 2.
-//     Together 20.04 KS + 2;
+//   accumulation: gamma_{21 KS + 6}(u) of Sabs <= (w_i + w_j) + r2/2.
+//     v_mfma_f32_32x32x16_f16 adds two groups of eight products; the products of
+//     a group are cut below 2^-24 of its largest exponent (less than u of Sabs
+//     each), then their sum joins the FP32 accumulator with one rounding (at most
+//     u, and u for what the accumulator loses when it is the smaller): 20 u an
+//     instruction, 20 KS for h.h'.  (Measured against exact sums over 65,536
+//     results of eight kinds -- mixed exponents, cancelling and dominating
+//     accumulators, subnormal parts: at most 6.4 u.)  The 2 KS instructions of the
+//     small products see sums of 2^-10 Sabs: 0.04 KS.  The FP32 step is two FMAs
+//     rounded to nearest: 2.  Together 20.04 KS + 2;
 //   the split: |x - (h + l)/s| <= 2^-22 |x| and the dropped l.l' <= 2^-22 |x||y|,
 //     in all 12u |x||y| <= 6u (w_i + w_j);
 //   FP16 subnormals, flushed or not: 2^-13/s absolute per coordinate and
@@ -2000,7 +2016,7 @@ struct SplitMargin {
 };
 static SplitMargin split_margin(int d, int ks, double r2) {
     const double u = std::ldexp(1.0, -24), u64 = std::ldexp(1.0, -53);
-    const double g = gamma_m(16 * ks + 6, 2.0 * u);
+    const double g = gamma_m(21 * ks + 6, u);
     SplitMargin m;
     const double S = 1.0 + 64.0 * u;  // evaluating the margin itself
     m.a = S * (g + 6.0 * u + u + 2.0 * u);
@@ -2411,13 +2427,63 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, KS <= 1 
     if (rvalid && mydeg && i < a.n) atomicAdd(&a.deg[i], mydeg);
 }
 
-// Band elements of the tile pairs that found the record list full (one wave per
-// pair, grid-stride, the count read on the device): U is recomputed by the same
-// instructions, every element in the band is decided in FP64 in reference
-// order by its own lane, and its bits are added to the stored words and degrees
-// of the pair and of its mirror.
+// Settles a queued tile pair whose values t the wave has recomputed: every element
+// that in_band() takes is decided in FP64 in reference order by its own lane, and
+// its bits are added to the stored words and degrees of the pair and of its
+// mirror.  s_u: the lanes' values (a private array indexed at run time would live
+// in memory; own lane's entries only).  d2_of: the FP32 form's d2 from the value.
+template <typename Band, typename D2>
+__device__ __forceinline__ void settle_pair(const DistArgs &a, const MfmaTile &t, int64_t k, int64_t R, int64_t C,
+                                            bool stats, float *s_u, Band &&in_band, D2 &&d2_of, unsigned &hits,
+                                            unsigned &flips, double &maxerr) {
+    const int lane = threadIdx.x & 63;
+    uint64_t flags = 0ull;
+#pragma unroll
+    for (int e = 0; e < 64; ++e) {
+        const int v = 4 * ((e & 31) >> 3) + (e & 3), blk = ((e >> 2) & 1) + 2 * (e >> 5);
+        const float x = blk == 0 ? t.c00[v] : blk == 1 ? t.c10[v] : blk == 2 ? t.c01[v] : t.c11[v];
+        s_u[e * 64 + lane] = x;
+        if (in_band(x)) flags |= 1ull << e;
+    }
+    uint32_t half[2] = {0u, 0u};  // new bits, layout of pack_halves
+    while (flags) {
+        const int e = __ffsll((unsigned long long)flags) - 1;
+        flags &= flags - 1;
+        int row, col;
+        band_element(lane, e, row, col);
+        const int64_t gi = R * 64 + row, gj = C * 64 + col;
+        if (gi >= a.n || gj >= a.n) continue;
+        NoValue none;
+        const double ex = exact_d2_grouped(a.xw64, a.d, gi, gj, none);
+        if (ex <= a.bp.r2) {
+            if (e < 32) half[0] |= 1u << e;
+            else half[1] |= 1u << (e - 32);
+        }
+        ++hits;
+        if (stats) band_pair_stats(d2_of(s_u[e * 64 + lane], gi, gj), ex, a.bp.r2, flips, maxerr);
+    }
+    const uint64_t colword = merge_col_words(half[0] & 0x0f0f0f0fu, (half[0] >> 4) & 0x0f0f0f0fu,
+                                             half[1] & 0x0f0f0f0fu, (half[1] >> 4) & 0x0f0f0f0fu);
+    const uint64_t word = transpose_bits(colword);  // lane i: row i's extra bits
+    const bool any_new = __ballot(word != 0ull) != 0ull;
+    if (a.pair_nz && lane == 0 && any_new) mark_pair_nz(a, k, R, C);
+    if (word) {
+        atomicOr(&a.mask[(k - a.k_base) * 64 + lane], (unsigned long long)word);
+        atomicAdd(&a.deg[R * 64 + lane], __popcll(word));
+    }
+    if (a.sym && C != R && colword) {
+        const int64_t km = mirror_of(a, k, R, C);
+        atomicOr(&a.mask[(km - a.k_base) * 64 + lane], (unsigned long long)colword);
+        atomicAdd(&a.deg[C * 64 + lane], __popcll(colword));
+    }
+}
+
+// Band elements of the tile pairs that have many or found the record list full
+// (one wave per pair, grid-stride, the count read on the device): U is recomputed
+// by the same instructions.  The statistics are those of U itself.
 template <int KS>
 __global__ __launch_bounds__(64) void k_split_band(DistArgs a) {
+    __shared__ float s_u[64 * 64];
     const int lane = threadIdx.x & 63;
     const int64_t n_redo = (int64_t)*a.redo_cnt;
     unsigned hits = 0, flips = 0;
@@ -2429,52 +2495,26 @@ __global__ __launch_bounds__(64) void k_split_band(DistArgs a) {
         const int64_t C = uniform64(tile_col(a, k, kb));
         SplitRows<KS> A;
         split_load_rows<KS>(a, R, A);
-        const float s_col = a.ss[C];
+        const float s_row = a.ss[R], s_col = a.ss[C];
         const float cb0 = lane < 32 ? s_col : a.sc[C * 64 + (lane & 31)];
         const float cb1 = lane < 32 ? s_col : a.sc[C * 64 + 32 + (lane & 31)];
-        const float E2 = split_e2(a.se[R], a.se[C], a.ss[R], s_col);
+        const float E2 = split_e2(a.se[R], a.se[C], s_row, s_col);
         const bool finite = E2 < INFINITY;
         MfmaTile t;
         split_tile<KS>(A, a.sx + C * (KS * 256) + lane, cb0, cb1, t);
-        uint64_t flags = 0ull;  // elements in the band
-#pragma unroll
-        for (int e = 0; e < 64; ++e) {
-            const int v = 4 * ((e & 31) >> 3) + (e & 3), blk = ((e >> 2) & 1) + 2 * (e >> 5);
-            const float x = blk == 0 ? t.c00[v] : blk == 1 ? t.c10[v] : blk == 2 ? t.c01[v] : t.c11[v];
-            const bool neg = (__float_as_uint(x) >> 31) != 0u;
-            if (!finite || (neg && (__float_as_uint(x + E2) >> 31) == 0u)) flags |= 1ull << e;
-        }
-        uint32_t half[2] = {0u, 0u};  // new bits, layout of pack_halves
-        while (flags) {
-            const int e = __ffsll((unsigned long long)flags) - 1;
-            flags &= flags - 1;
-            int row, col;
-            band_element(lane, e, row, col);
-            const int64_t gi = R * 64 + row, gj = C * 64 + col;
-            if (gi >= a.n || gj >= a.n) continue;
-            SplitValue val(a, gi, gj, a.ss[R], s_col);
-            const double ex = exact_d2_grouped(a.xw64, a.d, gi, gj, val);
-            if (ex <= a.bp.r2) {
-                if (e < 32) half[0] |= 1u << e;
-                else half[1] |= 1u << (e - 32);
-            }
-            ++hits;
-            if (finite) band_pair_stats(a.bp.r2 - 2.0 * val.value(), ex, a.bp.r2, flips, maxerr);
-        }
-        const uint64_t colword = merge_col_words(half[0] & 0x0f0f0f0fu, (half[0] >> 4) & 0x0f0f0f0fu,
-                                                 half[1] & 0x0f0f0f0fu, (half[1] >> 4) & 0x0f0f0f0fu);
-        const uint64_t word = transpose_bits(colword);  // lane i: row i's extra bits
-        const bool any_new = __ballot(word != 0ull) != 0ull;
-        if (a.pair_nz && lane == 0 && any_new) mark_pair_nz(a, k, R, C);
-        if (word) {
-            atomicOr(&a.mask[(k - a.k_base) * 64 + lane], (unsigned long long)word);
-            atomicAdd(&a.deg[R * 64 + lane], __popcll(word));
-        }
-        if (a.sym && C != R && colword) {
-            const int64_t km = mirror_of(a, k, R, C);
-            atomicOr(&a.mask[(km - a.k_base) * 64 + lane], (unsigned long long)colword);
-            atomicAdd(&a.deg[C * 64 + lane], __popcll(colword));
-        }
+        const double s_inv = 1.0 / ((double)s_row * (double)s_col);
+        settle_pair(
+            a, t, k, R, C, finite, s_u,
+            [&](float x) {
+                return !finite || ((__float_as_uint(x) >> 31) != 0u && (__float_as_uint(x + E2) >> 31) == 0u);
+            },
+            [&](float x, int64_t gi, int64_t gj) {
+                // T from U: the terms c instead of the terms c - e
+                const double T = (double)x * s_inv + ((double)a.caug[gi] - (double)a.sc[gi] / s_row) +
+                                 ((double)a.caug[gj] - (double)a.sc[gj] / s_col);
+                return a.bp.r2 - 2.0 * T;
+            },
+            hits, flips, maxerr);
     }
     flush_band(a, hits, flips, maxerr);
 }
@@ -2505,12 +2545,10 @@ static int split_chunk(int64_t n_rb, int64_t n_tiles, bool sym, int tuned) {
 
 // Band elements of the queued tile pairs (one wave per pair): the FP32 values
 // are recomputed exactly as in k_dist_mfma; every element with -E <= T < E is
-// decided in FP64 in reference order (one wave-wide evaluation per element),
-// and its bits are added to the stored words (and to the degrees) of the pair
-// and of its mirror.
+// settled.
 __global__ __launch_bounds__(64) void k_dist_mfma_band(DistArgs a) {
+    __shared__ float s_u[64 * 64];
     const int lane = threadIdx.x & 63;
-    const int r = lane & 31, h = lane >> 5;
     const int64_t n_redo = (int64_t)*a.redo_cnt;
     unsigned hits = 0, flips = 0;
     double maxerr = 0.0;
@@ -2519,52 +2557,11 @@ __global__ __launch_bounds__(64) void k_dist_mfma_band(DistArgs a) {
         int64_t kb, ke;
         tile_range(a, R, kb, ke);
         const int64_t C = uniform64(tile_col(a, k, kb));
-        const float e_row = wave_max(a.emarg[R * 64 + lane]);
-        const float E = pair_margin(e_row, wave_max(a.emarg[C * 64 + lane]));
-        const float nE = -E;
+        const float E = pair_margin(wave_max(a.emarg[R * 64 + lane]), wave_max(a.emarg[C * 64 + lane]));
         const MfmaTile t = mfma_tile(a, R, C);
-        const uint64_t cm = valid_cols(a.n, C);
-        const bool col_a = (cm >> r) & 1ull, col_b = (cm >> (32 + r)) & 1ull;
-        uint32_t a_lo = 0, a_hi = 0, b_lo = 0, b_hi = 0;
-        // element (row 4h + rr + rb, column cb + r) of lane (r, h) with value x,
-        // settled by its own lane: the exact FP64 distance in reference order
-        auto settle = [&](float x, int rr, int rb, int cb, bool col_ok, uint32_t &part) {
-            const bool band = !(x >= E) && !(x < nE) && col_ok && (R * 64 + 4 * h + rr + rb) < a.n;
-            if (band) {
-                const int64_t gi = R * 64 + 4 * h + rr + rb;
-                const int64_t gj = C * 64 + cb + r;
-                const double e = exact_d2(a.xw64, a.d, gi, gj);
-                const bool in = e <= a.bp.r2;
-                if (in) part |= 1u << rr;
-                ++hits;
-                const double d2 = a.bp.r2 - 2.0 * (double)x;
-                flips += (in != (d2 <= a.bp.r2));
-                const double err = fabs(d2 - e);
-                if (err == err) maxerr = fmax(maxerr, err);
-            }
-        };
-    #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int rr = 8 * (v >> 2) + (v & 3);
-            settle(t.c00[v], rr, 0, 0, col_a, a_lo);
-            settle(t.c10[v], rr, 32, 0, col_a, a_hi);
-            settle(t.c01[v], rr, 0, 32, col_b, b_lo);
-            settle(t.c11[v], rr, 32, 32, col_b, b_hi);
-        }
-        const uint64_t colword = merge_col_words(a_lo, a_hi, b_lo, b_hi);
-        const uint64_t word = transpose_bits(colword);  // lane i: row i's extra bits
-        const int64_t i = R * 64 + lane;
-        const bool any_new = __ballot(word != 0ull) != 0ull;
-        if (a.pair_nz && lane == 0 && any_new) mark_pair_nz(a, k, R, C);
-        if (word) {
-            atomicOr(&a.mask[(k - a.k_base) * 64 + lane], (unsigned long long)word);
-            atomicAdd(&a.deg[i], __popcll(word));
-        }
-        if (a.sym && C != R && colword) {
-            const int64_t km = a.tp_ptr ? a.mirror[k] : C * a.n_tiles + R;
-            atomicOr(&a.mask[(km - a.k_base) * 64 + lane], (unsigned long long)colword);
-            atomicAdd(&a.deg[C * 64 + lane], __popcll(colword));
-        }
+        settle_pair(
+            a, t, k, R, C, true, s_u, [&](float x) { return !(x >= E) && !(x < -E); },
+            [&](float x, int64_t, int64_t) { return a.bp.r2 - 2.0 * (double)x; }, hits, flips, maxerr);
     }
     flush_band(a, hits, flips, maxerr);
 }

@@ -126,31 +126,58 @@ def _split_d2(x, r2):
     return r2 - 2.0 * ((big + small).astype(f64) / (s[:, None].astype(f64) * s[None].astype(f64)))
 
 
-@pytest.mark.parametrize("records", [None, "1"])
-@pytest.mark.parametrize("n,d", [(200, 16), (257, 33), (190, 64), (130, 128)])
-def test_band_statistics(cuda, monkeypatch, n, d, records):
-    """Points 1000 from the form's origin (the median of nine rows, here all zero):
-    every pair of them lies inside the band, and the reported flips and largest
-    error are those of the split form's values over these pairs."""
-    if records is not None:
-        monkeypatch.setenv("CNN_HIP_BAND_RECORDS", records)
-    rng = np.random.default_rng(n)
-    x = (rng.normal(size=(n, d)) + 1000.0).astype(np.float32)
-    far = np.ones(n, bool)
+def _far_case(n, d, far):
+    """(x, r): the rows of `far` 1000 from the form's origin (the median of nine
+    rows, here all zero), the others at it."""
+    x = (np.random.default_rng(n).normal(size=(n, d)) + 1000.0).astype(np.float32)
     far[np.arange(9) * (n - 1) // 8] = False
     x[~far] = 0.0
-    r = np.sqrt(2.0 * d)
-    st = _check(x, r)
+    return x, np.sqrt(2.0 * d)
+
+
+def _exact_d2(x):
     y = x.astype(np.float64)
-    exact = np.zeros((n, n))
-    for k in range(d):
+    exact = np.zeros((len(x), len(x)))
+    for k in range(x.shape[1]):
         exact += (y[:, None, k] - y[None, :, k]) ** 2
-    value = _split_d2(x, r * r)
+    return exact
+
+
+@pytest.mark.parametrize("n,d", [(200, 16), (257, 33), (190, 64), (130, 128)])
+def test_band_statistics(cuda, n, d):
+    """Every pair of the far points (at most 11 a tile) lies inside the band: the
+    reported flips and largest error are those of the split form's values."""
+    far = np.arange(n) % 64 < 11
+    x, r = _far_case(n, d, far)
+    st = _check(x, r)
+    value, exact = _split_d2(x, r * r), _exact_d2(x)
     tile = np.arange(n) // 64
     pairs = (tile[:, None] <= tile[None]) & far[:, None] & far[None]  # a tile pair is evaluated once
     assert st["band_hits"] == pairs.sum()
     assert st["max_abs_err_band"] == pytest.approx(np.abs(value - exact)[pairs].max(), rel=1e-9)
     assert st["band_flips"] == ((value <= r * r) != (exact <= r * r))[pairs].sum()
+
+
+@pytest.mark.parametrize("records", [None, "1"])
+@pytest.mark.parametrize("n,d", [(200, 16), (257, 33), (190, 64), (130, 128)])
+def test_dense_band(cuda, monkeypatch, n, d, records):
+    """Nearly every pair inside the band: whole pairs are recomputed, and the values
+    of the matrix units lie within the margin (its accumulation, split and rounding
+    terms times |x|^2, twice for T = (r2 - d2) / 2) of the FP64 ones."""
+    if records is not None:
+        monkeypatch.setenv("CNN_HIP_BAND_RECORDS", records)
+    far = np.ones(n, bool)
+    x, r = _far_case(n, d, far)
+    st = _check(x, r)
+    tile = np.arange(n) // 64
+    pairs = (tile[:, None] <= tile[None]) & far[:, None] & far[None]
+    assert st["band_hits"] == pairs.sum()
+    w = (x.astype(np.float64) ** 2).sum(1).max()
+    units = 21 * ((d + 15) // 16) + 6 + 9
+    assert 0.0 < st["max_abs_err_band"] <= 2.0 * units * 2.0 ** -24 * (2.0 * w + 0.5 * r * r)
+    exact = _exact_d2(x)[pairs]
+    near = np.abs(exact - r * r) <= st["max_abs_err_band"]
+    assert st["band_flips"] <= near.sum()
 
 
 @pytest.mark.parametrize("dtype,shift", [(np.float32, 1024.0), (np.float64, 2.0 ** 30)])
