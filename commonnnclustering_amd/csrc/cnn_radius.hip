@@ -3493,14 +3493,23 @@ static KeySpec make_keyspec(int d, const std::vector<double> &lo, const std::vec
     return ks;
 }
 
-// Whether a graph keeps its words and drops (or never emits) its lists: a
-// resident graph when the words take no more memory (512 bytes per tile pair
-// against 4 per entry), a graph that lives inside one call always -- the words
-// exist anyway, and the label pass on them costs less than emitting lists and
-// merging them (n = 67,000, d = 3, 40 neighbours a point: 592 against 964 us a
-// fit; n = 1e5, d = 16: 3.46 against 3.68 ms).
+// Whether a graph keeps its words and drops (or never emits) its lists.  A
+// resident graph does when the words take no more memory (512 bytes per tile pair
+// against 4 per entry).  A graph that lives inside one call goes by the label
+// pass: a similarity test on words walks the tiles common to two rows, one on
+// lists their entries, and the lists cost their emission.  With at most
+// kWordsTiles candidate tiles a row tile, or kWordsFill entries a tile pair, the
+// words are the faster form: n = 67,000, d = 3, 40 neighbours a point 592 against
+// 964 us a fit; n = 1e5, d = 16, 66 entries a pair 1.65 against 2.46 ms.  Sparse
+// words of many tiles are the slower: n = 6e4, d = 64 uniform, 27 entries a pair
+// and 938 tiles 28.1 against 5.7 ms; n = 2e5, d = 5 with heavy tails, 10 and 2,650
+// 55 against 11 ms.  Over 880 fits (d = 1 to 64, n = 300 to 2e5, five kinds of
+// data, 4 to 1,500 neighbours) the better form of each is 1 % faster than this rule,
+// 7 % faster than words always.
+constexpr int64_t kWordsTiles = 128, kWordsFill = 56;
 static bool keeps_words(const cnn_graph *g, int64_t pairs, int64_t nnz) {
-    return g->arena || (int64_t)512 * pairs <= (int64_t)4 * nnz;
+    if (g->arena) return pairs <= kWordsTiles * g->n_tiles || nnz >= kWordsFill * pairs;
+    return (int64_t)512 * pairs <= (int64_t)4 * nnz;
 }
 
 // Candidate tile pairs, distance masks and CSR for a graph whose working

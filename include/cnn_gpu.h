@@ -73,8 +73,9 @@ enum {
 /* similarity kernel selection.  A similarity test |N(i) & N(j)| >= c_sim is
  * either a merge of the two sorted lists or an AND + popcount of the rows'
  * 64-bit words over the column tiles both rows reach.  CNN_SIM_AUTO takes the
- * words when the graph keeps them (spatial graphs whose words take no more
- * memory than their lists: at least two neighbours per word on average) or,
+ * words when the graph keeps them (resident graphs whose words take no more
+ * memory than their lists: at least two neighbours per word on average; fits:
+ * where the words are the faster form) or,
  * for lists, when a sample of their rows (every stride-th row, the stride at
  * least 16 and about nnz / 2^21) averages at least 8 entries per word
  * (dense rows; the threshold is tunable, cnn_tune_params); otherwise the

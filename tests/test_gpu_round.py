@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import c_oracle as C
-from commonnnclustering_amd import engine
+from commonnnclustering_amd import _lib, engine
 
 pytestmark = pytest.mark.gpu
 
@@ -46,6 +46,46 @@ def test_round_matches_oracle(cuda, n, d, sep, r, cuts):
             lab = engine.fit(X, r * r, 0, 1, precision="f64", member_cutoff=1)[0].cpu().numpy()
             full = C.fit(x, r, 0, member_cutoff=1)
             assert ((lab > 0) >= (full > 0)).all()
+
+
+@pytest.mark.parametrize("kind,n,d,deg,words", [
+    ("heavy", 20000, 5, 40, False), ("heavy", 20000, 5, 2000, True), ("uniform", 9000, 24, 30, False),
+    ("uniform", 9000, 24, 1500, True), ("basins", 20000, 3, 30, True),
+])
+@pytest.mark.parametrize("precision", ["f64", "f32_band"])
+def test_form_by_candidates_and_fill(cuda, kind, n, d, deg, words, precision):
+    """A fit tests similarities on its tile words or, where they are sparse over many
+    candidate tiles, on its lists; labels and predictions are the same."""
+    rng = np.random.default_rng(n + deg)
+    if kind == "heavy":
+        x = rng.standard_t(1.5, size=(n, d))
+    elif kind == "uniform":
+        x = rng.uniform(size=(n, d))
+    else:
+        x = _blobs(n, d, 4.0, n)
+    i, j = rng.integers(0, n, (2, 400_000))
+    r = float(np.sqrt(np.quantile(((x[i] - x[j]) ** 2).sum(1), deg / n)))
+    c = max(1, deg // 20)
+    want = C.fit(x, r, c, member_cutoff=3, use_grid=False)
+    X = torch.from_numpy(x).cuda()
+    lab, _, gs, ls = engine.fit(X, r * r, c + 2, c + 1, precision=precision, member_cutoff=3)
+    assert (lab.cpu().numpy() == want).all()
+    assert (ls["sim_form"] == _lib.CNN_SIM_FORM_TILE_WORDS) == words
+    # new points, against the lists of both sets together
+    y = x[rng.permutation(n)[:100]] + 0.1 * r / np.sqrt(d) * rng.normal(size=(100, d))
+    ids = list(range(1, min(int(want.max()), 5) + 1))
+    got = engine.predict(X, lab, torch.from_numpy(y).cuda(), r * r, c + 2, c + 1, ids, precision=precision)[0]
+    rp, col = C.neighbours_csr(np.concatenate([x, y]), r, use_grid=False)
+    refs = [col[rp[q]:rp[q + 1]][col[rp[q]:rp[q + 1]] < n] for q in range(n, n + 100)]
+    ref = np.zeros(100, np.int64)
+    for q, mine in enumerate(refs):
+        for m in mine if len(mine) > c + 1 else ():
+            other = col[rp[m]:rp[m + 1]]
+            other = other[other < n]
+            if want[m] in ids and len(other) > c + 1 and len(np.intersect1d(mine, other, True)) >= c + 2:
+                ref[q] = want[m]
+                break
+    assert (got.cpu().numpy() == ref).all()
 
 
 @pytest.mark.parametrize("capacity", ["1", "70"])
