@@ -1112,6 +1112,13 @@ __device__ __forceinline__ uint64_t band_resolve(const DistArgs &a, double r2, f
     return m;
 }
 
+// Statistics of one settled pair: d2 the FP32 form's value, ex the FP64 one.
+__device__ __forceinline__ void band_pair_stats(double d2, double ex, double r2, unsigned &flips, double &maxerr) {
+    flips += (ex <= r2) != (d2 <= r2);
+    const double err = fabs(d2 - ex);
+    if (err == err) maxerr = fmax(maxerr, err);
+}
+
 // Band statistics of the workgroup, added with one set of atomics per
 // workgroup (the counters are single addresses: per-wave atomics there
 // serialize).  Every thread of the workgroup must call it.
@@ -1351,18 +1358,25 @@ __global__ __launch_bounds__(256) void k_dist_f32_cols(DistArgs a) {
             const bool col_band = (band_cols >> lane) & 1ull;
             for (int i = 0; i < 64; ++i) {
                 if (!(groups & (1 << (i / kGroupRows)))) continue;
-                const float s = f32_d2_row<D>(rows, i, xc);
                 const int64_t gi = R * 64 + i;
-                if (plain && s < lo) colword |= 1ull << i;
-                const bool in_band = plain ? !(s < lo) && !(s > hi) : band_value<D>(rows, i, xc, base) <= width;
+                double s;  // the FP32 value
+                bool in_band;
+                if (plain) {
+                    const float f = f32_d2_row<D>(rows, i, xc);
+                    if (f < lo) colword |= 1ull << i;
+                    in_band = !(f < lo) && !(f > hi);
+                    s = f;
+                } else {
+                    const uint32_t x = band_value<D>(rows, i, xc, base);
+                    in_band = x <= width;
+                    s = (double)__uint_as_float(x) + (double)base;
+                }
                 if (col_band && in_band && row_real(a, gi)) {
                     const double e = exact_d2(a.xw64, D, gi, j);
                     const bool inx = e <= r2;
                     if (inx) colword |= 1ull << i;
                     ++hits;
-                    flips += (inx != ((double)s <= r2));
-                    const double err = fabs((double)s - e);
-                    if (err == err) maxerr = fmax(maxerr, err);
+                    band_pair_stats(s, e, r2, flips, maxerr);
                 }
             }
         }
@@ -1661,13 +1675,6 @@ __device__ __forceinline__ double exact_d2_grouped(const double *__restrict__ xw
     }
     val.end();
     return s;
-}
-
-// Statistics of one settled pair: d2 the FP32 form's value, ex the FP64 one.
-__device__ __forceinline__ void band_pair_stats(double d2, double ex, double r2, unsigned &flips, double &maxerr) {
-    flips += (ex <= r2) != (d2 <= r2);
-    const double err = fabs(d2 - ex);
-    if (err == err) maxerr = fmax(maxerr, err);
 }
 
 template <bool SPLIT>
