@@ -2039,10 +2039,10 @@ __global__ void k_segments(const int64_t *keys, const int32_t *vals, const int32
 }
 
 __global__ void k_seg_collect(const int64_t *keys, const int32_t *vals, const int32_t *seg_start,
-                              const int32_t *seg_end, int64_t n_seg, unsigned long long *K, uint64_t *okeys,
+                              const int32_t *seg_end, const int32_t *n_seg, unsigned long long *K, uint64_t *okeys,
                               int32_t *ovals) {
     int64_t sid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (sid >= n_seg) return;
+    if (sid >= *n_seg) return;
     const int32_t b = seg_start[sid];
     if (keys[b] == 0) return;
     const int32_t sz = seg_end[sid] - b + 1;
@@ -2068,32 +2068,90 @@ __global__ void k_seg_write(const int32_t *vals, const int32_t *segid, const int
 }
 
 // sort_by_size through a table over the labels 0 .. n (what the fits assign):
-// members and first index per label (runs of equal labels combined before the
-// atomics), the clusters collected and ranked by k_rank_clusters_small, labels
-// rewritten.  flags[0] clusters, [1] a label outside the table, [2] more
-// clusters than that kernel ranks: nothing is written then.
+// members and first index per label, the clusters collected and ranked by
+// k_rank_clusters_small, labels rewritten.  flags[0] clusters, [1] a label outside
+// the table, [2] more clusters than that kernel ranks: nothing is written then.
+//
+// Runs of one label cost one update; a workgroup counts the first kLabelLds labels
+// in LDS, so that labels in any order meet a few hundred updates an address in
+// memory (updates from every wave: 930 us for 1e6 points of 5 clusters in random
+// order, the sort 320, as here 50).
+constexpr int kLabelLds = 2048;
+constexpr int kLabelBlocks = 256;
+
 __global__ __launch_bounds__(256) void k_label_table(const int64_t *__restrict__ labels, int64_t n,
                                                      int32_t *__restrict__ cnt, int32_t *__restrict__ first,
-                                                     unsigned long long *__restrict__ flags, int steps) {
-    const int64_t base = run_base(steps);
-    KeyRun run;
-    bool outside = false;
-    for (int it = 0; it < steps; ++it) {
-        const int64_t i = base + it * 64 + __lane_id();
-        const int64_t l = i < n ? labels[i] : 0;
-        const bool in = l >= 0 && l <= n;
-        outside = outside || !in;
-        run_add(run, cnt, first, in && l != 0, in ? (int)l : 0, (int)i);
+                                                     unsigned long long *__restrict__ flags) {
+    __shared__ int32_t s_cnt[kLabelLds], s_first[kLabelLds];
+    for (int t = threadIdx.x; t < kLabelLds; t += 256) {
+        s_cnt[t] = 0;
+        s_first[t] = INT_MAX;
     }
-    run_flush(run, cnt, first);
-    if (__ballot(outside) != 0ull && __lane_id() == 0) flags[1] = 1ull;
+    __syncthreads();
+    auto add = [&](int key, int count, int at) {
+        if (key < kLabelLds) {
+            atomicAdd(&s_cnt[key], count);
+            atomicMin(&s_first[key], at);
+        } else {
+            atomicAdd(&cnt[key], count);
+            atomicMin(&first[key], at);
+        }
+    };
+    const int lane = __lane_id();
+    const int64_t waves = (int64_t)gridDim.x * 4, wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t per = ((n + waves - 1) / waves + 63) / 64 * 64;  // a wave's points, consecutive
+    const int64_t end = min(n, (wave + 1) * per);
+    bool outside = false;
+    KeyRun run;
+    constexpr int kU = 4;  // steps of 64 points loaded together
+    for (int64_t i0 = wave * per; i0 < end; i0 += 64 * kU) {
+        // another wave met a label outside: the table is not used
+        if (__hip_atomic_load(&flags[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
+        int64_t l[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const int64_t i = i0 + 64 * u + lane;
+            l[u] = i < end ? labels[i] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const bool in = l[u] >= 0 && l[u] <= n;
+            if (__ballot(!in) != 0ull && !outside) {
+                outside = true;
+                if (lane == 0) __hip_atomic_store(&flags[1], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            const int key = in ? (int)l[u] : 0;
+            const uint64_t act = __ballot(key != 0);
+            if (!act) continue;
+            const int at = (int)(i0 + 64 * u), lead = __ffsll((unsigned long long)act) - 1;
+            const int k = __shfl(key, lead, 64);
+            if (__ballot(key != 0 && key != k) != 0ull) {
+                if (key != 0) add(key, 1, at + lane);
+                continue;
+            }
+            if (k != run.key) {
+                if (run.key >= 0 && lane == 0) add(run.key, run.cnt, run.mn);
+                run.key = k;
+                run.cnt = 0;
+                run.mn = at + lead;
+            }
+            run.cnt += __popcll(act);
+        }
+    }
+    if (run.key >= 0 && lane == 0) add(run.key, run.cnt, run.mn);
+    __syncthreads();
+    for (int t = threadIdx.x; t < kLabelLds; t += 256)
+        if (s_cnt[t]) {
+            atomicAdd(&cnt[t], s_cnt[t]);
+            atomicMin(&first[t], s_first[t]);
+        }
 }
 
 __global__ void k_label_clusters(const int32_t *__restrict__ cnt, const int32_t *__restrict__ first, int64_t n,
                                  int64_t member_cutoff, unsigned long long *__restrict__ K, uint64_t *__restrict__ keys,
                                  int32_t *__restrict__ vals) {
     const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (l > n || cnt[l] == 0 || (int64_t)cnt[l] < member_cutoff) return;
+    if (l > n || K[1] || cnt[l] == 0 || (int64_t)cnt[l] < member_cutoff) return;  // K[1]: a label outside
     const unsigned long long idx = atomicAdd(K, 1ull);
     keys[idx] = ((uint64_t)(uint32_t)(0x7fffffff - cnt[l]) << 32) | (uint32_t)first[l];
     vals[idx] = (int32_t)l;
@@ -2102,7 +2160,7 @@ __global__ void k_label_clusters(const int32_t *__restrict__ cnt, const int32_t 
 __global__ void k_label_rewrite(int64_t *__restrict__ labels, int64_t n, const int32_t *__restrict__ newlab,
                                 const unsigned long long *__restrict__ flags) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && !flags[1] && !flags[2]) labels[i] = newlab[labels[i]];
+    if (i < n && !(flags && (flags[1] || flags[2]))) labels[i] = newlab[labels[i]];
 }
 
 __global__ void k_label_clear(int32_t *cnt, int32_t *first, int32_t *newlab, int64_t count,
@@ -2123,9 +2181,8 @@ static int64_t sort_by_size_table(cnn_ctx *ctx, int64_t *labels, int64_t n, int6
     Scratch<int32_t> cnt(ctx, n + 1), first(ctx, n + 1), newlab(ctx, n + 1), vals(ctx, n + 1);
     Scratch<uint64_t> keys(ctx, n + 1);
     Scratch<unsigned long long> flags(ctx, 3);
-    const int steps = run_steps(n);
     k_label_clear<<<blocks_for(n + 1), 256, 0, s>>>(cnt.p, first.p, newlab.p, n + 1, flags.p);
-    k_label_table<<<blocks_for(n, 256 * steps), 256, 0, s>>>(labels, n, cnt.p, first.p, flags.p, steps);
+    k_label_table<<<std::min<unsigned>(blocks_for(n), kLabelBlocks), 256, 0, s>>>(labels, n, cnt.p, first.p, flags.p);
     k_label_clusters<<<blocks_for(n + 1), 256, 0, s>>>(cnt.p, first.p, n, member_cutoff, flags.p, keys.p, vals.p);
     k_rank_clusters_small<<<1, kSmallClusters, 0, s>>>(keys.p, vals.p, flags.p, max_clusters, newlab.p, flags.p + 2);
     k_label_rewrite<<<blocks_for(n), 256, 0, s>>>(labels, n, newlab.p, flags.p);
@@ -2133,8 +2190,15 @@ static int64_t sort_by_size_table(cnn_ctx *ctx, int64_t *labels, int64_t n, int6
     PinnedReads rd(ctx);
     const unsigned long long *h = rd.get(flags.p, 3);
     rd.wait();
-    if (h[1] || h[2]) return -1;
+    if (h[1]) return -1;
     const int64_t K = (int64_t)h[0];
+    if (h[2]) {  // more clusters than one workgroup ranks: their keys are sorted
+        sort_pairs_u64_i32(ctx, keys.p, vals.p, K, 63);
+        k_rank_clusters<<<blocks_for(K), 256, 0, s>>>(vals.p, K, max_clusters, newlab.p);
+        k_label_rewrite<<<blocks_for(n), 256, 0, s>>>(labels, n, newlab.p, nullptr);
+        CNN_HIP(hipGetLastError());
+        CNN_HIP(hipStreamSynchronize(s));
+    }
     return max_clusters >= 0 ? std::min<int64_t>(K, max_clusters) : K;
 }
 
@@ -2142,8 +2206,8 @@ int64_t sort_by_size_generic(cnn_ctx *ctx, int64_t *labels, int64_t n, int64_t m
     hipStream_t s = ctx->stream;
     if (n == 0) return 0;
     if (n >= (int64_t)INT32_MAX) throw InvalidArg{"n exceeds the int32 index range"};
-    // labels as the fits assign them (0 .. n, at most 1024 clusters kept) need no
-    // sort: five kernels and one host read against 22 launches and four reads
+    // labels as the fits assign them (0 .. n) need no sort of the points: five
+    // kernels and one host read against 22 launches and four reads
     // (n = 8000: 47 against 330 us of a traced call)
     const int64_t kept_small = sort_by_size_table(ctx, labels, n, member_cutoff, max_clusters);
     if (kept_small >= 0) return kept_small;
@@ -2156,16 +2220,16 @@ int64_t sort_by_size_generic(cnn_ctx *ctx, int64_t *labels, int64_t n, int64_t m
     sort_pairs_i64_i32(ctx, keys.p, vals.p, n);  // stable: equal labels keep ascending index
     k_heads<<<blocks_for(n), 256, 0, s>>>(keys.p, n, head.p);
     inclusive_scan_u8_to_i32(ctx, head.p, segid.p, n);
-    const int64_t n_seg = read_scalar(ctx, segid.p + (n - 1));
-    Scratch<int32_t> seg_start(ctx, n_seg), seg_end(ctx, n_seg), seglab(ctx, n_seg);
+    // segid[n - 1] segments, at most n: the count stays on the device
+    Scratch<int32_t> seg_start(ctx, n), seg_end(ctx, n), seglab(ctx, n);
     k_segments<<<blocks_for(n), 256, 0, s>>>(keys.p, vals.p, segid.p, n, seg_start.p, seg_end.p);
-    fill_i32(ctx, seglab.p, 0, n_seg);
+    fill_i32(ctx, seglab.p, 0, n);
     Scratch<unsigned long long> K(ctx, 1);
-    CNN_HIP(hipMemsetAsync(K.p, 0, sizeof(unsigned long long), s));
-    Scratch<uint64_t> okeys(ctx, n_seg);
-    Scratch<int32_t> ovals(ctx, n_seg);
-    k_seg_collect<<<blocks_for(n_seg), 256, 0, s>>>(keys.p, vals.p, seg_start.p, seg_end.p, n_seg, K.p, okeys.p,
-                                                    ovals.p);
+    fill_u64(ctx, K.p, 0ull, 1);
+    Scratch<uint64_t> okeys(ctx, n);
+    Scratch<int32_t> ovals(ctx, n);
+    k_seg_collect<<<blocks_for(n), 256, 0, s>>>(keys.p, vals.p, seg_start.p, seg_end.p, segid.p + (n - 1), K.p, okeys.p,
+                                                ovals.p);
     CNN_HIP(hipGetLastError());
     const int64_t k = (int64_t)read_scalar(ctx, K.p);
     sort_pairs_u64_i32(ctx, okeys.p, ovals.p, k, 63);

@@ -83,6 +83,21 @@ def test_lists_are_checked(cuda):
         engine.labels_from_csr(rp, col[:-1], 2, 1)
 
 
+@pytest.mark.parametrize("n", [1, 255, 257, 70_001, 1_000_003])
+@pytest.mark.parametrize("k", [1, 3, 2047, 2049, 40_000])
+def test_sort_by_size_any_order(cuda, n, k):
+    """Labels in random order and in long runs, below and above those counted in LDS."""
+    rng = np.random.default_rng(n + k)
+    top = min(k, n)
+    for x in (rng.integers(0, top + 1, n), np.sort(rng.integers(0, top + 1, n))[::-1].copy()):
+        want = x.copy()
+        C.sort_by_size(want, 2, None)
+        dev = torch.from_numpy(x.copy()).cuda()
+        kept = engine.sort_by_size(dev, 2, None)
+        assert (dev.cpu().numpy() == want).all()
+        assert kept == len(set(want[want > 0].tolist()))
+
+
 @pytest.mark.parametrize("n", [1, 64, 1000, 200_003])
 @pytest.mark.parametrize("k", [1, 1023, 1024, 1025])
 def test_sort_by_size_table_and_beyond(cuda, n, k):
