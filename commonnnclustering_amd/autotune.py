@@ -44,7 +44,7 @@ D_BUCKETS = [(1, 1), (2, 2), (3, 3), (4, 8), (9, 15), (16, 32), (33, 64), (65, 1
 N_BUCKETS = [(0, 1 << 14), (1 << 14, 1 << 17), (1 << 17, 1 << 20), (1 << 20, 1 << 31)]
 
 CANDIDATES = {
-    "mfma_col_chunk": [32, 64, 128],
+    "mfma_col_chunk": [16, 32, 64],
     "wide_col_chunk": [16, 32, 64],
     "emit_waves": [4, 8],
     "root_passes": [1, 2, 3],
