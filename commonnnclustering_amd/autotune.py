@@ -52,6 +52,12 @@ CANDIDATES = {
 }
 
 
+# A value replaces the best so far only if the fit gets faster by this share: a
+# parameter that a fit does not reach (emission, when it keeps its words) would
+# otherwise be set by noise, and lists emitted elsewhere would pay for it.
+MIN_GAIN = 0.015
+
+
 def bucket_of(d: int, n: int):
     db = next(b for b in D_BUCKETS if b[0] <= d <= b[1])
     nb = next(b for b in N_BUCKETS if b[0] <= n < b[1])
@@ -132,7 +138,7 @@ def tune(X, radius_cutoff: float, cnn_cutoff: int, precision="f32_band", member_
             trials.append({"param": name, "value": v, "ms": t})
             if log:
                 log(f"  {name}={v}: {t:.2f} ms (best {t_best:.2f})")
-            if t < t_best:
+            if t < (1.0 - MIN_GAIN) * t_best:
                 t_best, best = t, cand
         set_entry(db, nb, precision, best)
     return {"d_lo": db[0], "d_hi": db[1], "n_lo": nb[0], "n_hi": nb[1], "precision": precision, "params": best,
