@@ -1594,7 +1594,7 @@ __device__ __forceinline__ uint64_t pack_halves(uint32_t a_lo, uint32_t a_hi, ui
 // number of records is read on the device.
 // Bound by the latency of the record and row reads: with the records read one
 // after another, 68 KB of LDS and whole-row loads it took 508 us for 443,000
-// elements of 64 dimensions, as here 236 us (18 of it the split form's value).
+// elements of 64 dimensions, as here 250 us (30 of it the split form's value).
 constexpr int kBandGroup = 64;     // records a workgroup flattens at a time
 constexpr int kBandElems = 4096;   // elements of its list; one record has at most as many
 
@@ -2296,12 +2296,13 @@ __device__ __forceinline__ float split_e2(float e_row, float e_col, float s_row,
 // before they are written to LDS (between the MFMAs and the stores of the
 // current pair, so that waiting for them waits for no recent store), the next
 // column's behind them.
-// n = 2e5, d = 64 (859,000 tile pairs): 1.72 ms against 6.1 to 6.4 ms of the FP32
+// n = 2e5, d = 64 (859,000 tile pairs): 1.75 ms against 6.1 to 6.4 ms of the FP32
 // MFMA form with one column of look-ahead and its index loads in the loop;
 // n = 1e5, d = 16 (758,000 pairs): 0.53 against 2.0 ms.  At d = 64 the matrix
-// units are busy 0.46 of the time (a bare loop of this MFMA reaches 1750
-// TFLOP/s here; without the epilogue the launch takes 1.40 ms, without any
-// staging 1.30), at d = 16 the vector instructions of the epilogue bound it.
+// units are busy 0.42 of the cycles (SQ_VALU_MFMA_BUSY_CYCLES over four times
+// SQ_BUSY_CU_CYCLES; a bare loop of this MFMA reaches 1750 TFLOP/s here; without
+// the epilogue the launch takes 1.40 ms, without any staging 1.30), at d = 16 the
+// vector instructions of the epilogue bound it.
 // Chunks of 16, 32 and 64 columns: 1.84, 1.77 and 1.76 ms.
 template <int KS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, KS <= 1 ? 3 : 2))) void k_dist_split(DistArgs a, int64_t n_rt,
@@ -3265,11 +3266,12 @@ static void launch_dist(cnn_ctx *ctx, const DistArgs &a, int64_t n_rt, bool band
         return;
     }
     if (band && a.d >= kMfmaMinD) {
-        // guard-band elements are listed (and, when the list is full, whole tile pairs,
-        // at most once each) and settled afterwards.  Half a record per pair: a wave
-        // reserves slots 8 at a time and leaves some empty, so at a quarter the list
-        // was full at 5.5e5 elements (n = 2e5, d = 64) and the recomputing kernel took
-        // 820 us, now 4; reserving 2 at a time instead cost k_dist_split 1.59 -> 2.28 ms.
+        // guard-band elements are listed (and, when a pair has many or the list is full,
+        // whole tile pairs, at most once each) and settled afterwards.  Half a record
+        // per pair, one per pair evaluated (528 bytes each): a wave reserves slots 8 at
+        // a time and leaves some empty, so at a quarter the list was full at 5.5e5
+        // elements (n = 2e5, d = 64) and the recomputing kernel took 820 us, now 4;
+        // reserving 2 at a time instead cost k_dist_split 1.59 -> 2.28 ms.
         int64_t cap = std::min<int64_t>(std::max<int64_t>(batch_pairs / 2, 1 << 14), (int64_t)1 << 21);
         if (const char *ev = std::getenv("CNN_HIP_BAND_RECORDS")) cap = std::max<int64_t>(1, std::atoll(ev));
         Scratch<int64_t> cnt(ctx, 2);
