@@ -3196,16 +3196,17 @@ __global__ void k_clear_build(int32_t *deg, int64_t n_deg, int32_t *diag, int64_
 //   FP32 accumulation of d rounded squares of rounded differences: gamma_{d+2}(u32) * D
 //   the reference's own FP64 rounding:                           gamma_{2d+2}(u64) * D
 //   rounding f64 coordinates to f32 (f64 input only):            2 u32 M sqrt(D) + u32^2 M^2
+//   squares and sums below the normal numbers:                   (d + 2) 2^-126
 // with M the largest point norm times two.  A safety factor 2 is applied.
 static BandParams make_band_direct(double r2, int d, bool rounded_coords, double max_norm) {
     const double u32 = std::ldexp(1.0, -24), u64 = std::ldexp(1.0, -53);
     const double D = 2.0 * r2;
-    double E = (gamma_m(d + 2, u32) + gamma_m(2 * d + 2, u64)) * D;
+    double E = (gamma_m(d + 2, u32) + gamma_m(2 * d + 2, u64)) * D + (d + 2) * (double)FLT_MIN;
     if (rounded_coords) {
         const double M = 2.0 * max_norm;
         E += 2.0 * u32 * M * std::sqrt(D) + u32 * u32 * M * M;
     }
-    E = 2.0 * E + 1e-300;
+    E = 2.0 * E;
     BandParams bp;
     bp.r2 = r2;
     double lo = r2 - E, hi = r2 + E;

@@ -53,3 +53,14 @@ def test_packed_ragged_tiles(cuda):
                            precision="f32_band", member_cutoff=2)[0].cpu().numpy()
     for b, x in enumerate(sets):
         assert (lab[off[b]:off[b + 1]] == C.fit(x, 0.7, 2, member_cutoff=2)).all()
+
+
+# squares below the smallest normal FP32 number, and below the smallest of all
+@pytest.mark.parametrize("n", [65, 500])
+@pytest.mark.parametrize("d", [1, 3, 8, 9, 15])
+@pytest.mark.parametrize("scale", [1e-18, 1e-20, 1e-22, 1e-24])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_squares_below_fp32(cuda, n, d, scale, dtype):
+    x = (np.random.default_rng(n * d).normal(size=(n, d)) * scale).astype(dtype)
+    for q in (0.3, 1.0, 4.0):
+        _same_lists(x, q * d * float(scale) ** 2)
