@@ -54,8 +54,9 @@ CANDIDATES = {
 
 # A value replaces the best so far only if the fit gets faster by this share: a
 # parameter that a fit does not reach (emission, when it keeps its words) would
-# otherwise be set by noise, and lists emitted elsewhere would pay for it.
-MIN_GAIN = 0.015
+# otherwise be set by noise, and lists emitted elsewhere would pay for it; and an
+# entry serves a whole class, of which the tuned size is one.
+MIN_GAIN = 0.05
 
 
 def bucket_of(d: int, n: int):
