@@ -2299,7 +2299,7 @@ __device__ __forceinline__ float split_e2(float e_row, float e_col, float s_row,
 // n = 2e5, d = 64 (859,000 tile pairs): 1.75 ms against 6.1 to 6.4 ms of the FP32
 // MFMA form with one column of look-ahead and its index loads in the loop;
 // n = 1e5, d = 16 (758,000 pairs): 0.53 against 2.0 ms.  At d = 64 the matrix
-// units are busy 0.42 of the cycles (SQ_VALU_MFMA_BUSY_CYCLES over four times
+// units are busy 0.43 of the cycles (SQ_VALU_MFMA_BUSY_CYCLES over four times
 // SQ_BUSY_CU_CYCLES; a bare loop of this MFMA reaches 1750 TFLOP/s here; without
 // the epilogue the launch takes 1.40 ms, without any staging 1.30), at d = 16 the
 // vector instructions of the epilogue bound it.
